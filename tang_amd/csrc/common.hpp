@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <string>
 #include <tuple>
+#include <vector>
 
 #include "../../include/tang_hip.h"
 
@@ -133,6 +134,10 @@ struct th_device {
     int* counters = nullptr;  // see device_counters
     void* noalloc_scratch = nullptr;  // this device's address of the th_gemm_q4_noalloc workspace
     size_t n_counters = 0;
+    // Workspace blocks that grew out of use after a graph capture: a recorded
+    // graph may still name them, so they stay until the device goes.
+    bool captured = false;
+    std::vector<void*> retired;
     int live = 0;          // buffers, weights and engines that hold this device
     bool closed = false;   // th_device_destroy ran; the struct waits for live == 0
     th::AqlDev* aql = nullptr;  // HSA queue for recorded sequences (created on first use)

@@ -26,46 +26,42 @@ static __device__ __align__(256) unsigned char scratch[TH_NOALLOC_SCRATCH_BYTES]
 static thread_local std::string g_last_error;
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 
-void* device_scratch(th_device* dev, size_t bytes) {
-    if (bytes <= dev->scratch_bytes) return dev->scratch;
-    if (dev->scratch) {
-        TH_HIP(hipStreamSynchronize(dev->stream));
-        TH_HIP(hipFree(dev->scratch));
-        dev->scratch = nullptr;
-        dev->scratch_bytes = 0;
-    }
+// Grow one of the device's workspaces to `bytes`.  Once a graph has been
+// captured on the device the outgrown block is kept (its graphs may name it)
+// and sizes double, so that the kept blocks stay below the one in use.
+static void* grow_workspace(th_device* dev, void*& ptr, size_t& have, size_t bytes) {
+    if (bytes <= have) return ptr;
     size_t want = std::max(bytes, (size_t)1 << 20);
-    TH_HIP(hipMalloc(&dev->scratch, want));
-    dev->scratch_bytes = want;
-    return dev->scratch;
+    if (ptr && dev->captured) {
+        want = std::max(want, 2 * have);
+        dev->retired.push_back(ptr);
+    } else if (ptr) {
+        TH_HIP(hipStreamSynchronize(dev->stream));
+        TH_HIP(hipFree(ptr));
+    }
+    ptr = nullptr;
+    have = 0;
+    TH_HIP(hipMalloc(&ptr, want));
+    have = want;
+    return ptr;
 }
 
+void* device_scratch(th_device* dev, size_t bytes) { return grow_workspace(dev, dev->scratch, dev->scratch_bytes, bytes); }
+
 void* device_scratch_x(th_device* dev, size_t bytes) {
-    if (bytes <= dev->scratch_x_bytes) return dev->scratch_x;
-    if (dev->scratch_x) {
-        TH_HIP(hipStreamSynchronize(dev->stream));
-        TH_HIP(hipFree(dev->scratch_x));
-        dev->scratch_x = nullptr;
-        dev->scratch_x_bytes = 0;
-    }
-    size_t want = std::max(bytes, (size_t)1 << 20);
-    TH_HIP(hipMalloc(&dev->scratch_x, want));
-    dev->scratch_x_bytes = want;
-    return dev->scratch_x;
+    return grow_workspace(dev, dev->scratch_x, dev->scratch_x_bytes, bytes);
 }
 
 int* device_counters(th_device* dev, size_t n) {
     if (n <= dev->n_counters) return dev->counters;
-    if (dev->counters) {
-        TH_HIP(hipStreamSynchronize(dev->stream));
-        TH_HIP(hipFree(dev->counters));
-        dev->counters = nullptr;
-        dev->n_counters = 0;
-    }
-    const size_t want = std::max(n, (size_t)4096);
-    TH_HIP(hipMalloc(&dev->counters, want * sizeof(int)));
-    TH_HIP(hipMemset(dev->counters, 0, want * sizeof(int)));
-    dev->n_counters = want;
+    size_t have = dev->n_counters * sizeof(int);
+    void* p = dev->counters;
+    dev->counters = nullptr;
+    dev->n_counters = 0;
+    p = grow_workspace(dev, p, have, n * sizeof(int));
+    TH_HIP(hipMemset(p, 0, have));
+    dev->counters = (int*)p;
+    dev->n_counters = have / sizeof(int);
     return dev->counters;
 }
 
@@ -273,6 +269,8 @@ int th_device_destroy(th_device* d) {
     if (d->scratch) (void)hipFree(d->scratch);
     if (d->scratch_x) (void)hipFree(d->scratch_x);
     if (d->counters) (void)hipFree(d->counters);
+    for (void* p : d->retired) (void)hipFree(p);
+    d->retired.clear();
     (void)hipEventDestroy(d->ev_start);
     (void)hipEventDestroy(d->ev_stop);
     (void)hipStreamDestroy(d->stream);
@@ -322,6 +320,7 @@ int th_capture_begin(th_device* d) {
     TH_API_BEGIN
     TH_REQUIRE(d, "null device");
     TH_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
+    d->captured = true;
     TH_API_END
 }
 
