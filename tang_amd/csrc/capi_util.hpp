@@ -33,6 +33,11 @@ inline void check_status(int rc) {
     if (rc != TH_OK) throw Error(rc, std::string("nested call failed: ") + th_last_error());
 }
 
+inline bool stream_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // Grow-only stream-ordered workspace owned by the device.
 void* device_scratch(th_device* dev, size_t bytes);
 // The configuration a sampler was created with (sampling.cpp).
@@ -82,6 +87,6 @@ void launch_q4_linear_prepared(const th_qweight* w, PreparedX xp, size_t m, floa
 void launch_q4_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
                       size_t ldy, hipStream_t stream, th_device* dev, void* ws = nullptr, size_t ws_bytes = 0);
 void launch_q8_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
-                      size_t ldy, hipStream_t stream);
+                      size_t ldy, hipStream_t stream, th_device* dev);
 
 }  // namespace th

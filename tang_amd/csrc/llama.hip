@@ -703,11 +703,6 @@ static bool llama_eager() {
     return eager;
 }
 
-static bool stream_capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-}
-
 // Every kernel of the step stores what later kernels read with write-through
 // stores (the epilogues, the attention merge, the argmax), so its AQL
 // sequence needs no release fences between kernels.

@@ -5,6 +5,7 @@
 
 #include "aql.hpp"
 #include "capi_util.hpp"
+#include "q8gemm.hpp"
 #include "qlinear.hpp"
 
 namespace th {
@@ -21,6 +22,17 @@ static void set_smem(K kernel, size_t bytes) {
         TH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
         d = bytes;
     }
+}
+
+// Whether a q8 linear runs as GEMV launches of four rows: up to four rows,
+// and up to eight on a matrix of at most 4M weights, where two launches cost
+// no more than the MFMA GEMM and its split-K reduction (2048 x 2048, m = 5:
+// 8.5 against 9.1 us).  Beyond that the GEMM reads the weights once where the
+// GEMV took a launch per four rows: 11008 x 4096, f32 rows, m = 5 28.0 -> 16
+// us, m = 100 429 -> 46 us; at four rows on 4096 x 4096 the GEMV is still the
+// faster one (7.9 against 12 us).
+static bool q8_uses_gemv(const th_qweight* w, size_t m) {
+    return m <= 4 || (m <= 8 && w->rows * w->cols <= ((size_t)1 << 22));
 }
 
 // Vector activation loads need K, the row stride and the base 16-byte aligned.
@@ -156,6 +168,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
 }
 
+static void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_t ldy, size_t ks, bool add,
+                                 hipStream_t s) {
+    const size_t total = m * n;
+    const bool vec4 = n % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0 && total < (1u << 31);
+    if (vec4)
+        TH_LAUNCH(splitk_reduce_kernel<true>, dim3((unsigned)std::min<size_t>(ceil_div(total / 4, 256), 4096)),
+                  dim3(256), 0, s, part, y, (int)m, (int)n, (int)ldy, (int)ks, (int)add);
+    else
+        TH_LAUNCH(splitk_reduce_kernel<false>, dim3((unsigned)std::min<size_t>(ceil_div(total, 256), 4096)), dim3(256),
+                  0, s, part, y, (int)m, (int)n, (int)ldy, (int)ks, (int)add);
+    TH_LAUNCH_CHECK();
+}
+
 // Convert m activation rows (f32 or bf16, rows of ldx) into the MFMA GEMM's
 // prepared layout in the device's operand workspace.
 size_t prepared_x_bytes(size_t m, size_t Kp) { return round_up(m * Kp * 2, 256) + round_up(m * sizeof(int), 256); }
@@ -232,17 +257,7 @@ static void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, float* y
                        dim3(256), 0, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x,
                        xp.xexp, epi, src, (int)w->rows, (int)w->cols, (int)w->Kp, (int)w->Kp, gps);
     TH_LAUNCH_CHECK();
-    if (ks > 1) {
-        const size_t total = m * w->rows;
-        const bool vec4 = w->rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0 && total < (1u << 31);
-        if (vec4)
-            TH_LAUNCH(splitk_reduce_kernel<true>, dim3((unsigned)std::min<size_t>(ceil_div(total / 4, 256), 4096)),
-                      dim3(256), 0, s, out, y, (int)m, (int)w->rows, (int)ldy, (int)ks, (int)accumulate);
-        else
-            TH_LAUNCH(splitk_reduce_kernel<false>, dim3((unsigned)std::min<size_t>(ceil_div(total, 256), 4096)),
-                      dim3(256), 0, s, out, y, (int)m, (int)w->rows, (int)ldy, (int)ks, (int)accumulate);
-        TH_LAUNCH_CHECK();
-    }
+    if (ks > 1) launch_splitk_reduce(out, y, m, w->rows, ldy, ks, accumulate, s);
 }
 
 // Tile shape by batch size: one 16-row block up to 16 rows; 64-row column
@@ -334,15 +349,67 @@ static void q8_launch(const th_qweight* w, const void* x, size_t ldx, float* y, 
     else q8_launch_v<M, XF32, PR, false>(w, x, ldx, y, ldy, s);
 }
 
+// K splits of the q8 GEMM: `base` workgroups times ks, chosen so that the
+// busiest CU has little more work than the average one, and two workgroups to
+// overlap where the work allows (alone on its CU a workgroup waits for each
+// step's loads).  11008 x 4096 at m = 100 (172 workgroups) runs in 74 us
+// unsplit, 45.9 with 2 splits, 37.0 with 4, 44.3 with 5; 4096 x 4096 at m = 100
+// (64) in 21.2 with 8 and 23.8 with 12.  Each split keeps four 64-wide chunks.
+static size_t q8_gemm_splits(size_t base, size_t NCH, size_t cus) {
+    size_t best = 1;
+    double best_fill = 0.0;
+    for (size_t ks = 1; ks <= std::min<size_t>(16, std::max<size_t>(1, NCH / 4)); ks++) {
+        if (ks > 1 && base * ks > 3 * cus) break;
+        const size_t per_cu = ceil_div(base * ks, cus);
+        const double fill = (double)(base * ks) / (double)(per_cu * cus) * (per_cu == 1 ? 0.7 : 1.0);
+        if (fill > best_fill) { best_fill = fill; best = ks; }
+    }
+    return best;
+}
+
+// While a stream is captured the workspace may not grow, so a call that has
+// none yet runs unsplit.
+template <int RT, int CB, int KG, bool XF32, bool PR, bool VEC>
+static void q8_gemm_launch(const th_qweight* w, const void* x, size_t m, size_t ldx, float* y, size_t ldy,
+                           hipStream_t s, th_device* dev) {
+    const size_t NT = w->Np / 16, NCH = w->Kp / 64;
+    const unsigned gx = (unsigned)ceil_div(NT, (size_t)(4 * RT)), gy = (unsigned)ceil_div(m, (size_t)(16 * CB));
+    const size_t part = m * w->rows * sizeof(float);
+    size_t ks = q8_gemm_splits((size_t)gx * gy, NCH, (size_t)dev->num_cus);
+    if (ks > 1 && ks * part > dev->scratch_bytes && stream_capturing(s)) ks = 1;
+    const size_t cps = round_up(ceil_div(NCH, ks), (size_t)KG);
+    ks = ceil_div(NCH, cps);
+    float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : y;
+    const int ldo = ks > 1 ? (int)w->rows : (int)ldy;
+    TH_LAUNCH((q8_gemm_kernel<RT, CB, KG, XF32, VEC, PR>), dim3(gx, gy, (unsigned)ks), dim3(256), 0, s,
+              (const uint4*)w->data, (const float*)w->scales, x, out, (int)m, (int)w->rows, (int)w->cols, (int)w->Kp,
+              (int)ldx, ldo, m * w->rows, (int)cps);
+    TH_LAUNCH_CHECK();
+    if (ks > 1) launch_splitk_reduce(out, y, m, w->rows, ldy, ks, false, s);
+}
+
+template <bool XF32, bool PR, bool VEC>
+static void q8_gemm_dispatch(const th_qweight* w, const void* x, size_t m, size_t ldx, float* y, size_t ldy,
+                             hipStream_t s, th_device* dev) {
+    if (m <= 16) q8_gemm_launch<2, 1, 2, XF32, PR, VEC>(w, x, m, ldx, y, ldy, s, dev);
+    else if (m <= 32) q8_gemm_launch<2, 2, XF32 && !PR ? 1 : 2, XF32, PR, VEC>(w, x, m, ldx, y, ldy, s, dev);
+    else q8_gemm_launch<2, 4, XF32 ? 1 : 2, XF32, PR, VEC>(w, x, m, ldx, y, ldy, s, dev);
+}
+
 template <bool XF32, bool PR>
 static void q8_dispatch(const th_qweight* w, const void* x, size_t m, size_t ldx, float* y, size_t ldy,
-                        hipStream_t s) {
-    // Process up to 4 activation rows per launch.
+                        hipStream_t s, th_device* dev) {
+    if (!q8_uses_gemv(w, m)) {
+        // the rows that the GEMV stages bound K for every m above three
+        TH_REQUIRE((Q8GemvSmem<4, 8>::bytes((int)w->Kp)) <= 160 * 1024, "activation too large for the LDS-staged GEMV");
+        if (x_vec_ok(x, ldx, w->cols)) q8_gemm_dispatch<XF32, PR, true>(w, x, m, ldx, y, ldy, s, dev);
+        else q8_gemm_dispatch<XF32, PR, false>(w, x, m, ldx, y, ldy, s, dev);
+        return;
+    }
     for (size_t m0 = 0; m0 < m; m0 += 4) {
-        const size_t mm = std::min<size_t>(4, m - m0);
         const void* xo = (const char*)x + m0 * ldx * (XF32 ? 4 : 2);
         float* yo = y + m0 * ldy;
-        switch (mm) {
+        switch (std::min<size_t>(4, m - m0)) {
             case 1: q8_launch<1, XF32, PR>(w, xo, ldx, yo, ldy, s); break;
             case 2: q8_launch<2, XF32, PR>(w, xo, ldx, yo, ldy, s); break;
             case 3: q8_launch<3, XF32, PR>(w, xo, ldx, yo, ldy, s); break;
@@ -352,16 +419,16 @@ static void q8_dispatch(const th_qweight* w, const void* x, size_t m, size_t ldx
 }
 
 void launch_q8_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
-                      size_t ldy, hipStream_t s) {
+                      size_t ldy, hipStream_t s, th_device* dev) {
     TH_REQUIRE(w && w->bits == 8, "not a q8 weight");
     TH_REQUIRE(xdt == TH_F32 || xdt == TH_BF16, "activations must be f32 or bf16");
     if (m == 0) return;
     if (xdt == TH_F32) {
-        if (w->per_row) q8_dispatch<true, true>(w, x, m, ldx, y, ldy, s);
-        else q8_dispatch<true, false>(w, x, m, ldx, y, ldy, s);
+        if (w->per_row) q8_dispatch<true, true>(w, x, m, ldx, y, ldy, s, dev);
+        else q8_dispatch<true, false>(w, x, m, ldx, y, ldy, s, dev);
     } else {
-        if (w->per_row) q8_dispatch<false, true>(w, x, m, ldx, y, ldy, s);
-        else q8_dispatch<false, false>(w, x, m, ldx, y, ldy, s);
+        if (w->per_row) q8_dispatch<false, true>(w, x, m, ldx, y, ldy, s, dev);
+        else q8_dispatch<false, false>(w, x, m, ldx, y, ldy, s, dev);
     }
 }
 
@@ -399,7 +466,7 @@ int th_gemv_q8(th_device* dev, const th_buffer* x, size_t m, const th_qweight* w
     TH_REQUIRE(w->bits == 8, "weight is not q8");
     require_len_any(x, m * w->cols, "x");
     require_len(y, TH_F32, m * w->rows, "y");
-    launch_q8_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream);
+    launch_q8_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream, dev);
     TH_API_END
 }
 
@@ -416,14 +483,14 @@ int th_bench_linear(th_device* dev, const th_buffer* x, size_t m, th_qweight* co
     auto call = [&](size_t i) {
         const th_qweight* w = ws[i % n_w];
         if (w->bits == 4) launch_q4_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream, dev);
-        else launch_q8_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream);
+        else launch_q8_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream, dev);
     };
     call(0);  // sizes the workspace before any capture
     TH_HIP(hipStreamSynchronize(dev->stream));
     if (use_graph == 2) {
-        // The GEMVs (q8, and q4 at m <= 16) store their output write-through:
-        // no release fences between the launches.
-        const bool wt = w0->bits == 8 || m <= 16;
+        // The GEMVs store their output write-through: no release fences
+        // between the launches.
+        const bool wt = w0->bits == 8 ? q8_uses_gemv(w0, m) : m <= 16;
         // Every call reads x and its weights and writes y: no call reads what
         // another writes (independent).
         // One sequence: whole passes over the copies (at least 240 launches,

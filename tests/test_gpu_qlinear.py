@@ -198,6 +198,42 @@ def test_q8_reference_blocks_per_group_scales(dev):
     assert max_abs_rel(y, ref) < TOL_F32
 
 
+@pytest.mark.parametrize("rows,cols", [(16, 64), (37, 3), (130, 200), (2050, 1096), (512, 4096), (1100, 4096)])
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 65, 129])  # either side of the 16/32/64/128-row blocks
+@pytest.mark.parametrize("scales", ["row", "group"])
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_q8_gemm(dev, rows, cols, m, scales, dt):
+    """The q8 linear beyond four rows (from nine rows, or 4M weights, on the
+    MFMA GEMM).  Every product is exact and the sums
+    are f32, so an output is off by at most (roundings on its way) * 2^-24 of
+    the sum of its terms' magnitudes: K products, plus one per group."""
+    rng = np.random.default_rng(rows + cols + m)
+    bpr = (cols + 31) // 32
+    q = rng.integers(-128 if scales == "row" else -127, 128, (rows, cols), np.int8)
+    sc = rng.uniform(0.005, 0.02, (rows, 1 if scales == "row" else bpr)).astype(np.float32)
+    if scales == "row":
+        w = dev.q8_upload_rowwise(q, sc.reshape(-1), rows, cols)
+    else:
+        blocks = np.zeros((rows, bpr), capi.Q8_BLOCK)
+        blocks["scale"] = sc
+        qp = np.zeros((rows, bpr * 32), np.int8)
+        qp[:, :cols] = q
+        blocks["values"] = qp.reshape(rows, bpr, 32)
+        w = dev.q8_upload_blocks(blocks.reshape(-1), rows, cols)
+    x = (rng.standard_normal((m, cols)) * 10.0 ** rng.uniform(-6, 6, (m, 1))).astype(np.float32)
+    if dt == "bf16":
+        xb = oracle.f32_to_bf16(x.reshape(-1))
+        x = oracle.bf16_to_f32(xb).reshape(m, cols)
+        xd = dev.upload(xb, capi.BF16)
+    else:
+        xd = dev.upload(x)
+    y = dev.gemv_q8(xd, m, w).to_numpy().reshape(m, rows).astype(np.float64)
+    wf = q.astype(np.float64) * np.repeat(sc.astype(np.float64), cols if scales == "row" else 32, axis=1)[:, :cols]
+    ref = x.astype(np.float64) @ wf.T
+    mag = np.abs(x).astype(np.float64) @ np.abs(wf).T
+    assert np.all(np.abs(y - ref) <= (cols + bpr + 16) * 2.0 ** -24 * mag)
+
+
 def test_reference_kats_on_device(dev):
     """q8_matvec_basic / q4_matvec_basic (quantize.rs:326-353) through the device."""
     wf = np.array([1, 2, 3, 4, 5, 6], np.float32)
