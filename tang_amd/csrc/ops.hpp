@@ -84,6 +84,13 @@ __device__ __forceinline__ bool last_arrival(int* counter, int total, int* s_fla
     return *s_flag != 0;
 }
 
+// Orders this wave's LDS accesses (no barrier: the rows are the wave's own).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // One DPP move inside rows of 16 lanes (CTRL: the dpp_ctrl encoding).
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {

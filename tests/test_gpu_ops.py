@@ -141,6 +141,80 @@ def test_kv_attention(dev, H, Hkv, D, start, ql, f16):
     assert err < 1e-4
 
 
+def _attention_f64(q, k, v, start, ql, H, Hkv, D):
+    q, k, v = (a.astype(np.float64) for a in (q.reshape(ql, H, D), k.reshape(-1, Hkv, D), v.reshape(-1, Hkv, D)))
+    out = np.empty((ql, H, D))
+    mag = 0.0
+    with np.errstate(invalid="ignore"):
+        for i in range(ql):
+            n = start + i + 1
+            for h in range(H):
+                kk, vv = k[:n, h * Hkv // H], v[:n, h * Hkv // H]
+                s = kk @ q[i, h] / np.sqrt(D)
+                mag = max(mag, np.max(np.abs(kk) @ np.abs(q[i, h])) / np.sqrt(D))
+                p = np.exp(s - s.max())
+                out[i, h] = (p / p.sum()) @ vv
+    return out.reshape(-1), mag
+
+
+@pytest.mark.parametrize("H,Hkv,D,start,ql", [
+    (1, 1, 64, 0, 1),       # one key
+    (4, 2, 128, 31, 1),     # a whole 32-key block
+    (4, 1, 128, 32, 3),     # one key past it, twelve rows
+    (8, 2, 64, 255, 4),     # sixteen rows, one key past a pass of the waves
+    (3, 1, 256, 130, 5),    # fifteen rows, three heads a kv head
+    (16, 2, 128, 1500, 2),  # sixteen rows, several splits
+    (6, 2, 128, 0, 11),     # 33 rows on the row-tile path, causal from the start
+    (17, 1, 64, 63, 1),     # seventeen rows of one query
+    (4, 4, 256, 100, 65),   # one row past a 64-row tile
+    (12, 4, 64, 700, 64),   # splits of the key blocks
+    (8, 8, 128, 17, 130),
+])
+@pytest.mark.parametrize("f16", [True, False])
+def test_kv_attention_tiles(dev, H, Hkv, D, start, ql, f16):
+    """Row and key counts around the tiles of the MFMA kernels.  A score is
+    off by some D/8 + 8 f32 roundings of its terms' magnitudes, an output by
+    twice that (weights and their sum) and by the roundings of its own sum."""
+    print(f"attention H={H} Hkv={Hkv} D={D} start={start} ql={ql} f16={f16}", flush=True)
+    rng = np.random.default_rng(H + D + start + ql)
+    T = start + ql
+    q = (rng.standard_normal((ql * H, D)) * 2.0 ** rng.uniform(-12, 2, (ql * H, 1))).astype(np.float32).reshape(-1)
+    k = rng.standard_normal(T * Hkv * D).astype(np.float32)
+    v = rng.standard_normal(T * Hkv * D).astype(np.float32)
+    if f16:
+        kh, vh = oracle.f32_to_f16(k), oracle.f32_to_f16(v)
+        kb, vb = dev.upload(kh, capi.F16), dev.upload(vh, capi.F16)
+        k, v = oracle.f16_to_f32(kh), oracle.f16_to_f32(vh)
+    else:
+        kb, vb = dev.upload(k), dev.upload(v)
+    qb = dev.upload(q)
+    ref, mag = _attention_f64(q, k, v, start, ql, H, Hkv, D)
+    bound = (2 * (D / 8 + 8) * mag + T / 16 + 32) * 2.0 ** -24 * np.max(np.abs(v))
+    for _ in range(2):  # the arrival counters are left at zero
+        out = dev.kv_attention(qb, kb, vb, start, ql, H, Hkv, D).to_numpy()
+        assert np.max(np.abs(out - ref)) <= bound
+
+
+@pytest.mark.parametrize("ql,start", [(1, 600), (40, 0), (40, 600)])  # decode, one split, several splits
+@pytest.mark.parametrize("f16", [True, False])
+def test_kv_attention_infinities(dev, ql, start, f16):
+    """An infinite V reaches the queries that attend to it, in its own dim
+    only; a K whose score is minus infinity has weight zero."""
+    H, Hkv, D, T = 4, 2, 64, start + ql
+    rng = np.random.default_rng(ql + start)
+    q = np.abs(rng.standard_normal(ql * H * D)).astype(np.float16).astype(np.float32)
+    k = rng.standard_normal((T, Hkv, D)).astype(np.float16).astype(np.float32)
+    v = rng.standard_normal((T, Hkv, D)).astype(np.float16).astype(np.float32)
+    v[T - 1, 0, 5] = np.inf
+    k[T // 2, 1, 7] = -np.inf
+    up = (lambda a: dev.upload(oracle.f32_to_f16(a.reshape(-1)), capi.F16)) if f16 else (lambda a: dev.upload(a))
+    out = dev.kv_attention(dev.upload(q), up(k), up(v), start, ql, H, Hkv, D).to_numpy()
+    ref, _ = _attention_f64(q, k, v, start, ql, H, Hkv, D)
+    assert np.array_equal(np.isinf(out), np.isinf(ref)) and np.isinf(ref).sum() == 2
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.max(np.abs(out[fin] - ref[fin])) < 1e-5
+
+
 def test_convert_roundtrip(dev):
     x = np.concatenate([capi.synth_normal(1, 5000), np.array([65504.0, 1e-7, -0.0], np.float32)]).astype(np.float32)
     b = dev.convert(dev.upload(x), capi.BF16).to_numpy()
