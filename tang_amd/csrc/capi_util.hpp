@@ -86,6 +86,10 @@ void launch_q4_linear_prepared(const th_qweight* w, PreparedX xp, size_t m, floa
 // activations, then split-K partials) instead of the device's grow-only one.
 void launch_q4_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
                       size_t ldy, hipStream_t stream, th_device* dev, void* ws = nullptr, size_t ws_bytes = 0);
+// y[m][n] (rows of ldy) = the sum of ks partials [ks][m][n] in split order,
+// added to y when add is set.
+void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_t ldy, size_t ks, bool add,
+                          hipStream_t s);
 void launch_q8_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
                       size_t ldy, hipStream_t stream, th_device* dev);
 

@@ -5,12 +5,15 @@
 // tang-expr element-wise kernels (compiled at run time with hiprtc).
 #include <hip/hiprtc.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "capi_util.hpp"
 #include "ops.hpp"
+#include "q8gemm.hpp"
 
 struct th_kernel {
     th_device* dev = nullptr;
@@ -22,121 +25,279 @@ namespace th {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// ---------------------------------------------------------------------------
-// matmul: C[m][n] (+)= op(A)[m][k] . op(B)[k][n] on v_mfma_f32_16x16x4_f32
-// (f32 products exact, f32 accumulation).  A is [m][k] row-major, or [k][m]
-// with TA; B is [k][n], or [n][k] with TB (device.rs:103,407,425).  A and B
-// are f32 or bf16 (converted exactly on load).
-// Workgroup: 256 threads = 4 waves in a 2x2 grid, 64x64 output tile, each
-// wave 32x32 = 2x2 MFMA tiles; K in steps of 16 staged through LDS with
-// padded rows (stride 68 floats: the MFMA operand reads hit distinct banks).
-// ---------------------------------------------------------------------------
-
 template <bool BF16>
 __device__ __forceinline__ float ld_el(const void* p, size_t i) {
     if constexpr (BF16) return __uint_as_float((uint32_t)((const uint16_t*)p)[i] << 16);
     else return ((const float*)p)[i];
 }
 
-constexpr int MM_T = 64, MM_K = 16, MM_LD = MM_T + 4;
+// ---------------------------------------------------------------------------
+// matmul: C[m][n] (+)= op(A)[m][k] . op(B)[k][n].  A is [m][k] row-major, or
+// [k][m] transposed; B is [k][n], or [n][k] transposed (device.rs:103,407,425);
+// both f32 or bf16.
+//
+// On v_mfma_f32_16x16x32_bf16, which has sixteen times the f32 MFMA's rate: an
+// f32 operand goes in as three bf16 parts (x = p0 + p1 + p2 exactly, eight
+// bits each), so f32 x bf16 takes three exact products and f32 x f32 the six
+// whose parts weigh 2^-16 or more of it (the rest is under 2^-22 of a product,
+// below the roundings of its sum); sums are f32.  A result that comes out NaN
+// (an infinity times a part that is zero, or a sum of parts that overflows
+// both ways) is summed again in plain f32 by its thread.
+//
+// Workgroup: 4 waves, WGM along m; each wave TM x TN 16x16 tiles; K in steps
+// of 32, both operands double-buffered in LDS as 8-value octets.  A step sums
+// up by itself before it joins the accumulators (short chains of additions).
+// Bound by the MFMAs and their LDS operands on large shapes, by the chain of
+// steps on small ones (K split over workgroups there).  Against 64x64 tiles
+// on the f32 MFMA: m 509, k 2048, n 5632, f32 x bf16 210 -> 65 us (541 TFLOP/s
+// of parts); m 1, k 4096 275 -> 21 us; m 1024, k = n = 4096, f32 x f32 374 -> 230
+// us, bf16 565 -> 104 us; error against 64 bits 8.1e-7 -> 1.6e-7.
+// ---------------------------------------------------------------------------
 
-template <bool TA, bool TB, bool ABF, bool BBF>
-__global__ __launch_bounds__(256) void matmul_kernel(const void* __restrict__ a, const void* __restrict__ b,
-                                                     float* __restrict__ c, int M, int N, int K, int accumulate) {
-    __shared__ float As[MM_K][MM_LD];  // As[kk][row]
-    __shared__ float Bs[MM_K][MM_LD];  // Bs[kk][col]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * MM_T, n0 = blockIdx.x * MM_T;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    f32x4_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+// An operand: `rows` rows of K values, element (row, k) at row * rs + k * ks.
+struct MatOperand {
+    const void* p;
+    int rows;
+    long rs, ks;
+};
 
-    // staging: each thread moves 4 elements of each 64x16 tile; the fast
-    // index follows the contiguous dimension of the source
-    auto stage = [&](int k0, float ra[4], float rb[4]) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int e = tid + 256 * u;
-            int row, kk;
-            if (TA) { row = e & 63; kk = e >> 6; }   // A[k][m]: m contiguous
-            else { kk = e & 15; row = e >> 4; }      // A[m][k]: k contiguous
-            const int gm = m0 + row, gk = k0 + kk;
-            ra[u] = (gm < M && gk < K) ? ld_el<ABF>(a, TA ? (size_t)gk * M + gm : (size_t)gm * K + gk) : 0.0f;
-            int col, kb;
-            if (TB) { kb = e & 15; col = e >> 4; }   // B[n][k]: k contiguous
-            else { col = e & 63; kb = e >> 6; }      // B[k][n]: n contiguous
-            const int gn = n0 + col, gkb = k0 + kb;
-            rb[u] = (gn < N && gkb < K) ? ld_el<BBF>(b, TB ? (size_t)gn * K + gkb : (size_t)gkb * N + gn) : 0.0f;
-        }
-    };
-    auto store = [&](const float ra[4], const float rb[4]) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int e = tid + 256 * u;
-            if (TA) As[e >> 6][e & 63] = ra[u];
-            else As[e & 15][e >> 4] = ra[u];
-            if (TB) Bs[e & 15][e >> 4] = rb[u];
-            else Bs[e >> 6][e & 63] = rb[u];
-        }
-    };
-    float ra[4], rb[4];
-    stage(0, ra, rb);
-    for (int k0 = 0; k0 < K; k0 += MM_K) {
-        store(ra, rb);
-        __syncthreads();
-        if (k0 + MM_K < K) stage(k0 + MM_K, ra, rb);  // next tile's loads in flight during the MFMAs
-#pragma unroll
-        for (int ks = 0; ks < MM_K; ks += 4) {
-            // 16x16x4: lane (g, r) supplies A[row r][k g] and B[k g][col r]
-            const int g = lane >> 4, r = lane & 15;
-            float av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) av[i] = As[ks + g][wm + 16 * i + r];
-#pragma unroll
-            for (int j = 0; j < 2; j++) bv[j] = Bs[ks + g][wn + 16 * j + r];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+// Octet k0..k0+7 of one row, raw: bf16 pairs in a, or f32 in a and b.  vec:
+// ks == 1, rows of whole dwords and the octet within K: one 16-byte load (two
+// for f32) through a resource; else eight loads (clamped to the last k).
+template <bool BF>
+__device__ __forceinline__ void mm_load8(const MatOperand& m, const __amdgpu_buffer_rsrc_t& rs, int row0, int row, int K,
+                                         int k0, bool vec, u32x4_t& a, u32x4_t& b) {
+    if (vec) {
+        const uint32_t off = ((uint32_t)(row - row0) * (uint32_t)m.rs + (uint32_t)k0) * (BF ? 2u : 4u);
+        a = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+        if constexpr (!BF) b = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16u, 0, 0);
+        return;
     }
-    // D: lane (g, r) holds rows 4g..4g+3 of column r
-    const int g = lane >> 4, r = lane & 15;
+    {
+        uint32_t v[8];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int col = n0 + wn + 16 * j + r;
-            if (col >= N) continue;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = m0 + wm + 16 * i + 4 * g + e;
-                if (row < M) {
-                    float* p = c + (size_t)row * N + col;
-                    *p = accumulate ? *p + acc[i][j][e] : acc[i][j][e];
-                }
-            }
+        for (int i = 0; i < 8; i++) {
+            const size_t at = (size_t)row * m.rs + (size_t)min(k0 + i, K - 1) * m.ks;
+            v[i] = BF ? (uint32_t)((const uint16_t*)m.p)[at] : ((const uint32_t*)m.p)[at];
         }
+        if constexpr (BF) {
+            a = u32x4_t{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
+        } else {
+            a = u32x4_t{v[0], v[1], v[2], v[3]};
+            b = u32x4_t{v[4], v[5], v[6], v[7]};
+        }
+    }
 }
 
-template <bool TA, bool TB>
-static void matmul_launch2(const th_buffer* a, const th_buffer* b, th_buffer* c, size_t m, size_t k, size_t n,
-                           int acc, hipStream_t s) {
-    const dim3 grid((unsigned)ceil_div(n, MM_T), (unsigned)ceil_div(m, MM_T));
-    const bool abf = a->dtype == TH_BF16, bbf = b->dtype == TH_BF16;
-#define TH_MM(AB, BB)                                                                                          \
-    TH_LAUNCH((matmul_kernel<TA, TB, AB, BB>), grid, dim3(256), 0, s, a->ptr, b->ptr, (float*)c->ptr, \
-                       (int)m, (int)n, (int)k, acc)
-    if (abf && bbf) TH_MM(true, true);
-    else if (abf) TH_MM(true, false);
-    else if (bbf) TH_MM(false, true);
-    else TH_MM(false, false);
-#undef TH_MM
+// Values at k >= K (n of the eight are real) to zero.
+template <bool BF>
+__device__ __forceinline__ void mm_mask(int n, u32x4_t& a, u32x4_t& b) {
+    if (n >= 8) return;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if constexpr (BF) {
+            a[i] = 2 * i + 1 < n ? a[i] : 2 * i < n ? a[i] & 0xFFFFu : 0u;
+        } else {
+            a[i] = i < n ? a[i] : 0u;
+            b[i] = i + 4 < n ? b[i] : 0u;
+        }
+    }
+}
+
+template <bool BF>
+__device__ __forceinline__ float mm_el(const MatOperand& m, int row, int k) {
+    return ld_el<BF>(m.p, (size_t)row * m.rs + (size_t)k * m.ks);
+}
+
+constexpr int MM_LD = 17;  // octet stride in 16-byte units (16 rows + 1: spreads the banks)
+
+template <bool ABF, bool BBF, bool AV, bool BV, int TM, int TN, int WGM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void matmul_kernel(
+    MatOperand A, MatOperand B, float* __restrict__ c, int K, size_t split_stride, int k_per_split, int accumulate) {
+    constexpr int PA = ABF ? 1 : 3, PB = BBF ? 1 : 3, WGN = 4 / WGM;
+    constexpr int MB = WGM * TM, NB = WGN * TN;           // 16-row blocks of the workgroup
+    constexpr int APL = MB * 4 * MM_LD, BPL = NB * 4 * MM_LD;  // one part of a step
+    constexpr int AO = MB * 64, BO = NB * 64;             // octets of a step
+    constexpr int AT = (AO + 255) / 256, BT = (BO + 255) / 256;
+    __shared__ uint4 lds[2][PA * APL + PB * BPL];
+    int bx = blockIdx.x, by = blockIdx.y, split = blockIdx.z;
+    gemm_xcd_tile(bx, by, split);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int m0 = by * MB * 16, n0 = bx * NB * 16;
+    const int wm = (wave / WGN) * TM, wn = (wave % WGN) * TN;
+    const int kb = split * k_per_split, ke = min(K, kb + k_per_split);
+    // resources based at the block's first row (offsets stay 32-bit)
+    auto rsrc = [&](const MatOperand& m, int row0, size_t es) {
+        const size_t left = ((size_t)(m.rows - 1 - row0) * m.rs + K) * es;  // (one row: rs need not be K)
+        return buffer_rsrc((const char*)m.p + (size_t)row0 * m.rs * es, (uint32_t)min(left, (size_t)0x7FFFFFF0));
+    };
+    const __amdgpu_buffer_rsrc_t ars = rsrc(A, AV ? m0 : 0, ABF ? 2 : 4), brs = rsrc(B, BV ? n0 : 0, BBF ? 2 : 4);
+
+    // octet idx of a step: (row, octet) with the index that is contiguous in
+    // memory running fastest over the threads
+    auto place = [](int idx, int rows, bool vec, int& row, int& o) {
+        row = vec ? idx >> 2 : idx % rows;
+        o = vec ? idx & 3 : idx / rows;
+    };
+    u32x4_t ra[AT][2], rb[BT][2];
+    auto load = [&](int k) {
+        const bool whole = k + 32 <= K;  // uniform: all but the last step
+#pragma unroll
+        for (int i = 0; i < AT; i++) {
+            int row, o;
+            place(min(tid + 256 * i, AO - 1), MB * 16, AV, row, o);
+            mm_load8<ABF>(A, ars, m0, min(m0 + row, A.rows - 1), K, k + o * 8, AV && whole, ra[i][0], ra[i][1]);
+        }
+#pragma unroll
+        for (int i = 0; i < BT; i++) {
+            int row, o;
+            place(min(tid + 256 * i, BO - 1), NB * 16, BV, row, o);
+            mm_load8<BBF>(B, brs, n0, min(n0 + row, B.rows - 1), K, k + o * 8, BV && whole, rb[i][0], rb[i][1]);
+        }
+    };
+    auto put = [&](auto bf, uint4* dst, int plane, int row, int o, u32x4_t (&v)[2], int k) {
+        constexpr bool BF = decltype(bf)::value;
+        mm_mask<BF>(K - (k + o * 8), v[0], v[1]);
+        dst += ((row >> 4) * 4 + o) * MM_LD + (row & 15);
+        if constexpr (BF) {
+            *dst = __builtin_bit_cast(uint4, v[0]);
+        } else {
+            uint4 p[3];
+            split3_bf16(__builtin_bit_cast(uint4, v[0]), __builtin_bit_cast(uint4, v[1]), p);
+#pragma unroll
+            for (int e = 0; e < 3; e++) dst[e * plane] = p[e];
+        }
+    };
+    auto store = [&](uint4* t, int k) {
+#pragma unroll
+        for (int i = 0; i < AT; i++) {
+            int row, o;
+            place(tid + 256 * i, MB * 16, AV, row, o);
+            if (AO % 256 == 0 || tid + 256 * i < AO) put(std::integral_constant<bool, ABF>{}, t, APL, row, o, ra[i], k);
+        }
+#pragma unroll
+        for (int i = 0; i < BT; i++) {
+            int row, o;
+            place(tid + 256 * i, NB * 16, BV, row, o);
+            if (BO % 256 == 0 || tid + 256 * i < BO)
+                put(std::integral_constant<bool, BBF>{}, t + PA * APL, BPL, row, o, rb[i], k);
+        }
+    };
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    load(kb);
+    store(lds[0], kb);
+    __syncthreads();
+    int buf = 0;
+    for (int k = kb; k < ke; k += 32) {
+        const uint4 *ta = lds[buf], *tb = ta + PA * APL;
+        const bool more = k + 32 < ke;
+        if (more) load(k + 32);
+        bf16x8_t bv[TN][PB];
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int p = 0; p < PB; p++)
+                bv[j][p] = __builtin_bit_cast(bf16x8_t, tb[p * BPL + ((wn + j) * 4 + q) * MM_LD + r]);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            bf16x8_t av[PA];
+#pragma unroll
+            for (int p = 0; p < PA; p++)
+                av[p] = __builtin_bit_cast(bf16x8_t, ta[p * APL + ((wm + i) * 4 + q) * MM_LD + r]);
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                // D = (rows of B) x (rows of A): a lane holds four consecutive n of one m
+                f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int w = 2; w >= 0; w--)  // the smallest products first
+#pragma unroll
+                    for (int p = 0; p <= w; p++)
+                        if (p < PA && w - p < PB)
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j][w - p], av[p], d, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[i][j][e] += d[e];
+            }
+        }
+        // The additions stay in this block: moved past the branch below they
+        // follow their MFMA with too few wait states (the compiler counts none
+        // across a taken branch), and read it too early.
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) asm volatile("" : "+v"(acc[i][j]));
+        buf ^= 1;
+        if (more) store(lds[buf], k + 32);
+        __syncthreads();
+    }
+    float* cb = c + (size_t)split * split_stride;
+    const int N = B.rows;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int m = m0 + (wm + i) * 16 + r;
+        if (m >= A.rows) continue;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int n = n0 + (wn + j) * 16 + 4 * q;
+            float* p = cb + (size_t)m * N + n;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (n + e >= N || acc[i][j][e] == acc[i][j][e]) continue;
+                float s = 0.0f;  // NaN: in plain f32
+                for (int k = kb; k < ke; k++) s = __builtin_fmaf(mm_el<ABF>(A, m, k), mm_el<BBF>(B, n + e, k), s);
+                acc[i][j][e] = s;
+            }
+            if (N % 4 == 0 && n < N) {
+                f32x4_t v = acc[i][j];
+                if (accumulate) v = *(const f32x4_t*)p + v;
+                *(f32x4_t*)p = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < N) p[e] = accumulate ? p[e] + acc[i][j][e] : acc[i][j][e];
+            }
+        }
+    }
+}
+
+template <bool ABF, bool BBF, bool AV, bool BV, int TM, int TN, int WGM>
+static void matmul_launch(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
+    const size_t m = A.rows, n = B.rows, part = m * n * sizeof(float), cus = dev->num_cus;
+    const unsigned gx = (unsigned)ceil_div(n, (size_t)(4 / WGM * TN * 16)), gy = (unsigned)ceil_div(m, (size_t)(WGM * TM * 16));
+    // Split K where the tiles leave CUs idle: two workgroups per CU, each
+    // split at least 128 deep.  (While a stream is captured the workspace may
+    // not grow: a call that has none yet runs unsplit.)
+    size_t ks = std::max<size_t>(1, std::min({2 * cus / ((size_t)gx * gy), k / 128, (size_t)16}));
+    if (ks > 1 && ks * part > dev->scratch_bytes && stream_capturing(dev->stream)) ks = 1;
+    const size_t per = round_up(ceil_div(k, ks), (size_t)32);
+    ks = ceil_div(k, per);
+    float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : c;
+    TH_LAUNCH((matmul_kernel<ABF, BBF, AV, BV, TM, TN, WGM>), dim3(gx, gy, (unsigned)ks), dim3(256), 0, dev->stream, A, B,
+              out, (int)k, m * n, (int)per, ks > 1 ? 0 : acc);
     TH_LAUNCH_CHECK();
+    if (ks > 1) launch_splitk_reduce(out, c, m, n, n, ks, acc != 0, dev->stream);
+}
+
+template <bool ABF, bool BBF, bool AV, bool BV>
+static void matmul_shape(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
+    if (A.rows <= 16) matmul_launch<ABF, BBF, AV, BV, 1, 1, 1>(A, B, c, k, acc, dev);  // 16 x 64
+    else matmul_launch<ABF, BBF, AV, BV, 2, 4, 2>(A, B, c, k, acc, dev);               // 64 x 128
+}
+
+template <bool ABF, bool BBF>
+static void matmul_dispatch(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
+    // one 16-byte load per octet where k is contiguous, rows are whole dwords
+    // and a block's offsets fit 32 bits
+    auto vec = [](const MatOperand& m, bool bf) { return m.ks == 1 && (!bf || m.rs % 2 == 0) && m.rs <= (1l << 21); };
+    const bool av = vec(A, ABF), bv = vec(B, BBF);
+    if (av && bv) matmul_shape<ABF, BBF, true, true>(A, B, c, k, acc, dev);
+    else if (av) matmul_shape<ABF, BBF, true, false>(A, B, c, k, acc, dev);
+    else if (bv) matmul_shape<ABF, BBF, false, true>(A, B, c, k, acc, dev);
+    else matmul_shape<ABF, BBF, false, false>(A, B, c, k, acc, dev);
 }
 
 // ---------------------------------------------------------------------------
@@ -201,17 +362,20 @@ int th_matmul_ex(th_device* dev, const th_buffer* a, const th_buffer* b, size_t 
     require_len_any(a, m * k, "a");
     require_len_any(b, k * n, "b");
     require_len(c, TH_F32, m * n, "c");
-    TH_REQUIRE(m < (1u << 31) / MM_T && n < (1u << 31) / MM_T && k < (1u << 31), "matmul: dimension too large");
+    TH_REQUIRE(m < (1u << 31) / 64 && n < (1u << 31) / 64 && k < (1u << 31), "matmul: dimension too large");
     if (m == 0 || n == 0) return TH_OK;
-    hipStream_t s = dev->stream;
     if (k == 0) {  // an empty sum: C = 0 (or C unchanged when accumulating)
         if (!accumulate) check_status(th_buffer_zero(c));
         return TH_OK;
     }
-    if (trans_a && trans_b) matmul_launch2<true, true>(a, b, c, m, k, n, accumulate, s);
-    else if (trans_a) matmul_launch2<true, false>(a, b, c, m, k, n, accumulate, s);
-    else if (trans_b) matmul_launch2<false, true>(a, b, c, m, k, n, accumulate, s);
-    else matmul_launch2<false, false>(a, b, c, m, k, n, accumulate, s);
+    const MatOperand A{a->ptr, (int)m, trans_a ? 1l : (long)k, trans_a ? (long)m : 1l};
+    const MatOperand B{b->ptr, (int)n, trans_b ? (long)k : 1l, trans_b ? 1l : (long)n};
+    float* out = (float*)c->ptr;
+    const bool abf = a->dtype == TH_BF16, bbf = b->dtype == TH_BF16;
+    if (abf && bbf) matmul_dispatch<true, true>(A, B, out, k, accumulate, dev);
+    else if (abf) matmul_dispatch<true, false>(A, B, out, k, accumulate, dev);
+    else if (bbf) matmul_dispatch<false, true>(A, B, out, k, accumulate, dev);
+    else matmul_dispatch<false, false>(A, B, out, k, accumulate, dev);
     TH_API_END
 }
 

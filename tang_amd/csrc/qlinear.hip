@@ -168,8 +168,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
 }
 
-static void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_t ldy, size_t ks, bool add,
-                                 hipStream_t s) {
+void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_t ldy, size_t ks, bool add,
+                          hipStream_t s) {
     const size_t total = m * n;
     const bool vec4 = n % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0 && total < (1u << 31);
     if (vec4)

@@ -41,6 +41,53 @@ def test_matmul_variants(dev, m, k, n, ta, tb):
     assert err < 1e-5
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 1, 3), (16, 31, 64), (17, 33, 65), (64, 32, 128), (65, 130, 129), (3, 1000, 70),
+                                   (130, 515, 260), (1, 100, 1)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("ad,bd", [("f32", "bf16"), ("bf16", "f32"), ("bf16", "bf16"), ("f32", "f32")])
+def test_matmul_tiles_and_types(dev, m, k, n, ta, tb, ad, bd):
+    """Edges of the 16- and 64-row tiles, the 32-deep steps and the K splits,
+    for every operand type and order, added to C.  Products of bf16 parts are
+    exact (f32 x f32 leaves out under 2^-22 of one), sums are f32: an output
+    is off by at most (k + 4) roundings of its terms' magnitudes."""
+    rng = np.random.default_rng(m * 7 + k + n)
+    a = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-8, 8, (m, 1))).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    c0 = rng.standard_normal((m, n)).astype(np.float32)
+
+    def up(x, t, dt):
+        x = (x.T if t else x).reshape(-1).copy()
+        return dev.upload(oracle.f32_to_bf16(x), capi.BF16) if dt == "bf16" else dev.upload(x)
+
+    if ad == "bf16":
+        a = _bf16_round(a.reshape(-1)).reshape(m, k)
+    if bd == "bf16":
+        b = _bf16_round(b.reshape(-1)).reshape(k, n)
+    c = dev.upload(c0)
+    dev.matmul(up(a, ta, ad), up(b, tb, bd), m, k, n, trans_a=ta, trans_b=tb, accumulate_into=c)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    ref, mag = c0 + a @ b, np.abs(c0) + np.abs(a) @ np.abs(b)
+    assert np.all(np.abs(c.to_numpy().reshape(m, n) - ref) <= (k + 4) * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("m", [5, 70])
+@pytest.mark.parametrize("bd", ["f32", "bf16"])
+def test_matmul_infinities(dev, m, bd):
+    """An infinity times finite values gives infinities, times zero NaN, and
+    reaches no other row or column."""
+    k, n = 200, 40
+    rng = np.random.default_rng(m)
+    a = rng.integers(1, 9, (m, k)).astype(np.float32)
+    b = rng.integers(1, 9, (k, n)).astype(np.float32)
+    a[1, 7], a[2, 150], b[7, 3], b[90, 5] = np.inf, -np.inf, 0.0, np.inf
+    db = dev.upload(oracle.f32_to_bf16(b.reshape(-1)), capi.BF16) if bd == "bf16" else dev.upload(b)
+    c = dev.matmul(dev.upload(a), db, m, k, n).to_numpy().reshape(m, n)
+    with np.errstate(invalid="ignore"):
+        ref = np.stack([(a[:, [i]].astype(np.float64) * b[[i]]) for i in range(k)]).sum(0)
+    assert np.isnan(ref[1, 3]) and np.isnan(ref[2, 5]) and np.isinf(ref[1, 0])
+    assert np.array_equal(c, ref.astype(np.float32), equal_nan=True)
+
+
 def test_matmul_kats_and_accumulate(dev):
     """cpu.rs:785-822 known answers; matmul_accumulate (device.rs:391) adds."""
     c = dev.matmul(dev.upload(np.array([1, 0, 0, 1], np.float32)), dev.upload(np.array([1, 2, 3, 4], np.float32)),
