@@ -174,12 +174,11 @@ int th_gemv_q8(th_device* dev, const th_buffer* x, size_t m, const th_qweight* w
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * kernels and results as th_gemm_q4, but the MFMA path's workspace (the
- * prepared activations, then the split-K partials) is a fixed per-GPU device
- * array of TH_NOALLOC_SCRATCH_BYTES, not an allocation: the call makes no
- * hipMalloc / hipFree.  Fails with TH_ERR_INVALID when the prepared
- * activations, about 2*m*K bytes, do not fit (split-K is narrowed to what
- * fits).  Every call on one GPU shares the array: calls that overlap on one
- * GPU (two streams, two threads) race. */
+ * prepared activations) is a fixed per-GPU device array of
+ * TH_NOALLOC_SCRATCH_BYTES, not an allocation: the call makes no hipMalloc /
+ * hipFree.  Fails with TH_ERR_INVALID when the prepared activations, about
+ * 2*m*K bytes, do not fit.  Every call on one GPU shares the array: calls that
+ * overlap on one GPU (two streams, two threads) race. */
 #define TH_NOALLOC_SCRATCH_BYTES (64u << 20)
 int th_gemm_q4_noalloc(th_device* dev, const th_buffer* x, size_t m, const th_qweight* w, th_buffer* y);
 

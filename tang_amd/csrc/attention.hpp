@@ -4,6 +4,7 @@
 
 #include "common.hpp"
 #include "ops.hpp"
+#include "qlinear.hpp"
 
 namespace th {
 
@@ -351,8 +352,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
                 z[i] = __shfl_xor(y[i], 16, 64);
             }
             if (qi < n && (g & 1) == 0) {
-                uint16_t* op = out + (size_t)qi * ldo + h * D + dt * 16 + 4 * g;
-                *(uint4*)op = make_uint4(attn_pack_h2(y[0], z[0]), attn_pack_h2(y[1], z[1]),
+                ((uint4*)out)[xp_index(qi, (h * D + dt * 16 + 4 * g) >> 3, ldo >> 3)] = make_uint4(attn_pack_h2(y[0], z[0]), attn_pack_h2(y[1], z[1]),
                                          attn_pack_h2(y[2], z[2]), attn_pack_h2(y[3], z[3]));
             }
         }
@@ -367,9 +367,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
     }
 }
 
-// out: bf16 rows of ldo, or (xp) the MFMA GEMM's prepared f16 layout (rows
-// of ldo >= n_heads * head_dim, which must then be the consumer's Kp) with
-// row exponents xexp.
+// out: bf16 rows of ldo, or (xp) the MFMA GEMM's prepared f16 layout
+// (xp_index; ldo >= n_heads * head_dim must then be the consumer's Kp) with row
+// exponents xexp.
 inline void launch_attn_prefill(const float* q, int ldq, const _Float16* kc, const _Float16* vc, int n_heads,
                                 int n_kv_heads, int head_dim, int pos0, int n, uint16_t* out, int ldo, bool xp,
                                 int* xexp, hipStream_t s) {

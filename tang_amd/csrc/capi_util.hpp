@@ -66,24 +66,29 @@ th_qweight* q8_pack(th_device* dev, const int8_t* q, size_t ldq, const float* sc
 // Quantized linear launchers (qlinear.hip).  x: [m][ldx] f32 or bf16,
 // y: [m][ldy] f32.
 // Activations in the MFMA GEMM's prepared layout: row r holds the f16 values
-// x[r][k] * 2^-xexp[r] in rows of the weight's Kp (zero past K), each 8-value
-// chunk ordered x0,x4,x1,x5,x2,x6,x3,x7.
+// x[r][k] * 2^-xexp[r] up to the weight's Kp (zero past K), each 8-value chunk
+// ordered x0,x4,x1,x5,x2,x6,x3,x7 and placed at xp_index (blocks of 16 rows,
+// the last one whole).
 struct PreparedX {
     const uint16_t* x;
     const int* xexp;
 };
 // prepare_x writes that layout for m rows of x (input row rows[r] for output
 // row r when rows is set) into the device's operand workspace.
-// workspace (optional): prepared_x_bytes(m, Kp) bytes to use instead.
+// workspace (optional): prepared_x_bytes(m, Kp) bytes to use instead.  blocked =
+// false: rows of Kp one after the other, for the grouped source.
 PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t ldx, size_t K, size_t Kp,
-                    hipStream_t s, const int* rows = nullptr, void* workspace = nullptr);
+                    hipStream_t s, const int* rows = nullptr, void* workspace = nullptr, bool blocked = true);
 size_t prepared_x_bytes(size_t m, size_t Kp);
+// Beyond TH_NOALLOC_SCRATCH_BYTES: room for the last block's padding rows (K up
+// to 139,000).
+constexpr size_t NOALLOC_SLACK = (size_t)4 << 20;
 // The MFMA GEMM on prepared activations, for producers that write the layout
 // directly.  accumulate: y += x.W^T (a fused residual add) instead of y = x.W^T.
 void launch_q4_linear_prepared(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
-                               th_device* dev, bool accumulate = false);
-// ws / ws_bytes (optional): a workspace for the MFMA path (prepared
-// activations, then split-K partials) instead of the device's grow-only one.
+                               bool accumulate = false);
+// ws / ws_bytes (optional): a workspace for the MFMA path's prepared
+// activations instead of the device's grow-only one.
 void launch_q4_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
                       size_t ldy, hipStream_t stream, th_device* dev, void* ws = nullptr, size_t ws_bytes = 0);
 // y[m][n] (rows of ldy) = the sum of ks partials [ks][m][n] in split order,

@@ -16,12 +16,12 @@
 namespace th {
 
 // Workspace of th_gemm_q4_noalloc (the allocation-free GEMM): a file-scope
-// device array, TH_NOALLOC_SCRATCH_BYTES per GPU, held by every GPU the
+// device array, TH_NOALLOC_SCRATCH_BYTES (and the slack) per GPU, held by every GPU the
 // library runs on until the process ends.  Host code never uses its name as
 // an address: th_device_create looks up the array's address on its device
 // (th_device::noalloc_scratch) and kernels receive that.  Every call on one
 // GPU shares it.
-static __device__ __align__(256) unsigned char scratch[TH_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[TH_NOALLOC_SCRATCH_BYTES + NOALLOC_SLACK];
 
 static thread_local std::string g_last_error;
 void set_last_error(const std::string& msg) { g_last_error = msg; }

@@ -29,6 +29,7 @@
 #include "attention.hpp"
 #include "capi_util.hpp"
 #include "ops.hpp"
+#include "q4gemm.hpp"
 #include "qlinear.hpp"
 
 namespace th {
@@ -283,8 +284,8 @@ __global__ __launch_bounds__(64) void prefill_rmsnorm_kernel(const float* __rest
             chunk(c * 8, y);
 #pragma unroll
             for (int i = 0; i < 8; i++) y[i] = __builtin_amdgcn_ldexpf(y[i], -e);
-            *(uint4*)(orow + c * 8) = make_uint4(pack_half2(y[0], y[4]), pack_half2(y[1], y[5]),
-                                                 pack_half2(y[2], y[6]), pack_half2(y[3], y[7]));
+            ((uint4*)out)[xp_index(row, c, ldo >> 3)] = make_uint4(pack_half2(y[0], y[4]), pack_half2(y[1], y[5]),
+                                                                   pack_half2(y[2], y[6]), pack_half2(y[3], y[7]));
         }
     } else {
         for (int c = lane; c * 8 < d; c += 64) {
@@ -360,10 +361,6 @@ __global__ void prefill_swiglu_kernel(const float* __restrict__ gu, int ff, uint
     }
 }
 
-// The same values in the MFMA GEMM's prepared layout (as the XP RMSNorm
-// above): one 256-thread workgroup per row stages the row's bf16 values in
-// LDS (dynamic, ldo halves), takes their largest magnitude, then writes the
-// scaled f16 chunks (zero past ff) and the row exponent.
 // RMSNorm into the prepared GEMM layout with the row held in registers:
 // 256 threads per row, U chunks of 8 elements per thread (d <= 2048 * U), so
 // the row is read once (one wave re-reading it per pass was latency-bound:
@@ -376,7 +373,7 @@ __global__ __launch_bounds__(256) void prefill_rmsnorm_xp_kernel(const float* __
                                                                  uint16_t* __restrict__ out, int ldo,
                                                                  int* __restrict__ xexp) {
     __shared__ float red_sum[4], red_max[4];
-    const int row = blockIdx.x, t = threadIdx.x;
+    const int row = xp_block_row(blockIdx.x, gridDim.x), t = threadIdx.x;
     const float* xr = x + (size_t)row * d;
     float y[U][8];
     uint4 wv[U];
@@ -417,7 +414,6 @@ __global__ __launch_bounds__(256) void prefill_rmsnorm_xp_kernel(const float* __
     }
     const int e = range_exp(block_absmax256(mx, red_max), XPREP_TOP);
     if (t == 0) xexp[row] = e;
-    uint16_t* orow = out + (size_t)row * ldo;
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int c = t + 256 * u;
@@ -425,8 +421,8 @@ __global__ __launch_bounds__(256) void prefill_rmsnorm_xp_kernel(const float* __
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = __builtin_amdgcn_ldexpf(y[u][i], -e);  // zero past d
-        *(uint4*)(orow + c * 8) = make_uint4(pack_half2(v[0], v[4]), pack_half2(v[1], v[5]), pack_half2(v[2], v[6]),
-                                             pack_half2(v[3], v[7]));
+        ((uint4*)out)[xp_index(row, c, ldo >> 3)] = make_uint4(pack_half2(v[0], v[4]), pack_half2(v[1], v[5]),
+                                                               pack_half2(v[2], v[6]), pack_half2(v[3], v[7]));
     }
 }
 
@@ -450,40 +446,6 @@ struct EpiGemmSwiGLU {
             make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
     }
 };
-
-__global__ __launch_bounds__(256) void prefill_swiglu_xp_kernel(const float* __restrict__ gu, int ff,
-                                                               uint16_t* __restrict__ out, int ldo,
-                                                               int* __restrict__ xexp) {
-    extern __shared__ uint16_t hrow[];
-    __shared__ float red4[4];
-    const int row = blockIdx.x;
-    const float* g = gu + (size_t)row * 2 * ff;
-    float mx = 0.0f;
-    for (int j = threadIdx.x; j < ldo; j += 256) {
-        uint16_t hb = 0;
-        if (j < ff) {
-            const int b = j >> 3, rr = j & 7;
-            hb = swiglu_bf16(g[16 * b + rr], g[16 * b + 8 + rr]);
-            mx = fmaxf(mx, fabsf(bf16_bits_to_f32(hb)));
-        }
-        hrow[j] = hb;
-    }
-    const int e = range_exp(block_absmax256(mx, red4), XPREP_TOP);  // its barrier also orders hrow
-    if (threadIdx.x == 0) xexp[row] = e;
-    uint16_t* orow = out + (size_t)row * ldo;
-    for (int c = threadIdx.x; c * 8 < ldo; c += 256) {
-        const uint4 hv = *(const uint4*)&hrow[c * 8];
-        const uint32_t w4[4] = {hv.x, hv.y, hv.z, hv.w};
-        float y[8];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            y[2 * i] = __builtin_amdgcn_ldexpf(bf16_bits_to_f32(w4[i] & 0xFFFF), -e);
-            y[2 * i + 1] = __builtin_amdgcn_ldexpf(bf16_bits_to_f32(w4[i] >> 16), -e);
-        }
-        *(uint4*)(orow + c * 8) = make_uint4(pack_half2(y[0], y[4]), pack_half2(y[1], y[5]), pack_half2(y[2], y[6]),
-                                             pack_half2(y[3], y[7]));
-    }
-}
 
 // The last prompt row into the decode engine's residual, with the
 // per-16-element sums of squares its RMSNorm prologue reads.
@@ -569,7 +531,7 @@ struct th_llama {
     size_t pf_rows = 0;
     float *pf_x = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_y = nullptr, *pf_gu = nullptr;
     uint16_t *pf_xb = nullptr, *pf_att = nullptr, *pf_sg = nullptr;
-    int* pf_xe = nullptr;  // row exponents of prepared pf_xb, pf_att, pf_sg ([3][rows])
+    int* pf_xe = nullptr;  // row exponents of prepared pf_xb, pf_att ([2][rows])
     int32_t* pf_tok = nullptr;
 };
 
@@ -754,10 +716,11 @@ static void prefill_reserve(th_llama* m, size_t rows) {
     m->pf_qkv = dalloc<float>(rows * (m->qd + 2 * m->kvd));
     m->pf_q = dalloc<float>(rows * m->qd);
     m->pf_gu = dalloc<float>(rows * 2 * ff);
-    m->pf_xb = dalloc<uint16_t>(rows * round_up(d, 128));  // bf16 rows, or prepared rows of Kp
-    m->pf_att = dalloc<uint16_t>(rows * round_up((size_t)m->qd, 128));
-    m->pf_sg = dalloc<uint16_t>(rows * round_up(ff, 128));
-    m->pf_xe = dalloc<int>(3 * rows);
+    const size_t rows16 = round_up(rows, 16);  // prepared rows come in blocks of 16
+    m->pf_xb = dalloc<uint16_t>(rows16 * round_up(d, 128));  // bf16 rows, or prepared rows of Kp
+    m->pf_att = dalloc<uint16_t>(rows16 * round_up((size_t)m->qd, 128));
+    m->pf_sg = dalloc<uint16_t>(rows16 * round_up(ff, 128));
+    m->pf_xe = dalloc<int>(2 * rows);
     m->pf_tok = dalloc<int32_t>(rows);
     m->pf_rows = rows;
 }
@@ -811,28 +774,6 @@ static void prefill_rmsnorm_xp(const float* x, const uint16_t* w, int d, float e
     TH_LAUNCH_CHECK();
 }
 
-// A prefill linear with its epilogue fused (no split-K: used from
-// PREFILL_FUSED_ROWS rows, where the grid covers the chip without it).
-constexpr size_t PREFILL_FUSED_ROWS = 256;
-template <typename Epi>
-static void prefill_gemm_epi(const th_qweight* w, PreparedX xp, size_t n, const Epi& epi, hipStream_t s) {
-    const size_t NT = w->Np / 16;
-    const int GQ = (int)(w->Kp / 128);
-    GemmDense src;
-    src.M = (int)n;
-    if (n <= 1024)
-        TH_LAUNCH((q4_gemm_mfma_kernel<2, 4, _Float16, GemmDense, Epi>),
-                  dim3((unsigned)ceil_div(NT, (size_t)8), (unsigned)ceil_div(n, (size_t)64), 1), dim3(256), 0, s,
-                  (const uint4*)w->data, (const _Float16*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
-                  (int)w->rows, (int)w->cols, (int)w->Kp, (int)w->Kp, GQ);
-    else
-        TH_LAUNCH((q4_gemm_mfma_kernel<2, 8, _Float16, GemmDense, Epi>),
-                  dim3((unsigned)ceil_div(NT, (size_t)8), (unsigned)ceil_div(n, (size_t)128), 1), dim3(256), 0, s,
-                  (const uint4*)w->data, (const _Float16*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
-                  (int)w->rows, (int)w->cols, (int)w->Kp, (int)w->Kp, GQ);
-    TH_LAUNCH_CHECK();
-}
-
 static void prefill_chunk(th_llama* m, const int32_t* tok_host, size_t n, size_t pos0) {
     const th_llama_config& c = m->cfg;
     th_device* dev = m->dev;
@@ -843,11 +784,10 @@ static void prefill_chunk(th_llama* m, const int32_t* tok_host, size_t n, size_t
     TH_LAUNCH_CHECK();
     const size_t cache_layer = (size_t)c.max_seq * m->kvd;
     // Above 16 rows the linears run on the MFMA GEMM, whose activation layout
-    // the RMSNorm and SwiGLU kernels then write directly.
+    // the RMSNorm and attention kernels then write directly.
     const bool xp = n > 16;
-    int* xe_xb = m->pf_xe;  // row exponents of the prepared pf_xb, pf_att, pf_sg
+    int* xe_xb = m->pf_xe;  // row exponents of the prepared pf_xb, pf_att
     int* xe_att = m->pf_xe + m->pf_rows;
-    int* xe_sg = m->pf_xe + 2 * m->pf_rows;
     auto prefill_norm = [&](const uint16_t* w, const th_qweight* consumer) {
         if (xp && d <= 8192 && (int)consumer->Kp <= 8192)
             prefill_rmsnorm_xp(m->pf_x, w, d, c.eps, m->pf_xb, (int)consumer->Kp, xe_xb, n, s);
@@ -859,32 +799,26 @@ static void prefill_chunk(th_llama* m, const int32_t* tok_host, size_t n, size_t
                                c.eps, m->pf_xb, d, (int*)nullptr);
         TH_LAUNCH_CHECK();
     };
-    auto linear = [&](const th_qweight* w, const uint16_t* xin, const int* xe, int k, float* y, int ldy) {
-        if (xp) launch_q4_linear_prepared(w, PreparedX{xin, xe}, n, y, ldy, s, dev);
-        else launch_q4_linear(w, xin, TH_BF16, n, k, y, ldy, s, dev);
+    auto linear = [&](const th_qweight* w, const uint16_t* xin, int k, float* y, int ldy) {
+        launch_q4_linear(w, xin, TH_BF16, n, k, y, ldy, s, dev);
     };
     // split attention: few enough splits that q_len * heads * splits records fit the scratch
     const size_t attended = pos0 + n;
     const int subs = (int)std::max<size_t>(1, ceil_div(attended, (size_t)ATTN_SUB * 8));
     const int n_splits = (int)ceil_div(attended, (size_t)subs * ATTN_SUB);
-    // From PREFILL_FUSED_ROWS rows: RoPE/KV append in the QKV GEMM epilogue,
-    // SwiGLU in the gate/up GEMM epilogue (engine weights: f16 scales)
-    const bool fused = xp && n >= PREFILL_FUSED_ROWS && m->wqkv[0]->scale_dtype == TH_F16 &&
-                       m->wgu[0]->scale_dtype == TH_F16;
     for (int l = 0; l < c.n_layers; l++) {
         _Float16* kc = m->kcache + l * cache_layer;
         _Float16* vc = m->vcache + l * cache_layer;
         prefill_norm(m->attn_norm + (size_t)l * d, m->wqkv[l]);
-        if (fused) {  // RoPE and the K/V append in the QKV GEMM's epilogue
-            prefill_gemm_epi(m->wqkv[l], PreparedX{m->pf_xb, xe_xb}, n,
-                             EpiGemmQKVRope{m->pf_q, kc, vc, m->rope_cos, m->rope_sin, (int)pos0, m->qd, m->kvd, hd},
-                             s);
+        if (xp) {  // RoPE and the K/V append in the QKV GEMM's epilogue (engine weights: f16 scales)
+            q4_gemm_dense<_Float16>(m->wqkv[l], PreparedX{m->pf_xb, xe_xb}, n,
+                                    EpiGemmQKVRope{m->pf_q, kc, vc, m->rope_cos, m->rope_sin, (int)pos0, m->qd, m->kvd, hd},
+                                    s);
         } else {
-        linear(m->wqkv[l], m->pf_xb, xe_xb, d, m->pf_qkv, W);
-        TH_LAUNCH(prefill_rope_kv_kernel, dim3((unsigned)ceil_div((size_t)W / 8, (size_t)256), (unsigned)n), dim3(256),
-                  0, s, m->pf_qkv, (int)pos0,
-                           m->rope_cos, m->rope_sin, m->qd, m->kvd, hd, m->pf_q, kc, vc);
-        TH_LAUNCH_CHECK();
+            linear(m->wqkv[l], m->pf_xb, d, m->pf_qkv, W);
+            TH_LAUNCH(prefill_rope_kv_kernel, dim3((unsigned)ceil_div((size_t)W / 8, (size_t)256), (unsigned)n),
+                      dim3(256), 0, s, m->pf_qkv, (int)pos0, m->rope_cos, m->rope_sin, m->qd, m->kvd, hd, m->pf_q, kc, vc);
+            TH_LAUNCH_CHECK();
         }
         const bool xp_att = xp && (hd == 64 || hd == 128);
         if (hd == 64 || hd == 128) {  // causal flash attention on MFMA
@@ -897,41 +831,29 @@ static void prefill_chunk(th_llama* m, const int32_t* tok_host, size_t n, size_t
                                     n_splits, part, counters, (void*)m->pf_att, nullptr, s);
         }
         if (xp_att) {  // x += att.Wo^T in the GEMM's epilogue
-            launch_q4_linear_prepared(m->wo[l], PreparedX{m->pf_att, xe_att}, n, m->pf_x, d, s, dev, true);
+            launch_q4_linear_prepared(m->wo[l], PreparedX{m->pf_att, xe_att}, n, m->pf_x, d, s, true);
         } else {
             launch_q4_linear(m->wo[l], m->pf_att, TH_BF16, n, m->qd, m->pf_y, d, s, dev);
             TH_LAUNCH(prefill_add_kernel, dim3(1024), dim3(256), 0, s, m->pf_x, m->pf_y, n * d);
             TH_LAUNCH_CHECK();
         }
         prefill_norm(m->ffn_norm + (size_t)l * d, m->wgu[l]);
-        if (fused) {
+        if (xp) {
             // SwiGLU in the gate/up GEMM's epilogue (bf16 rows in pf_gu's
             // memory), prepared for the down GEMM by the activation pass, and
             // x += sg.Wd^T in the down GEMM's epilogue
             uint16_t* h = (uint16_t*)m->pf_gu;
-            prefill_gemm_epi(m->wgu[l], PreparedX{m->pf_xb, xe_xb}, n, EpiGemmSwiGLU{h, ff}, s);
+            q4_gemm_dense<_Float16>(m->wgu[l], PreparedX{m->pf_xb, xe_xb}, n, EpiGemmSwiGLU{h, ff}, s);
             const PreparedX sg = prepare_x(dev, h, false, n, ff, ff, m->wd[l]->Kp, s);
-            launch_q4_linear_prepared(m->wd[l], sg, n, m->pf_x, d, s, dev, true);
+            launch_q4_linear_prepared(m->wd[l], sg, n, m->pf_x, d, s, true);
             continue;
         }
-        linear(m->wgu[l], m->pf_xb, xe_xb, d, m->pf_gu, 2 * ff);
-        if (xp) {
-            const int ldo = (int)m->wd[l]->Kp;
-            TH_REQUIRE(ldo * 2 <= 64 * 1024, "prefill: d_ff above 32768");
-            TH_LAUNCH(prefill_swiglu_xp_kernel, dim3((unsigned)n), dim3(256), (size_t)ldo * 2, s, m->pf_gu,
-                               ff, m->pf_sg, ldo, xe_sg);
-        } else {
-            TH_LAUNCH(prefill_swiglu_kernel, dim3(8, (unsigned)n), dim3(256), 0, s, m->pf_gu, ff, m->pf_sg,
-                               ff);
-        }
+        linear(m->wgu[l], m->pf_xb, d, m->pf_gu, 2 * ff);
+        TH_LAUNCH(prefill_swiglu_kernel, dim3(8, (unsigned)n), dim3(256), 0, s, m->pf_gu, ff, m->pf_sg, ff);
         TH_LAUNCH_CHECK();
-        if (xp) {  // x += sg.Wd^T in the GEMM's epilogue
-            launch_q4_linear_prepared(m->wd[l], PreparedX{m->pf_sg, xe_sg}, n, m->pf_x, d, s, dev, true);
-        } else {
-            linear(m->wd[l], m->pf_sg, nullptr, ff, m->pf_y, d);
-            TH_LAUNCH(prefill_add_kernel, dim3(1024), dim3(256), 0, s, m->pf_x, m->pf_y, n * d);
-            TH_LAUNCH_CHECK();
-        }
+        linear(m->wd[l], m->pf_sg, ff, m->pf_y, d);
+        TH_LAUNCH(prefill_add_kernel, dim3(1024), dim3(256), 0, s, m->pf_x, m->pf_y, n * d);
+        TH_LAUNCH_CHECK();
     }
 }
 

@@ -591,13 +591,14 @@ static void moe_grouped_gemm(const th_moe* m, const th_qweight* w0, const uint4*
                              const _Float16* const* scales, const int* const* wexps, const uint16_t* x, size_t x_rows,
                              const int* slot_token, size_t max_work, Epi epi) {
     // the x_rows activation rows (tokens, or slots) prepared once
-    const PreparedX xp = prepare_x(m->dev, x, false, x_rows, w0->cols, w0->cols, w0->Kp, m->dev->stream);
+    const PreparedX xp =
+        prepare_x(m->dev, x, false, x_rows, w0->cols, w0->cols, w0->Kp, m->dev->stream, nullptr, nullptr, false);
     MoeGemmSrc src{m->work, data, scales, wexps, slot_token};
     const unsigned gx = (unsigned)ceil_div(w0->Np / 16, (size_t)(4 * MOE_GEMM_RT));
     TH_LAUNCH((q4_gemm_mfma_kernel<MOE_GEMM_RT, MOE_GEMM_CB, _Float16, MoeGemmSrc, Epi>),
                        dim3(gx, (unsigned)max_work, 1), dim3(256), 0, m->dev->stream, (const uint4*)nullptr,
                        (const _Float16*)nullptr, (const int*)nullptr, xp.x, xp.xexp, epi, src, (int)w0->rows,
-                       (int)w0->cols, (int)w0->Kp, (int)w0->Kp, (int)(w0->Kp / 128));
+                       (int)w0->Kp, (int)w0->Kp);
     TH_LAUNCH_CHECK();
 }
 

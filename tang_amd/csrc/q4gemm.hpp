@@ -1,0 +1,96 @@
+// Launchers of the dense int4 MFMA GEMM (prepared activations) with any
+// epilogue: the linear entry points store, the prefill fuses RoPE and SwiGLU.
+#pragma once
+
+#include <algorithm>
+#include <map>
+#include <mutex>
+
+#include "capi_util.hpp"
+#include "qlinear.hpp"
+
+namespace th {
+
+// Raise a kernel's dynamic-LDS limit (once per kernel and size).
+template <typename K>
+inline void set_smem(K kernel, size_t bytes) {
+    static std::mutex mu;
+    static std::map<const void*, size_t> done;
+    if (bytes <= 48 * 1024) return;
+    std::lock_guard<std::mutex> lock(mu);
+    size_t& d = done[(const void*)kernel];
+    if (bytes > d) {
+        TH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+        d = bytes;
+    }
+}
+
+template <int RT, int CB, int KW, typename ST, typename Epi>
+inline void q4_wave_launch(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
+    GemmDense src;
+    src.M = (int)m;
+    auto k = q4_gemm_wave_kernel<RT, CB, KW, ST, GemmDense, Epi>;
+    const size_t lds = (size_t)KW * RT * CB * 1024;
+    set_smem(k, lds);
+    TH_LAUNCH(k, dim3((unsigned)ceil_div(w->Np / 16, (size_t)RT), (unsigned)ceil_div(m, (size_t)(16 * CB))), dim3(64 * KW),
+              lds, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
+              (int)w->rows, (int)w->Kp, (int)w->Kp);
+    TH_LAUNCH_CHECK();
+}
+
+// Weight tiles and waves of a workgroup by the number of workgroups that four
+// tiles each would give (`wgs`): the more there are, the larger the tile and
+// the fewer the waves that split its K.  Measured, us (4x4 / 4x8 / 2x8 / 1x8,
+// tiles x waves): 2048 x 2048, m = 512 (256) 15.9 / 15.4 / 18.4 / 21.8; m = 384
+// (192) 14.8 / 14.3 / 17.1 / 18.0; m = 192 (96) 13.9 / 12.9 / 11.2 / 13.2;
+// m = 64 (32) 13.4 / 11.9 / 10.1 / 9.4; 11008 x 4096, m = 96 (344) 26.2 / 29.4 /
+// 30.0 / 38.4.  Up to 32 rows four tiles never pay (22016 x 4096, m = 32: 4x4
+// 22.0, 2x4 19.7, 2x8 20.5), and a single block of rows over a long K takes
+// sixteen waves (4096 x 11008, m = 16: 1x8 14.8, 1x16 13.3).
+template <int CB, typename ST, typename Epi>
+inline void q4_wave_shape(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
+    const size_t wgs = ceil_div(w->Np / 16, (size_t)4) * ceil_div(m, (size_t)(16 * CB));
+    if constexpr (CB <= 2) {
+        if (wgs > 144) return q4_wave_launch<2, CB, 4, ST>(w, xp, m, epi, s);
+    } else {
+        if (wgs > 224) return q4_wave_launch<4, CB, 4, ST>(w, xp, m, epi, s);
+        if (wgs > 144) return q4_wave_launch<4, CB, 8, ST>(w, xp, m, epi, s);
+    }
+    if (wgs > 72) return q4_wave_launch<2, CB, 8, ST>(w, xp, m, epi, s);
+    if constexpr (CB == 1) {
+        if (w->Kp >= 32 * 128) return q4_wave_launch<1, CB, 16, ST>(w, xp, m, epi, s);
+    }
+    q4_wave_launch<1, CB, 8, ST>(w, xp, m, epi, s);
+}
+
+template <int RT, int CB, typename ST, typename Epi>
+inline void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
+    GemmDense src;
+    src.M = (int)m;
+    TH_LAUNCH((q4_gemm_mfma_kernel<RT, CB, ST, GemmDense, Epi>),
+              dim3((unsigned)ceil_div(w->Np / 16, (size_t)(4 * RT)), (unsigned)ceil_div(m, (size_t)(16 * CB)), 1), dim3(256),
+              0, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
+              (int)w->rows, (int)w->Kp, (int)w->Kp);
+    TH_LAUNCH_CHECK();
+}
+
+// The kernel with activations staged in LDS once a workgroup's waves would
+// load them from L2 too often: from some 5600 tiles of 64 x 64 (us, wave kernel
+// / this one: 22016 x 4096, m = 768 191 / 199, 1024 253 / 249, 1536 381 / 364;
+// 11008 x 4096, m = 1536 195 / 220; 4096 x 4096 79 / 102).  128-row blocks
+// beyond m = 1024, 64-row ones before.
+template <typename ST, typename Epi>
+inline void q4_gemm_dense(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
+    const size_t tiles = ceil_div(w->Np / 16, (size_t)4) * ceil_div(m, (size_t)64);
+    if (tiles >= 5600) {
+        if (m > 1024) q4_mfma_launch<2, 8, ST>(w, xp, m, epi, s);
+        else q4_mfma_launch<2, 4, ST>(w, xp, m, epi, s);
+        return;
+    }
+    if (m <= 16) q4_wave_shape<1, ST>(w, xp, m, epi, s);
+    else if (m <= 32) q4_wave_shape<2, ST>(w, xp, m, epi, s);
+    else if (m <= 48) q4_wave_shape<3, ST>(w, xp, m, epi, s);
+    else q4_wave_shape<4, ST>(w, xp, m, epi, s);
+}
+
+}  // namespace th

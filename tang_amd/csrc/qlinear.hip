@@ -1,28 +1,13 @@
 // Launchers and C entry points for the quantized linear kernels.
 #include <cstdlib>
-#include <map>
-#include <mutex>
 
 #include "aql.hpp"
 #include "capi_util.hpp"
+#include "q4gemm.hpp"
 #include "q8gemm.hpp"
 #include "qlinear.hpp"
 
 namespace th {
-
-// Raise a kernel's dynamic-LDS limit (once per kernel and size).
-template <typename K>
-static void set_smem(K kernel, size_t bytes) {
-    static std::mutex mu;
-    static std::map<const void*, size_t> done;
-    if (bytes <= 48 * 1024) return;
-    std::lock_guard<std::mutex> lock(mu);
-    size_t& d = done[(const void*)kernel];
-    if (bytes > d) {
-        TH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-        d = bytes;
-    }
-}
 
 // Whether a q8 linear runs as GEMV launches of four rows: up to four rows,
 // and up to eight on a matrix of at most 4M weights, where two launches cost
@@ -183,12 +168,12 @@ void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_
 
 // Convert m activation rows (f32 or bf16, rows of ldx) into the MFMA GEMM's
 // prepared layout in the device's operand workspace.
-size_t prepared_x_bytes(size_t m, size_t Kp) { return round_up(m * Kp * 2, 256) + round_up(m * sizeof(int), 256); }
+size_t prepared_x_bytes(size_t m, size_t Kp) { return round_up(m, 16) * Kp * 2 + round_up(m * sizeof(int), 256); }
 
 PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t ldx, size_t K, size_t Kp,
-                    hipStream_t s, const int* rows, void* workspace) {
+                    hipStream_t s, const int* rows, void* workspace, bool blocked) {
     TH_REQUIRE(m * Kp * 2 < 0x7FFFFFF0u, "prepared activations above 2 GiB");  // 32-bit buffer offsets
-    const size_t xbytes = round_up(m * Kp * 2, 256);
+    const size_t xbytes = round_up(m, 16) * Kp * 2;
     char* ws = workspace ? (char*)workspace : (char*)device_scratch_x(dev, prepared_x_bytes(m, Kp));
     PreparedX p{(const uint16_t*)ws, (const int*)(ws + xbytes)};
     const size_t cpr = Kp / 8;
@@ -197,7 +182,7 @@ PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t l
             constexpr bool XF = decltype(xf)::value;
             constexpr int UU = decltype(u)::value;
             TH_LAUNCH((q4_gemm_xprep_row_kernel<XF, UU>), dim3((unsigned)m), dim3(256), 0, s, x, (int)ldx, (int)K,
-                      (int)Kp, rows, (uint4*)ws, (int*)(ws + xbytes));
+                      (int)Kp, (int)blocked, rows, (uint4*)ws, (int*)(ws + xbytes));
         };
         auto by_u = [&](auto xf) {
             if (cpr <= 256) row_kernel(xf, std::integral_constant<int, 1>{});
@@ -213,66 +198,23 @@ PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t l
     const unsigned grid = (unsigned)ceil_div(m, (size_t)4);
     if (xf32)
         TH_LAUNCH((q4_gemm_xprep_kernel<true>), dim3(grid), dim3(256), 0, s, x, (int)ldx, (int)K, (int)Kp,
-                           (int)m, rows, (uint4*)ws, (int*)(ws + xbytes));
+                           (int)m, (int)blocked, rows, (uint4*)ws, (int*)(ws + xbytes));
     else
         TH_LAUNCH((q4_gemm_xprep_kernel<false>), dim3(grid), dim3(256), 0, s, x, (int)ldx, (int)K, (int)Kp,
-                           (int)m, rows, (uint4*)ws, (int*)(ws + xbytes));
+                           (int)m, (int)blocked, rows, (uint4*)ws, (int*)(ws + xbytes));
     TH_LAUNCH_CHECK();
     return p;
 }
 
-// A caller-provided workspace for the split-K partials (part_bytes of it);
-// with none the device's grow-only workspace is used.
-struct SplitWorkspace {
-    float* part = nullptr;
-    size_t part_bytes = 0;
-};
-
-template <int RT, int CB, typename ST>
-static void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
-                           th_device* dev, bool accumulate, SplitWorkspace sw) {
-    const size_t NT = w->Np / 16, GQ = w->Kp / 128;
-    const unsigned gx = (unsigned)ceil_div(NT, 4 * RT);
-    const unsigned gy = (unsigned)ceil_div(m, 16 * CB);
-    // Split K so that the grid covers the chip at least twice (and, with a
-    // caller's workspace, only as far as its partials fit).
-    const size_t target = 2 * (size_t)(dev ? dev->num_cus : 256);
-    const size_t part_row = m * w->rows * sizeof(float);
-    size_t ks = 1;
-    while ((size_t)gx * gy * ks < target && ks * 2 <= GQ && ks < 16 &&
-           (!sw.part || ks * 2 * part_row <= sw.part_bytes))
-        ks *= 2;
-    const int gps = (int)ceil_div(GQ, ks);
-    ks = ceil_div(GQ, (size_t)gps);
-    float* out = y;
-    int ldo = (int)ldy;
-    if (ks > 1) {
-        out = sw.part ? sw.part : (float*)device_scratch(dev, ks * part_row);
-        ldo = (int)w->rows;
-    }
-    GemmDense src;
-    src.M = (int)m;
-    EpiGemmStore epi{out, ldo, (size_t)m * (size_t)ldo, ks > 1 ? 0 : (int)accumulate};
-    TH_LAUNCH((q4_gemm_mfma_kernel<RT, CB, ST, GemmDense, EpiGemmStore>), dim3(gx, gy, (unsigned)ks),
-                       dim3(256), 0, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x,
-                       xp.xexp, epi, src, (int)w->rows, (int)w->cols, (int)w->Kp, (int)w->Kp, gps);
-    TH_LAUNCH_CHECK();
-    if (ks > 1) launch_splitk_reduce(out, y, m, w->rows, ldy, ks, accumulate, s);
-}
-
-// Tile shape by batch size: one 16-row block up to 16 rows; 64-row column
-// blocks up to M=1024, 128-row blocks beyond (measured best of 2x4, 1x8, 2x6,
-// 2x8, 4x4, 4x8).
 template <typename ST>
-static void q4_mfma_dispatch(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
-                             th_device* dev, bool accumulate, SplitWorkspace sw = SplitWorkspace{}) {
-    if (m <= 16) q4_mfma_launch<1, 1, ST>(w, xp, m, y, ldy, s, dev, accumulate, sw);
-    else if (m <= 1024) q4_mfma_launch<2, 4, ST>(w, xp, m, y, ldy, s, dev, accumulate, sw);
-    else q4_mfma_launch<2, 8, ST>(w, xp, m, y, ldy, s, dev, accumulate, sw);
+static void q4_gemm_store(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
+                          bool accumulate) {
+    const bool vec4 = w->rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0;
+    q4_gemm_dense<ST>(w, xp, m, EpiGemmStore{y, (int)ldy, (int)accumulate, vec4}, s);
 }
 
 // ws (optional, ws_bytes long): the caller's workspace for the MFMA path's
-// prepared activations followed by its split-K partials.
+// prepared activations.
 template <bool XF32, typename ST>
 static void q4_linear_t(const th_qweight* w, const void* x, size_t m, size_t ldx, float* y, size_t ldy,
                         hipStream_t s, th_device* dev, void* ws = nullptr, size_t ws_bytes = 0) {
@@ -290,26 +232,24 @@ static void q4_linear_t(const th_qweight* w, const void* x, size_t m, size_t ldx
     else if (!XF32 && m <= 8 && fits8) q4_span_launch<8, false, ST>(w, x, m, ldx, y, ldy, s, cus);
     else if (!XF32 && m <= 16 && fits16) q4_span_launch<16, false, ST>(w, x, m, ldx, y, ldy, s, cus);
     else {  // activations prepared once per call, then the MFMA GEMM
-        SplitWorkspace sw;
-        void* xws = nullptr;
         if (ws) {
             const size_t xb = prepared_x_bytes(m, w->Kp);
-            TH_REQUIRE(xb <= ws_bytes, "workspace too small for the prepared activations (m x K too large)");
-            xws = ws;
-            sw.part = (float*)((char*)ws + xb);
-            sw.part_bytes = ws_bytes - xb;
+            // the whole blocks' padding rows go into the workspace's slack
+            TH_REQUIRE(round_up(m * w->Kp * 2, 256) + round_up(m * sizeof(int), 256) <= TH_NOALLOC_SCRATCH_BYTES &&
+                           xb <= ws_bytes,
+                       "workspace too small for the prepared activations (m x K too large)");
         }
-        const PreparedX xp = prepare_x(dev, x, XF32, m, ldx, w->cols, w->Kp, s, nullptr, xws);
-        q4_mfma_dispatch<ST>(w, xp, m, y, ldy, s, dev, false, sw);
+        const PreparedX xp = prepare_x(dev, x, XF32, m, ldx, w->cols, w->Kp, s, nullptr, ws);
+        q4_gemm_store<ST>(w, xp, m, y, ldy, s, false);
     }
 }
 
 void launch_q4_linear_prepared(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
-                               th_device* dev, bool accumulate) {
+                               bool accumulate) {
     TH_REQUIRE(w && w->bits == 4, "not a q4 weight");
     if (m == 0) return;
-    if (w->scale_dtype == TH_F16) q4_mfma_dispatch<_Float16>(w, xp, m, y, ldy, s, dev, accumulate);
-    else q4_mfma_dispatch<float>(w, xp, m, y, ldy, s, dev, accumulate);
+    if (w->scale_dtype == TH_F16) q4_gemm_store<_Float16>(w, xp, m, y, ldy, s, accumulate);
+    else q4_gemm_store<float>(w, xp, m, y, ldy, s, accumulate);
 }
 
 void launch_q4_linear(const th_qweight* w, const void* x, th_dtype xdt, size_t m, size_t ldx, float* y,
@@ -456,7 +396,7 @@ int th_gemm_q4_noalloc(th_device* dev, const th_buffer* x, size_t m, const th_qw
     require_len_any(x, m * w->cols, "x");
     require_len(y, TH_F32, m * w->rows, "y");
     launch_q4_linear(w, x->ptr, x->dtype, m, w->cols, (float*)y->ptr, w->rows, dev->stream, dev, dev->noalloc_scratch,
-                     TH_NOALLOC_SCRATCH_BYTES);
+                     TH_NOALLOC_SCRATCH_BYTES + NOALLOC_SLACK);
     TH_API_END
 }
 

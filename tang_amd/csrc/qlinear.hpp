@@ -989,9 +989,7 @@ __global__ __launch_bounds__(64 * NW) void q8_gemv_kernel(const uint4* __restric
 // of 16 activation rows.  Per group (K = 32 = one MFMA) a lane dequantises its
 // eight weights to f16 as (n-8)*s' (exact n-8 via the 1024+n magic, one f16
 // rounding of the product).  The activations come prepared (f16, permuted,
-// see q4_gemm_xprep_kernel) and go through LDS.  With KS > 1 each workgroup
-// covers a K slice and writes f32 partials [KS][m][n] that
-// splitk_reduce_kernel sums in a fixed order.
+// see q4_gemm_xprep_kernel) and go through LDS.
 //
 // Range: f16 holds 2^-14..65504 at full precision, far less than the f32 /
 // bf16 inputs of the reference's f64 q4_matvec (quantize.rs:256-289).  Both
@@ -1022,6 +1020,24 @@ __device__ __forceinline__ void nib_pairs_f16(uint32_t w, half2_t s2, half2_t ou
 __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
     half2_t h = {(_Float16)a, (_Float16)b};
     return __builtin_bit_cast(uint32_t, h);
+}
+
+// The prepared activations' layout: blocks of 16 rows, in each the rows' 8-value
+// chunks side by side, [row / 16][chunk][row % 16] in 16-byte units (cpr =
+// Kp / 8 chunks a row).  An MFMA operand of 16 rows x 32 k is then 1 KiB of
+// consecutive memory, one piece per lane: row-major, consecutive lanes are
+// rows apart and every 16 bytes is a cache access of its own (the dense GEMM
+// at M = 2048 lost 13% to it, at M = 64 16%).  The grouped source gathers its
+// rows one by one and keeps them row-major: there a line holds eight chunks of
+// the one row it needs (MoE, T = 512: 205 against 215 us).
+__host__ __device__ inline size_t xp_index(size_t row, size_t chunk, size_t cpr) {
+    return ((row >> 4) * cpr + chunk) * 16 + (row & 15);
+}
+// Row of workgroup i of m one-row workgroups: the 16 rows of a block go to
+// workgroups of one XCD (i mod 8), in whose L2 their pieces of a line meet.
+__device__ __forceinline__ int xp_block_row(int i, int m) {
+    const int g = i & ~127;
+    return g + 128 <= m ? g + (i & 7) * 16 + ((i >> 3) & 15) : i;
 }
 
 // Exponent that brings a row whose largest magnitude is mx to [2^(top-1),
@@ -1069,12 +1085,17 @@ struct GemmDense {
 struct EpiGemmStore {
     float* y;
     int ldy;
-    size_t split_stride;  // split-K partials: y + split * split_stride
-    int add = 0;          // y += v (a residual add, device.rs:721) instead of y = v
-    int split = 0;        // this workgroup's K split (set by the kernel)
+    int add;   // y += v (a residual add, device.rs:721) instead of y = v
+    int vec4;  // N and ldy are multiples of 4 and y is 16-byte aligned
     __device__ __forceinline__ void operator()(int out_row, int n0, int N, bool live, const float4_t& v) const {
         if (!live) return;
-        float* yb = y + (size_t)split * split_stride + (size_t)out_row * ldy;
+        float* yb = y + (size_t)out_row * ldy;
+        if (vec4) {  // whole, aligned quads (n0 is a multiple of 4)
+            if (n0 >= N) return;
+            float4_t* p = (float4_t*)(yb + n0);
+            *p = add ? *p + v : v;
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (n0 + i < N) yb[n0 + i] = add ? yb[n0 + i] + v[i] : v[i];
@@ -1084,7 +1105,8 @@ struct EpiGemmStore {
 // Activations prepared for the MFMA GEMM: one wave per row.  Pass 1
 // finds the row's largest magnitude, pass 2 writes x * 2^-xexp[row] as f16
 // (RNE; exact for a bf16 input within 2^26 of the row maximum), each 8-value
-// chunk in nibble-pair order (x0,x4,x1,x5,x2,x6,x3,x7), zero past K up to Kp.
+// chunk in nibble-pair order (x0,x4,x1,x5,x2,x6,x3,x7), zero past K up to Kp,
+// at xp_index.
 // Row r of the output is input row rows[r] (rows == nullptr: row r).
 template <bool XF32>
 __device__ __forceinline__ void xprep_load8(const void* xin, size_t ldx, int row, int K, int k0, bool vec, float xv[8]) {
@@ -1117,7 +1139,7 @@ __device__ __forceinline__ void xprep_load8(const void* xin, size_t ldx, int row
 
 template <bool XF32>
 __global__ __launch_bounds__(256) void q4_gemm_xprep_kernel(const void* __restrict__ xin, int ldx, int K, int Kp,
-                                                            int M, const int* __restrict__ rows,
+                                                            int M, int blocked, const int* __restrict__ rows,
                                                             uint4* __restrict__ out, int* __restrict__ xexp) {
     // one wave per row, four rows per workgroup
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1141,7 +1163,7 @@ __global__ __launch_bounds__(256) void q4_gemm_xprep_kernel(const void* __restri
         xprep_load8<XF32>(xin, (size_t)ldx, row, K, c * 8, vec, xv);
 #pragma unroll
         for (int i = 0; i < 8; i++) xv[i] = __builtin_amdgcn_ldexpf(xv[i], -e);
-        out[(size_t)r * cpr + c] = make_uint4(pack_half2(xv[0], xv[4]), pack_half2(xv[1], xv[5]),
+        out[blocked ? xp_index(r, c, cpr) : (size_t)r * cpr + c] = make_uint4(pack_half2(xv[0], xv[4]), pack_half2(xv[1], xv[5]),
                                               pack_half2(xv[2], xv[6]), pack_half2(xv[3], xv[7]));
     }
 }
@@ -1152,10 +1174,10 @@ __global__ __launch_bounds__(256) void q4_gemm_xprep_kernel(const void* __restri
 // not depend on the order).
 template <bool XF32, int U>
 __global__ __launch_bounds__(256) void q4_gemm_xprep_row_kernel(const void* __restrict__ xin, int ldx, int K, int Kp,
-                                                                const int* __restrict__ rows, uint4* __restrict__ out,
+                                                                int blocked, const int* __restrict__ rows, uint4* __restrict__ out,
                                                                 int* __restrict__ xexp) {
     __shared__ float red4[4];
-    const int r = blockIdx.x, t = threadIdx.x;
+    const int r = xp_block_row(blockIdx.x, gridDim.x), t = threadIdx.x;
     const int row = rows ? rows[r] : r;
     const int cpr = Kp >> 3;
     const bool vec = (ldx & 7) == 0 && (((uintptr_t)xin) & 15) == 0;
@@ -1182,13 +1204,12 @@ __global__ __launch_bounds__(256) void q4_gemm_xprep_row_kernel(const void* __re
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = __builtin_amdgcn_ldexpf(xv[u][i], -e);
-        out[(size_t)r * cpr + c] = make_uint4(pack_half2(v[0], v[4]), pack_half2(v[1], v[5]), pack_half2(v[2], v[6]),
+        out[blocked ? xp_index(r, c, cpr) : (size_t)r * cpr + c] = make_uint4(pack_half2(v[0], v[4]), pack_half2(v[1], v[5]), pack_half2(v[2], v[6]),
                                               pack_half2(v[3], v[7]));
     }
 }
 
-// Workgroup -> (weight block, activation block, K split) of a dense GEMM
-// grid.  Linear workgroup i runs on XCD i mod 8; this hands each XCD a
+// Workgroup -> (weight block, activation block, K split) of a GEMM grid.  Linear workgroup i runs on XCD i mod 8; this hands each XCD a
 // contiguous range of tiles of the (x, y + gy * z) plane, walked in bands of
 // 8 activation blocks, so the workgroups resident on one XCD share 8
 // activation and 8 weight blocks in its L2.
@@ -1206,25 +1227,25 @@ __device__ __forceinline__ void gemm_xcd_tile(int& bx, int& by, int& bz) {
     by = yz - bz * gy;
 }
 
-// xin: prepared rows (f16, ldx = Kp halves, row exponents xexp); wexp: the
+// xin: prepared rows (f16, xp_index with ldx = Kp, row exponents xexp); wexp: the
 // weight rows' scale exponents (th_qweight::row_exp).
 template <int RT, int CB, typename ST, typename Src = GemmDense, typename Epi = EpiGemmStore>
 __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restrict__ wt,
                                                            const ST* __restrict__ sc, const int* __restrict__ wexp,
                                                            const uint16_t* __restrict__ xin,
                                                            const int* __restrict__ xexp, Epi epi, Src src,
-                                                           int N, int K, int Kp, int ldx, int gq_per_split) {
+                                                           int N, int Kp, int ldx) {
     // LDS B tile: [CB][4 j][4 q][16 col] uint4 (8 f16 each)
     // two B tiles: the next group-quad's is written while this one is read,
     // so one barrier per step orders both
     __shared__ uint4 bt2[2][CB * 4 * 4 * 16];
-    int mrows = 0, tile_blk = 0, split = blockIdx.z;
+    int mrows = 0, tile_blk = 0;
     {
         const uint4* wsel = wt;
         const ST* ssel = sc;
         const int* esel = wexp;
-        int bx = blockIdx.x, by = blockIdx.y;
-        if constexpr (!Src::GROUPED) gemm_xcd_tile(bx, by, split);
+        int bx = blockIdx.x, by = blockIdx.y, bz = 0;
+        if constexpr (!Src::GROUPED) gemm_xcd_tile(bx, by, bz);
         tile_blk = bx;
         if (!src.select(by, CB * 16, wsel, ssel, esel, mrows)) return;
         wt = wsel;
@@ -1239,9 +1260,6 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
     const int q = lane >> 4, r = lane & 15;
     const int tile0 = (tile_blk * 4 + wave) * RT;  // first 16-row tile of this wave
     const int NT = (N + 15) >> 4;
-    const int gq0 = split * gq_per_split;
-    if constexpr (std::is_same<Epi, EpiGemmStore>::value) epi.split = split;
-    const int gq1 = min(GQ, gq0 + gq_per_split);
 
     float4_t acc[RT][CB];
 #pragma unroll
@@ -1253,12 +1271,12 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
 #pragma unroll
     for (int a = 0; a < RT; a++) wneg[a] = -wexp[min(tile0 + a, NT - 1) * 16 + r];
 
-    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xin, 0x7FFFFFF0u);  // in-range offsets only
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xin, 0xFFFFFFF0u);  // in-range offsets only
     // staging assignment: CB*16 cols * 16 chunks (4 groups x 4 quads) = CB*256 chunks.
     // A thread's chunks keep their row and their place in the group-quad
     // over the whole K loop: their offsets (for the grouped source, after the
     // slot -> token lookup) are formed once, so no step waits on that lookup.
-    uint32_t xoff[CB];   // halves: row * ldx + j * 32 + qq * 8
+    uint32_t xoff[CB];   // halves: place of the row's chunk 4j + qq (xp_index; grouped: row-major)
     bool xlive[CB];
 #pragma unroll
     for (int i = 0; i < CB; i++) {
@@ -1272,13 +1290,13 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
             // branch-free: rows past mrows re-read the last live row (a finite
             // copy whose D columns are never stored)
             xlive[i] = true;
-            xoff[i] = (uint32_t)(src.x_row(min(ml, mrows - 1)) * ldx + j * 32 + qq * 8);
+            xoff[i] = (uint32_t)xp_index(src.x_row(min(ml, mrows - 1)), j * 4 + qq, ldx >> 3) * 8u;
         }
     }
     auto load_x = [&](int gq, uint4 (&regs)[CB]) {
 #pragma unroll
         for (int i = 0; i < CB; i++) {
-            const uint32_t off = xoff[i] + (uint32_t)gq * 128u;
+            const uint32_t off = xoff[i] + (uint32_t)gq * (Src::GROUPED ? 128u : 2048u);
             if constexpr (Src::GROUPED) {
                 regs[i] = xlive[i] ? *(const uint4*)(xin + off) : make_uint4(0, 0, 0, 0);
             } else {
@@ -1307,15 +1325,13 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
             s.load(sc + q4_scale_index(std::is_same<ST, _Float16>::value, tt, gq, r, 0, GQ), a);
         }
     };
-    if (gq0 < gq1) {
-        load_x(gq0, xr);
-        load_w(gq0, wcur, scur);
-        store_x(bt2[0], xr);
-        __syncthreads();
-    }
-    for (int gq = gq0; gq < gq1; gq++) {
-        const uint4* bt = bt2[(gq - gq0) & 1];
-        const bool more = gq + 1 < gq1;
+    load_x(0, xr);
+    load_w(0, wcur, scur);
+    store_x(bt2[0], xr);
+    __syncthreads();
+    for (int gq = 0; gq < GQ; gq++) {
+        const uint4* bt = bt2[gq & 1];
+        const bool more = gq + 1 < GQ;
         if (more) {
             load_x(gq + 1, xr);
             load_w(gq + 1, wnxt, snxt);
@@ -1341,7 +1357,7 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
         }
         // the other tile was last read in the previous step, before the
         // barrier that ended it
-        if (more) store_x(bt2[(gq + 1 - gq0) & 1], xr);
+        if (more) store_x(bt2[(gq + 1) & 1], xr);
         __syncthreads();
 #pragma unroll
         for (int a = 0; a < RT; a++) wcur[a] = wnxt[a];
@@ -1369,6 +1385,125 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
             for (int i = 0; i < 4; i++) v[i] = __builtin_amdgcn_ldexpf(acc[a][b][i], xe[b] + wev[i]);
             epi(src.out_row(live ? ml : 0), n0, N, live, v);
         }
+    }
+}
+
+// The same product for batches whose grid does not fill the chip several
+// times over: a workgroup's KW waves share one tile of RT weight tiles x CB
+// activation blocks and split its K between them (wave w takes group-quads w,
+// w + KW, ...), each straight from memory to MFMA operands: no LDS staging, no
+// barrier and no split-K pass over memory.  A wave keeps a whole group-quad of
+// activations (two halves, each re-requested as soon as its MFMAs have read
+// it) and the next group-quad's weights in flight.
+// The waves' partial tiles meet in LDS, where wave w sums tiles w, w + KW, ...
+// in wave order and runs the epilogue on them.
+// Bound by latency on few rows, then by the activations' way from L2 (every
+// weight tile reads them again), which larger RT x CB tiles halve and halve
+// again.  us, against the LDS kernel with its split-K partials summed by a
+// second launch (same prepared layout): 2048 x 2048, m = 64 17.0 -> 9.4, m = 384
+// 25.7 -> 14.3; 4096 x 4096, m = 64 20.3 -> 13.0, m = 512 43 -> 33; 11008 x 4096,
+// m = 32 24.6 -> 14.5, m = 256 53 -> 40, m = 1024 145 -> 131 (705 TFLOP/s).
+template <int RT, int CB, int KW, typename ST, typename Src = GemmDense, typename Epi = EpiGemmStore>
+__global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __restrict__ wt, const ST* __restrict__ sc,
+                                                               const int* __restrict__ wexp,
+                                                               const uint16_t* __restrict__ xin,
+                                                               const int* __restrict__ xexp, Epi epi, Src src, int N,
+                                                               int Kp, int ldx) {
+    extern __shared__ __align__(16) char wave_lds[];
+    float4_t* part = (float4_t*)wave_lds;  // [KW][RT * CB][64]
+    int mrows = 0, bx = blockIdx.x, by = blockIdx.y, bz = 0;
+    if constexpr (!Src::GROUPED) gemm_xcd_tile(bx, by, bz);
+    {
+        const uint4* wsel = wt;
+        const ST* ssel = sc;
+        const int* esel = wexp;
+        if (!src.select(by, CB * 16, wsel, ssel, esel, mrows)) return;
+        wt = wsel;
+        sc = ssel;
+        wexp = esel;
+    }
+    const int GQ = Kp >> 7, NT = (N + 15) >> 4, tile0 = bx * RT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int steps = wave < GQ ? (GQ - wave + KW - 1) / KW : 0;
+    float4_t acc[RT][CB];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CB; b++) acc[a][b] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    int wneg[RT];
+#pragma unroll
+    for (int a = 0; a < RT; a++) wneg[a] = -wexp[min(tile0 + a, NT - 1) * 16 + r];
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xin, 0xFFFFFFF0u);  // in-range offsets only
+    uint32_t xoff[CB];  // bytes; rows past mrows re-read the last live row (never stored)
+#pragma unroll
+    for (int b = 0; b < CB; b++) xoff[b] = (uint32_t)xp_index(src.x_row(min(b * 16 + r, mrows - 1)), q, ldx >> 3) * 16u;
+    u32x4_t xh[2][2][CB];  // [half][group of the half][block]
+    auto load_x = [&](int gq, int h) {
+#pragma unroll
+        for (int b = 0; b < CB; b++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                xh[h][j][b] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[b] + (uint32_t)(gq * 4096 + h * 2048 + j * 1024), 0, 0);
+    };
+    u32x4_t wcur[RT], wnxt[RT];
+    ScaleVec<RT, ST> scur, snxt;
+    auto load_w = [&](int gq, u32x4_t (&w)[RT], ScaleVec<RT, ST>& s) {
+#pragma unroll
+        for (int a = 0; a < RT; a++) {
+            const int tt = min(tile0 + a, NT - 1);
+            w[a] = *(const u32x4_t*)(wt + ((size_t)tt * GQ + gq) * 64 + lane);
+            s.load(sc + q4_scale_index(std::is_same<ST, _Float16>::value, tt, gq, r, 0, GQ), a);
+        }
+    };
+    auto gq_of = [&](int i) { return wave + KW * min(i, steps - 1); };  // past the end: the last one again
+    if (steps > 0) {
+        load_w(gq_of(0), wcur, scur);
+        load_x(gq_of(0), 0);
+        load_x(gq_of(0), 1);
+    }
+    for (int i = 0; i < steps; i++) {
+        const int gn = gq_of(i + 1);
+        load_w(gn, wnxt, snxt);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int a = 0; a < RT; a++) {
+                    const _Float16 s = scur.get_ldexp(a, 2 * h + j, wneg[a]);
+                    const half2_t s2 = {s, s};
+                    half2_t p[4];
+                    nib_pairs_f16(wcur[a][2 * h + j], s2, p);
+                    const half8_t af = {p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y};
+#pragma unroll
+                    for (int b = 0; b < CB; b++)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, __builtin_bit_cast(half8_t, xh[h][j][b]),
+                                                                           acc[a][b], 0, 0, 0);
+                }
+            load_x(gn, h);
+        }
+#pragma unroll
+        for (int a = 0; a < RT; a++) wcur[a] = wnxt[a];
+        scur = snxt;
+    }
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CB; b++) part[(wave * RT * CB + a * CB + b) * 64 + lane] = acc[a][b];
+    __syncthreads();
+    for (int t = wave; t < RT * CB; t += KW) {
+        const int a = t / CB, b = t - a * CB, ml = b * 16 + r, tile = tile0 + a;
+        float4_t v = part[t * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < KW; w++) v += part[(w * RT * CB + t) * 64 + lane];
+        const int xe = xexp[src.x_row(ml < mrows ? ml : 0)];
+        const int4 we = *(const int4*)(wexp + min(tile, NT - 1) * 16 + 4 * q);
+        const int wev[4] = {we.x, we.y, we.z, we.w};
+        const bool live = ml < mrows && tile < NT;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_ldexpf(v[e], xe + wev[e]);
+        epi(src.out_row(live ? ml : 0), tile * 16 + 4 * q, N, live, v);
     }
 }
 

@@ -198,6 +198,34 @@ def test_q8_reference_blocks_per_group_scales(dev):
     assert max_abs_rel(y, ref) < TOL_F32
 
 
+@pytest.mark.parametrize("rows,cols,m", [
+    (40, 100, 20),       # one group-quad: all waves but one have no step
+    (1000, 1100, 17),    # nine group-quads over eight waves, two 16-row blocks
+    (500, 4200, 9),      # sixteen waves, fewer live rows than a block
+    (2500, 300, 33),     # three blocks
+    (4700, 520, 65),     # 64-row blocks with one live row in the last
+    (9000, 260, 130),    # four tiles, four waves
+    (22000, 200, 1050),  # activations staged in LDS, 128-row blocks
+    (44000, 140, 600),   # the same with 64-row blocks
+])
+@pytest.mark.parametrize("scales", ["f16", "f32"])
+def test_q4_gemm_shapes(dev, rows, cols, m, scales):
+    """Every tile and wave split of the dense int4 GEMM.  Weight and activation
+    are rounded to f16 once each (2^-11 of a product), the sums are f32."""
+    rng = np.random.default_rng(rows + m)
+    bpr = (cols + 31) // 32
+    nib = np.frombuffer(rng.bytes(rows * bpr * 16), np.uint8).reshape(rows, bpr * 16)
+    sc = rng.uniform(0.002, 0.01, (rows, bpr)).astype(np.float16 if scales == "f16" else np.float32)
+    w = dev.q4_upload_packed(nib, sc.view(np.uint16) if scales == "f16" else sc, rows, cols,
+                             capi.F16 if scales == "f16" else capi.F32)
+    x = (rng.standard_normal((m, cols)) * 10.0 ** rng.uniform(-6, 6, (m, 1))).astype(np.float32)
+    y = dev.gemm_q4(dev.upload(x), m, w).to_numpy().reshape(m, rows)
+    v = np.stack((nib & 15, nib >> 4), -1).reshape(rows, bpr, 32).astype(np.float64) - 8.0
+    wf = (v * sc.astype(np.float64)[:, :, None]).reshape(rows, -1)[:, :cols]
+    ref, mag = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    assert np.all(np.abs(y - ref) <= (2.0 ** -10 + cols * 2.0 ** -24) * mag)
+
+
 @pytest.mark.parametrize("rows,cols", [(16, 64), (37, 3), (130, 200), (2050, 1096), (512, 4096), (1100, 4096)])
 @pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 65, 129])  # either side of the 16/32/64/128-row blocks
 @pytest.mark.parametrize("scales", ["row", "group"])
