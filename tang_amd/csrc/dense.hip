@@ -270,9 +270,9 @@ static void matmul_launch(const MatOperand& A, const MatOperand& B, float* c, si
     const unsigned gx = (unsigned)ceil_div(n, (size_t)(4 / WGM * TN * 16)), gy = (unsigned)ceil_div(m, (size_t)(WGM * TM * 16));
     // Split K where the tiles leave CUs idle: two workgroups per CU, each
     // split at least 128 deep.  (While a stream is captured the workspace may
-    // not grow: a call that has none yet runs unsplit.)
+    // not grow: a call takes the splits that it holds.)
     size_t ks = std::max<size_t>(1, std::min({2 * cus / ((size_t)gx * gy), k / 128, (size_t)16}));
-    if (ks > 1 && ks * part > dev->scratch_bytes && stream_capturing(dev->stream)) ks = 1;
+    if (ks * part > dev->scratch_bytes && stream_capturing(dev->stream)) ks = std::max<size_t>(1, dev->scratch_bytes / part);
     const size_t per = round_up(ceil_div(k, ks), (size_t)32);
     ks = ceil_div(k, per);
     float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : c;

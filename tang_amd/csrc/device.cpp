@@ -29,6 +29,8 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 // Grow one of the device's workspaces to `bytes`.  Once a graph has been
 // captured on the device the outgrown block is kept (its graphs may name it)
 // and sizes double, so that the kept blocks stay below the one in use.
+constexpr size_t FIRST_WORKSPACE = (size_t)32 << 20;
+
 static void* grow_workspace(th_device* dev, void*& ptr, size_t& have, size_t bytes) {
     if (bytes <= have) return ptr;
     size_t want = std::max(bytes, (size_t)1 << 20);
@@ -254,6 +256,15 @@ int th_device_create(int ordinal, th_device** out) {
     hipDeviceProp_t prop;
     TH_HIP(hipGetDeviceProperties(&prop, ordinal));
     d->num_cus = prop.multiProcessorCount;
+    // Enough for the K splits of ordinary batches, so that a graph captured
+    // before any call of its size is not left unsplit.  Without it the device
+    // works all the same.
+    if (hipMalloc(&d->scratch, FIRST_WORKSPACE) == hipSuccess) {
+        d->scratch_bytes = FIRST_WORKSPACE;
+    } else {
+        d->scratch = nullptr;
+        (void)hipGetLastError();
+    }
     *out = d;
     TH_API_END
 }
