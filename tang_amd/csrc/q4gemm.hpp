@@ -63,6 +63,42 @@ inline void q4_wave_shape(const th_qweight* w, PreparedX xp, size_t m, const Epi
     q4_wave_launch<1, CB, 8, ST>(w, xp, m, epi, s);
 }
 
+template <int RT, int KW, typename ST, typename Epi>
+inline void q4_rows_launch(const th_qweight* w, const float* x, size_t m, size_t ldx, const Epi& epi, hipStream_t s) {
+    const size_t lds = (size_t)KW * 4096;
+    auto k = q4_gemm_rows_kernel<RT, KW, ST, Epi>;
+    set_smem(k, lds);
+    TH_LAUNCH(k, dim3((unsigned)ceil_div(w->Np / 16, (size_t)RT)), dim3(64 * KW), lds, s, (const uint4*)w->data,
+              (const ST*)w->scales, (const int*)w->row_exp, x, epi, (int)m, (int)w->rows, (int)w->cols, (int)w->Kp,
+              (int)ldx);
+    TH_LAUNCH_CHECK();
+}
+
+// Whether at most 16 rows of f32 go to q4_gemm_rows_kernel unprepared: the
+// preparation and its launch (4 to 6 us) against converting all of x again in
+// every workgroup.  us, prepared / not, m = 16: 256 x 1024 5.7 / 3.4, 2500 x 2500
+// 7.6 / 4.9, 2500 x 6700 11.7 / 9.5, 4096 x 11008 13.0 / 13.7; several workgroups a
+// CU: 6700 x 2500 8.3 / 6.3, 11264 x 2048 8.7 / 7.8, 11008 x 4096 12.1 / 12.7.
+// Rows that cannot be read in aligned fours are prepared (scalar loads took
+// 3333 x 3333 from 76 to 137 us over eight linears).
+inline bool q4_rows_direct(const th_qweight* w, const float* x, size_t m, size_t ldx) {
+    const size_t tiles = w->Np / 16;
+    return m <= 16 && w->cols % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
+           w->cols <= (tiles <= 256 ? 8192u : 3072u) && ldx < ((size_t)1 << 25);  // 32-bit offsets into 16 rows
+}
+
+// One weight tile a workgroup while that is at most one workgroup a CU, two
+// beyond, and four waves instead of eight once there are several (us at m = 16,
+// 1x8 / 2x8 / 2x4 tiles x waves: 2048 x 2048 4.4 / 5.1 / 5.4; 5632 x 2048 6.3 /
+// 5.2 / 5.5; 11264 x 2048 9.2 / 8.2 / 7.8).
+template <typename ST, typename Epi>
+inline void q4_gemm_rows(const th_qweight* w, const float* x, size_t m, size_t ldx, const Epi& epi, hipStream_t s) {
+    const size_t tiles = w->Np / 16;
+    if (tiles <= 256) q4_rows_launch<1, 8, ST>(w, x, m, ldx, epi, s);
+    else if (tiles <= 512) q4_rows_launch<2, 8, ST>(w, x, m, ldx, epi, s);
+    else q4_rows_launch<2, 4, ST>(w, x, m, ldx, epi, s);
+}
+
 template <int RT, int CB, typename ST, typename Epi>
 inline void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
     GemmDense src;

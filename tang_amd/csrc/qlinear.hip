@@ -206,11 +206,14 @@ PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t l
     return p;
 }
 
+static EpiGemmStore q4_store_epi(const th_qweight* w, float* y, size_t ldy, bool accumulate) {
+    return {y, (int)ldy, (int)accumulate, w->rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0};
+}
+
 template <typename ST>
 static void q4_gemm_store(const th_qweight* w, PreparedX xp, size_t m, float* y, size_t ldy, hipStream_t s,
                           bool accumulate) {
-    const bool vec4 = w->rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0;
-    q4_gemm_dense<ST>(w, xp, m, EpiGemmStore{y, (int)ldy, (int)accumulate, vec4}, s);
+    q4_gemm_dense<ST>(w, xp, m, q4_store_epi(w, y, ldy, accumulate), s);
 }
 
 // ws (optional, ws_bytes long): the caller's workspace for the MFMA path's
@@ -238,6 +241,12 @@ static void q4_linear_t(const th_qweight* w, const void* x, size_t m, size_t ldx
             TH_REQUIRE(round_up(m * w->Kp * 2, 256) + round_up(m * sizeof(int), 256) <= TH_NOALLOC_SCRATCH_BYTES &&
                            xb <= ws_bytes,
                        "workspace too small for the prepared activations (m x K too large)");
+        }
+        if constexpr (XF32) {
+            if (q4_rows_direct(w, (const float*)x, m, ldx)) {
+                q4_gemm_rows<ST>(w, (const float*)x, m, ldx, q4_store_epi(w, y, ldy, false), s);
+                return;
+            }
         }
         const PreparedX xp = prepare_x(dev, x, XF32, m, ldx, w->cols, w->Kp, s, nullptr, ws);
         q4_gemm_store<ST>(w, xp, m, y, ldy, s, false);

@@ -1507,4 +1507,140 @@ __global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __re
     }
 }
 
+// The wave kernel for at most 16 rows of f32 that nothing has prepared: each
+// wave brings its own part of them to f16 on the way, so a call is one launch
+// and needs no workspace.  Four lanes read 128 bytes of a row, which LDS turns
+// into MFMA operands.  The power of two that the preparation takes from a whole
+// row here follows the largest magnitude the wave has met so far: the sums are
+// scaled down, exactly, when a larger one comes, and no value keeps fewer bits
+// than with the row's.  Every workgroup converts all the rows again (K / KW
+// values of 16 rows a wave), which is why more rows are prepared once instead.
+// Bound by latency: 2048 x 2048, m = 16 6.3 us in two launches -> 4.4.
+// Needs K % 4 == 0, ldx % 4 == 0 and a 16-byte aligned x.
+template <int RT, int KW, typename ST, typename Epi>
+__global__ __launch_bounds__(64 * KW) void q4_gemm_rows_kernel(const uint4* __restrict__ wt, const ST* __restrict__ sc,
+                                                               const int* __restrict__ wexp, const float* __restrict__ x,
+                                                               Epi epi, int M, int N, int K, int Kp, int ldx) {
+    constexpr int NONE = -1000;  // exponent of rows without a value so far
+    extern __shared__ __align__(16) char wave_lds[];
+    __shared__ int wexps[KW][16];  // the waves' row exponents
+    const int GQ = Kp >> 7, NT = (N + 15) >> 4, tile0 = blockIdx.x * RT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r = lane & 15;    // MFMA operand: chunk of the group, row
+    const int lr = lane >> 2, lp = lane & 3;   // loads: row, chunk of the group
+    uint4* xt = (uint4*)wave_lds + wave * 256;  // [16 chunks][16 rows]; later the partial tiles
+    const int steps = wave < GQ ? (GQ - wave + KW - 1) / KW : 0;
+    float4_t acc[RT];
+    int wneg[RT];
+#pragma unroll
+    for (int a = 0; a < RT; a++) {
+        acc[a] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        wneg[a] = -wexp[min(tile0 + a, NT - 1) * 16 + r];
+    }
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((M - 1) * ldx + K) * 4u);
+    const uint32_t xrow = lr < M ? (uint32_t)(lr * ldx) * 4u : 0xC0000000u;  // past the rows: out of range, zeros
+    u32x4_t xv[4][2];  // chunk j: its eight values
+    auto load_x = [&](int gq) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int k = gq * 128 + j * 32 + lp * 8 + h * 4;
+                const uint32_t off = xrow + (uint32_t)k * 4u;
+                xv[j][h] = __builtin_amdgcn_raw_buffer_load_b128(xrs, k < K ? off : 0xC0000000u, 0, 0);
+            }
+    };
+    u32x4_t wcur[RT], wnxt[RT];
+    ScaleVec<RT, ST> scur, snxt;
+    auto load_w = [&](int gq, u32x4_t (&w)[RT], ScaleVec<RT, ST>& s) {
+#pragma unroll
+        for (int a = 0; a < RT; a++) {
+            const int tt = min(tile0 + a, NT - 1);
+            w[a] = *(const u32x4_t*)(wt + ((size_t)tt * GQ + gq) * 64 + lane);
+            s.load(sc + q4_scale_index(std::is_same<ST, _Float16>::value, tt, gq, r, 0, GQ), a);
+        }
+    };
+    auto gq_of = [&](int i) { return wave + KW * min(i, steps - 1); };  // past the end: the last one again
+    if (steps > 0) {
+        load_x(gq_of(0));
+        load_w(gq_of(0), wcur, scur);
+    }
+    int xe = NONE;  // row lr's exponent (the same in its four lanes)
+    for (int i = 0; i < steps; i++) {
+        float mx = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) mx = fmaxf(mx, fabsf(__uint_as_float(xv[j][h][e])));
+        mx = fmaxf(mx, dpp_move<0xB1>(mx));  // the row's four lanes
+        mx = fmaxf(mx, dpp_move<0x4E>(mx));
+        const int en = mx > 0.0f ? max(xe, range_exp(mx, XPREP_TOP)) : xe;
+        const int down = __shfl(xe - en, 4 * r, 64);  // row r's, where its sums are
+        xe = en;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = __builtin_amdgcn_ldexpf(__uint_as_float(xv[j][e >> 2][e & 3]), -xe);
+            xt[(j * 4 + lp) * 16 + (lr ^ (4 * lp))] = make_uint4(pack_half2(v[0], v[4]), pack_half2(v[1], v[5]),
+                                                                 pack_half2(v[2], v[6]), pack_half2(v[3], v[7]));
+        }
+        const int gn = gq_of(i + 1);
+        load_x(gn);
+        load_w(gn, wnxt, snxt);
+#pragma unroll
+        for (int a = 0; a < RT; a++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[a][e] = __builtin_amdgcn_ldexpf(acc[a][e], down);
+        wave_lds_fence();
+        half8_t bf[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) bf[j] = __builtin_bit_cast(half8_t, xt[(j * 4 + q) * 16 + (r ^ (4 * q))]);
+        wave_lds_fence();  // before the next step's writes
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int a = 0; a < RT; a++) {
+                const _Float16 s = scur.get_ldexp(a, j, wneg[a]);
+                const half2_t s2 = {s, s};
+                half2_t p[4];
+                nib_pairs_f16(wcur[a][j], s2, p);
+                const half8_t af = {p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y};
+                acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[a], 0, 0, 0);
+            }
+#pragma unroll
+        for (int a = 0; a < RT; a++) wcur[a] = wnxt[a];
+        scur = snxt;
+#pragma unroll
+        for (int a = 0; a < RT; a++) asm volatile("" : "+v"(acc[a]));  // MFMA results are read past the loop's branch
+    }
+    if (lp == 0) wexps[wave][lr] = xe;
+    __syncthreads();  // the activations' LDS becomes the partial tiles'
+    float4_t* part = (float4_t*)wave_lds;  // [KW][RT][64]
+#pragma unroll
+    for (int a = 0; a < RT; a++) part[(wave * RT + a) * 64 + lane] = acc[a];
+    __syncthreads();
+    for (int t = wave; t < RT; t += KW) {
+        const int tile = tile0 + t;
+        int top = NONE;
+#pragma unroll
+        for (int w = 0; w < KW; w++) top = max(top, wexps[w][r]);
+        float4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < KW; w++) {
+            const float4_t p = part[(w * RT + t) * 64 + lane];
+            const int d = wexps[w][r] - top;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] += __builtin_amdgcn_ldexpf(p[e], d);
+        }
+        const int4 we = *(const int4*)(wexp + min(tile, NT - 1) * 16 + 4 * q);
+        const int wev[4] = {we.x, we.y, we.z, we.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_ldexpf(v[e], top + wev[e]);
+        epi(r, tile * 16 + 4 * q, N, r < M && tile < NT, v);
+    }
+}
+
 }  // namespace th

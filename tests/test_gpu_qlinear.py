@@ -226,6 +226,40 @@ def test_q4_gemm_shapes(dev, rows, cols, m, scales):
     assert np.all(np.abs(y - ref) <= (2.0 ** -10 + cols * 2.0 ** -24) * mag)
 
 
+@pytest.mark.parametrize("rows,cols,m", [
+    (40, 100, 9),       # one group-quad, fewer rows than a block
+    (1000, 1100, 16),   # nine group-quads over eight waves
+    (4500, 3072, 13),   # two tiles a workgroup, the widest taken
+    (8300, 260, 16),    # four waves, one of three group-quads short
+])
+@pytest.mark.parametrize("scales", ["f16", "f32"])
+def test_q4_rows_direct(dev, rows, cols, m, scales):
+    """The int4 GEMM that converts its few f32 rows on the way: magnitudes that
+    rise and fall by 2^30 along a row, an all-zero row and a row with an
+    infinity.  Weight and activation are rounded to f16 once each (2^-11 of a
+    product; an activation 2^26 below its row's largest keeps less, at most
+    2^-38 of that); the sums are f32."""
+    rng = np.random.default_rng(rows + m)
+    bpr = (cols + 31) // 32
+    nib = np.frombuffer(rng.bytes(rows * bpr * 16), np.uint8).reshape(rows, bpr * 16)
+    sc = rng.uniform(0.002, 0.01, (rows, bpr)).astype(np.float16 if scales == "f16" else np.float32)
+    w = dev.q4_upload_packed(nib, sc.view(np.uint16) if scales == "f16" else sc, rows, cols,
+                             capi.F16 if scales == "f16" else capi.F32)
+    x = rng.standard_normal((m, cols)).astype(np.float32)
+    x *= np.exp2(rng.integers(-15, 16, (m, bpr))).astype(np.float32).repeat(32, 1)[:, :cols]
+    x *= 10.0 ** rng.uniform(-30, 20, (m, 1)).astype(np.float32)
+    x[1] = 0.0
+    x[2, cols // 2] = np.inf
+    y = dev.gemm_q4(dev.upload(x), m, w).to_numpy().reshape(m, rows)
+    assert not y[1].any() and not np.isfinite(y[2]).any()
+    x[2], y[2] = 0.0, 0.0
+    v = np.stack((nib & 15, nib >> 4), -1).reshape(rows, bpr, 32).astype(np.float64) - 8.0
+    wf = (v * sc.astype(np.float64)[:, :, None]).reshape(rows, -1)[:, :cols]
+    ref, mag = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    low = 2.0 ** -38 * np.abs(x).max(1, keepdims=True) * np.abs(wf).sum(1)
+    assert np.all(np.abs(y - ref) <= (2.0 ** -10 + cols * 2.0 ** -24) * mag + low)
+
+
 @pytest.mark.parametrize("rows,cols", [(16, 64), (37, 3), (130, 200), (2050, 1096), (512, 4096), (1100, 4096)])
 @pytest.mark.parametrize("m", [5, 16, 17, 33, 64, 65, 129])  # either side of the 16/32/64/128-row blocks
 @pytest.mark.parametrize("scales", ["row", "group"])
