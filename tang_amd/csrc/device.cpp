@@ -26,11 +26,12 @@ static __device__ __align__(256) unsigned char scratch[TH_NOALLOC_SCRATCH_BYTES 
 static thread_local std::string g_last_error;
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 
+// The workspace that a device starts with.
+constexpr size_t FIRST_WORKSPACE = (size_t)32 << 20;
+
 // Grow one of the device's workspaces to `bytes`.  Once a graph has been
 // captured on the device the outgrown block is kept (its graphs may name it)
 // and sizes double, so that the kept blocks stay below the one in use.
-constexpr size_t FIRST_WORKSPACE = (size_t)32 << 20;
-
 static void* grow_workspace(th_device* dev, void*& ptr, size_t& have, size_t bytes) {
     if (bytes <= have) return ptr;
     size_t want = std::max(bytes, (size_t)1 << 20);

@@ -29,3 +29,26 @@ def test_failed_capture_leaves_stream_usable(dev):
             assert np.array_equal(y.to_numpy(), eager)
     finally:
         g.free()
+
+
+@pytest.mark.parametrize("m", [6, 20])
+def test_captured_gemm_splits_before_any_call(m):
+    """A q8 GEMM captured as a device's first call splits K in the workspace the
+    device starts with: every replay matches the eager call bit for bit."""
+    dev = capi.HipComputeDevice(0)
+    rows, cols = 1000, 1096
+    rng = np.random.default_rng(m)
+    w = dev.q8_upload_rowwise(rng.integers(-128, 128, (rows, cols), np.int8),
+                              rng.uniform(0.005, 0.02, rows).astype(np.float32), rows, cols)
+    x = dev.upload(rng.standard_normal(m * cols).astype(np.float32))
+    y = dev.alloc(m * rows)
+    g = dev.capture(lambda: dev.gemv_q8(x, m, w, y))
+    try:
+        eager = dev.gemv_q8(x, m, w).to_numpy()
+        for _ in range(3):
+            y.upload(np.zeros(m * rows, np.float32))
+            g.launch()
+            dev.sync()
+            assert np.array_equal(y.to_numpy(), eager)
+    finally:
+        g.free()
