@@ -356,6 +356,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float* __restri
                                          attn_pack_h2(y[2], z[2]), attn_pack_h2(y[3], z[3]));
             }
         }
+        // The row's end is zero up to Kp, as every writer of the layout leaves
+        // it: the weights there are zero, but zero times what an earlier owner
+        // of the memory left (an infinity, a NaN) is not.
+        if (h == n_heads - 1 && qi < n)
+            for (int c = n_heads * (D / 8) + g; c < ldo >> 3; c += 4)
+                ((uint4*)out)[xp_index(qi, c, ldo >> 3)] = make_uint4(0, 0, 0, 0);
     } else if (qi < n) {
         uint16_t* op = out + (size_t)qi * ldo + h * D + 4 * g;
 #pragma unroll

@@ -298,6 +298,34 @@ def test_small_llama_prefill_matches_oracle(dev, n, hd):
     assert list(cont) == r_cont
 
 
+@pytest.mark.parametrize("heads,kv", [(9, 3), (5, 1)])  # 576 and 320 columns: rows end 64 short of a multiple of 128
+def test_prefill_ignores_what_its_memory_held(dev, heads, kv):
+    """The O projection multiplies the attention's rows up to a multiple of 128
+    columns.  Memory that held NaNs of every width, freed just before the
+    prompt's workspaces are allocated (a short prompt's, then a longer one's),
+    leaves no trace in the logits."""
+    cfg = dict(CONFIG_SMALL, n_heads=heads, n_kv_heads=kv, d_model=64 * heads)
+    prefill = 20
+    ref = OracleLlama(cfg, 7, 8, prefill)
+    m = device_llama(dev, cfg, 7, 8, prefill)
+    print(f"prefill over used memory, {heads} heads", flush=True)
+    try:
+        pos = prefill
+        for n in (18, 90):
+            for size in (1 << 14, 1 << 16, 1 << 18, 1 << 20, 1 << 22):
+                held = [dev.upload(np.full(size // 2, 0x7FFF, np.uint16), capi.F16) for _ in range(12)]
+                for b in held:
+                    b.free()
+            toks = [int(t) for t in np.random.default_rng(n).integers(0, cfg["vocab"], n)]
+            for i, t in enumerate(toks):
+                _, r_logits = ref.step(t, pos + i)
+            _, logits = _prefill(m, cfg, toks, pos)
+            assert np.all(np.isfinite(logits)) and max_abs_rel(logits, r_logits) < 2e-2
+            pos += n
+    finally:
+        capi.lib().th_llama_destroy(m)
+
+
 @pytest.mark.parametrize("tied", [False, True])
 def test_llama_from_safetensors_matches_oracle(dev, tmp_path, tied):
     """th_llama_load_safetensors (load_model, smollm.rs:364-420) on a small
