@@ -37,21 +37,23 @@ __device__ __forceinline__ float ld_el(const void* p, size_t i) {
 // both f32 or bf16.
 //
 // On v_mfma_f32_16x16x32_bf16, which has sixteen times the f32 MFMA's rate: an
-// f32 operand goes in as three bf16 parts (x = p0 + p1 + p2 exactly, eight
-// bits each), so f32 x bf16 takes three exact products and f32 x f32 the six
-// whose parts weigh 2^-16 or more of it (the rest is under 2^-22 of a product,
-// below the roundings of its sum); sums are f32.  A result that comes out NaN
-// (an infinity times a part that is zero, or a sum of parts that overflows
-// both ways) is summed again in plain f32 by its thread.
+// f32 operand goes in as three bf16 parts (x = p0 + p1 + p2 exactly, eight bits
+// each), so f32 x bf16 takes three exact products and f32 x f32 the eight whose
+// parts weigh 2^-24 or more of it (the ninth is under 2^-30 of a product).  A
+// tile with a result that is not finite (an infinity times a part that is zero)
+// is summed again on the f32 MFMA by its workgroup.  So is a K of one step, where
+// the truncation inside an MFMA costs more than f32's roundings (from two steps
+// on it costs less).
 //
 // Workgroup: 4 waves, WGM along m; each wave TM x TN 16x16 tiles; K in steps
 // of 32, both operands double-buffered in LDS as 8-value octets.  A step sums
 // up by itself before it joins the accumulators (short chains of additions).
 // Bound by the MFMAs and their LDS operands on large shapes, by the chain of
 // steps on small ones (K split over workgroups there).  Against 64x64 tiles
-// on the f32 MFMA: m 509, k 2048, n 5632, f32 x bf16 210 -> 65 us (541 TFLOP/s
-// of parts); m 1, k 4096 275 -> 21 us; m 1024, k = n = 4096, f32 x f32 374 -> 230
-// us, bf16 565 -> 104 us; error against 64 bits 8.1e-7 -> 1.6e-7.
+// on the f32 MFMA: m 509, k 2048, n 5632, f32 x bf16 210 -> 69 us (510 TFLOP/s
+// of parts; 261 if every tile holds a NaN); m 1, k 4096
+// 275 -> 17 us; m 1024, k = n = 4096, f32 x f32 374 -> 265 us, bf16 565 -> 104 us;
+// error against 64 bits 8.1e-7 -> 1.0e-7.
 // ---------------------------------------------------------------------------
 
 // An operand: `rows` rows of K values, element (row, k) at row * rs + k * ks.
@@ -104,9 +106,11 @@ __device__ __forceinline__ void mm_mask(int n, u32x4_t& a, u32x4_t& b) {
     }
 }
 
+// Value e of an octet that mm_load8 loaded.
 template <bool BF>
-__device__ __forceinline__ float mm_el(const MatOperand& m, int row, int k) {
-    return ld_el<BF>(m.p, (size_t)row * m.rs + (size_t)k * m.ks);
+__device__ __forceinline__ float mm_value(int e, const u32x4_t& a, const u32x4_t& b) {
+    if constexpr (BF) return __uint_as_float(e & 1 ? a[e >> 1] & 0xFFFF0000u : a[e >> 1] << 16);
+    else return __uint_as_float(e < 4 ? a[e] : b[e - 4]);
 }
 
 constexpr int MM_LD = 17;  // octet stride in 16-byte units (16 rows + 1: spreads the banks)
@@ -115,6 +119,7 @@ template <bool ABF, bool BBF, bool AV, bool BV, int TM, int TN, int WGM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void matmul_kernel(
     MatOperand A, MatOperand B, float* __restrict__ c, int K, size_t split_stride, int k_per_split, int accumulate) {
     constexpr int PA = ABF ? 1 : 3, PB = BBF ? 1 : 3, WGN = 4 / WGM;
+    constexpr bool PARTS = PA * PB > 1;
     constexpr int MB = WGM * TM, NB = WGN * TN;           // 16-row blocks of the workgroup
     constexpr int APL = MB * 4 * MM_LD, BPL = NB * 4 * MM_LD;  // one part of a step
     constexpr int AO = MB * 64, BO = NB * 64;             // octets of a step
@@ -185,54 +190,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         }
     };
     f32x4_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    load(kb);
-    store(lds[0], kb);
-    __syncthreads();
-    int buf = 0;
-    for (int k = kb; k < ke; k += 32) {
-        const uint4 *ta = lds[buf], *tb = ta + PA * APL;
-        const bool more = k + 32 < ke;
-        if (more) load(k + 32);
-        bf16x8_t bv[TN][PB];
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int p = 0; p < PB; p++)
-                bv[j][p] = __builtin_bit_cast(bf16x8_t, tb[p * BPL + ((wn + j) * 4 + q) * MM_LD + r]);
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            bf16x8_t av[PA];
-#pragma unroll
-            for (int p = 0; p < PA; p++)
-                av[p] = __builtin_bit_cast(bf16x8_t, ta[p * APL + ((wm + i) * 4 + q) * MM_LD + r]);
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                // D = (rows of B) x (rows of A): a lane holds four consecutive n of one m
-                f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int w = 2; w >= 0; w--)  // the smallest products first
-#pragma unroll
-                    for (int p = 0; p <= w; p++)
-                        if (p < PA && w - p < PB)
-                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j][w - p], av[p], d, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][j][e] += d[e];
-            }
-        }
-        // The additions stay in this block: moved past the branch below they
-        // follow their MFMA with too few wait states (the compiler counts none
-        // across a taken branch), and read it too early.
+    auto sum = [&]() {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) asm volatile("" : "+v"(acc[i][j]));
-        buf ^= 1;
-        if (more) store(lds[buf], k + 32);
+            for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        load(kb);
+        store(lds[0], kb);
         __syncthreads();
+        int buf = 0;
+        for (int k = kb; k < ke; k += 32) {
+            const uint4 *ta = lds[buf], *tb = ta + PA * APL;
+            const bool more = k + 32 < ke;
+            if (more) load(k + 32);
+            bf16x8_t bv[TN][PB];
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int p = 0; p < PB; p++)
+                    bv[j][p] = __builtin_bit_cast(bf16x8_t, tb[p * BPL + ((wn + j) * 4 + q) * MM_LD + r]);
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                bf16x8_t av[PA];
+#pragma unroll
+                for (int p = 0; p < PA; p++)
+                    av[p] = __builtin_bit_cast(bf16x8_t, ta[p * APL + ((wm + i) * 4 + q) * MM_LD + r]);
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    // D = (rows of B) x (rows of A): a lane holds four consecutive n of one m
+                    f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int w = 3; w >= 0; w--)  // the smallest products first
+#pragma unroll
+                        for (int p = 0; p <= w; p++)
+                            if (p < PA && w - p < PB)
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j][w - p], av[p], d, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] += d[e];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) mfma_pin(acc[i][j]);
+            buf ^= 1;
+            if (more) store(lds[buf], k + 32);
+            __syncthreads();
+        }
+    };
+    // the same on the f32 MFMA, straight from memory: lane (q, r) takes octet q of row r
+    auto sum_f32 = [&]() {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int k = kb; k < ke; k += 32) {
+            const bool whole = k + 32 <= K;
+            const int k0 = k + 8 * q;
+            u32x4_t a[TM][2], b[TN][2];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+                mm_load8<ABF>(A, ars, m0, min(m0 + (wm + i) * 16 + r, A.rows - 1), K, k0, AV && whole, a[i][0], a[i][1]);
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                mm_load8<BBF>(B, brs, n0, min(n0 + (wn + j) * 16 + r, B.rows - 1), K, k0, BV && whole, b[j][0], b[j][1]);
+#pragma unroll
+            for (int i = 0; i < TM; i++) mm_mask<ABF>(ke - k0, a[i][0], a[i][1]);
+#pragma unroll
+            for (int j = 0; j < TN; j++) mm_mask<BBF>(ke - k0, b[j][0], b[j][1]);
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(mm_value<BBF>(e, b[j][0], b[j][1]),
+                                                                 mm_value<ABF>(e, a[i][0], a[i][1]), d, 0, 0, 0);
+                    acc[i][j] += d;
+                    mfma_pin(acc[i][j]);
+                }
+        }
+    };
+    sum();
+    if constexpr (PARTS) {
+        auto any = [&](auto test) {
+            bool t = false;
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t |= test(fabsf(acc[i][j][e]));
+            return t;
+        };
+        const auto nonfinite = [](float v) { return !(v <= 3.402823466e38f); };
+        if (__syncthreads_or(ke <= kb + 32 || any(nonfinite))) sum_f32();
     }
     float* cb = c + (size_t)split * split_stride;
     const int N = B.rows;
@@ -244,13 +297,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         for (int j = 0; j < TN; j++) {
             const int n = n0 + (wn + j) * 16 + 4 * q;
             float* p = cb + (size_t)m * N + n;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (n + e >= N || acc[i][j][e] == acc[i][j][e]) continue;
-                float s = 0.0f;  // NaN: in plain f32
-                for (int k = kb; k < ke; k++) s = __builtin_fmaf(mm_el<ABF>(A, m, k), mm_el<BBF>(B, n + e, k), s);
-                acc[i][j][e] = s;
-            }
             if (N % 4 == 0 && n < N) {
                 f32x4_t v = acc[i][j];
                 if (accumulate) v = *(const f32x4_t*)p + v;

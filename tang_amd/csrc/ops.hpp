@@ -91,6 +91,21 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
+// MFMA results and branches.  The compiler keeps a read of a result the
+// required wait states behind its MFMA in straight code; moved past a taken
+// branch, a read was seen one or two states behind.  So every kernel keeps to
+// one of two forms: mfma_pin after reads that belong before a branch (the
+// additions of a step's sums), which holds them there, or mfma_settle on sums
+// that are first read behind their loop, which waits out the longest MFMA.
+template <typename V>
+__device__ __forceinline__ void mfma_pin(V& v) {
+    asm volatile("" : "+v"(v));
+}
+template <typename V>
+__device__ __forceinline__ void mfma_settle(V& v) {
+    asm volatile("s_nop 15\n\ts_nop 3" : "+v"(v));
+}
+
 // One DPP move inside rows of 16 lanes (CTRL: the dpp_ctrl encoding).
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {

@@ -48,7 +48,7 @@ def test_matmul_variants(dev, m, k, n, ta, tb):
 def test_matmul_tiles_and_types(dev, m, k, n, ta, tb, ad, bd):
     """Edges of the 16- and 64-row tiles, the 32-deep steps and the K splits,
     for every operand type and order, added to C.  Products of bf16 parts are
-    exact (f32 x f32 leaves out under 2^-22 of one), sums are f32: an output
+    exact (f32 x f32 leaves out under 2^-30 of one), sums are f32: an output
     is off by at most (k + 4) roundings of its terms' magnitudes."""
     rng = np.random.default_rng(m * 7 + k + n)
     a = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-8, 8, (m, 1))).astype(np.float32)
@@ -68,6 +68,27 @@ def test_matmul_tiles_and_types(dev, m, k, n, ta, tb, ad, bd):
     a, b = a.astype(np.float64), b.astype(np.float64)
     ref, mag = c0 + a @ b, np.abs(c0) + np.abs(a) @ np.abs(b)
     assert np.all(np.abs(c.to_numpy().reshape(m, n) - ref) <= (k + 4) * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("ad,bd", [("f32", "f32"), ("f32", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("m,k", [(5, 1), (40, 1), (40, 2), (40, 32), (40, 45)])
+def test_matmul_full_mantissas(dev, m, k, ad, bd):
+    """Significands that truncate worst in parts, all of one sign: one product is
+    rounded once, as in f32.  A sum's bound is two roundings for its steps and
+    one of an eighth of the terms for each of them."""
+    worst = {"f32": 0x3F80FFFF, "bf16": 0x3FFF0000}
+    rng = np.random.default_rng(k)
+    a = np.full((m, k), worst[ad], np.uint32).view(np.float32)
+    b = np.full((k, 30), worst[bd], np.uint32).view(np.float32)
+    if ad == "f32":
+        a[1:] = rng.uniform(1, 2, (m - 1, k)).astype(np.float32)
+    if bd == "f32":
+        b[:, 1:] = rng.uniform(1, 2, (k, 29)).astype(np.float32)
+    up = lambda x, dt: dev.upload(oracle.f32_to_bf16(x.reshape(-1)), capi.BF16) if dt == "bf16" else dev.upload(x)
+    c = dev.matmul(up(a, ad), up(b, bd), m, k, 30).to_numpy().reshape(m, 30).astype(np.float64)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    err = (c - ref) / ref * 2.0 ** 24
+    assert np.max(np.abs(err)) <= (1 if k == 1 else k / 8 + 2)
 
 
 @pytest.mark.parametrize("m", [5, 70])
