@@ -207,7 +207,7 @@ int th_bench_linear(th_device* dev, const th_buffer* x, size_t m, th_qweight* co
  * (trans_a: stored [k][m]), B is [k][n] (trans_b: stored [n][k], the
  * Linear::forward_2d weight layout, modules.rs:56); A and B f32 or bf16, C
  * f32; accumulate != 0 adds to C.  Products to 2^-30 or better, f32 accumulation
- * on MFMA; infinities and NaN as in plain f32. */
+ * on MFMA; infinities, NaN and f32's whole range as in plain f32. */
 int th_matmul_ex(th_device* dev, const th_buffer* a, const th_buffer* b, size_t m, size_t k, size_t n, int trans_a,
                  int trans_b, int accumulate, th_buffer* c);
 /* ComputeDevice::matmul (device.rs:103; CpuDevice cpu.rs:99,760). */

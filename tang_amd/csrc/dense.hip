@@ -39,11 +39,14 @@ __device__ __forceinline__ float ld_el(const void* p, size_t i) {
 // On v_mfma_f32_16x16x32_bf16, which has sixteen times the f32 MFMA's rate: an
 // f32 operand goes in as three bf16 parts (x = p0 + p1 + p2 exactly, eight bits
 // each), so f32 x bf16 takes three exact products and f32 x f32 the eight whose
-// parts weigh 2^-24 or more of it (the ninth is under 2^-30 of a product).  A
-// tile with a result that is not finite (an infinity times a part that is zero)
-// is summed again on the f32 MFMA by its workgroup.  So is a K of one step, where
-// the truncation inside an MFMA costs more than f32's roundings (from two steps
-// on it costs less).
+// parts weigh 2^-24 or more of it (the ninth is under 2^-30 of a product).  Two
+// exceptions, found by each workgroup for its tile:
+// - Operands or results so small that parts of them vanish: the tile is summed
+//   once more with its f32 operands times 2^SPLIT_EXP.
+// - A result that is not finite (an infinity times a part that is zero, a value
+//   or a sum too large for that factor): summed on the f32 MFMA.  So is a K of
+//   one step, where the truncation inside an MFMA costs more than f32's
+//   roundings (from two steps on it costs less).
 //
 // Workgroup: 4 waves, WGM along m; each wave TM x TN 16x16 tiles; K in steps
 // of 32, both operands double-buffered in LDS as 8-value octets.  A step sums
@@ -51,7 +54,7 @@ __device__ __forceinline__ float ld_el(const void* p, size_t i) {
 // Bound by the MFMAs and their LDS operands on large shapes, by the chain of
 // steps on small ones (K split over workgroups there).  Against 64x64 tiles
 // on the f32 MFMA: m 509, k 2048, n 5632, f32 x bf16 210 -> 69 us (510 TFLOP/s
-// of parts; 261 if every tile holds a NaN); m 1, k 4096
+// of parts; 149 if every tile holds vanishing parts, 261 if NaN); m 1, k 4096
 // 275 -> 17 us; m 1024, k = n = 4096, f32 x f32 374 -> 265 us, bf16 565 -> 104 us;
 // error against 64 bits 8.1e-7 -> 1.0e-7.
 // ---------------------------------------------------------------------------
@@ -161,7 +164,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             mm_load8<BBF>(B, brs, n0, min(n0 + row, B.rows - 1), K, k + o * 8, BV && whole, rb[i][0], rb[i][1]);
         }
     };
-    auto put = [&](auto bf, uint4* dst, int plane, int row, int o, u32x4_t (&v)[2], int k) {
+    uint32_t lost = 0;
+    auto put = [&](auto ex, auto bf, uint4* dst, int plane, int row, int o, u32x4_t (&v)[2], int k) {
         constexpr bool BF = decltype(bf)::value;
         mm_mask<BF>(K - (k + o * 8), v[0], v[1]);
         dst += ((row >> 4) * 4 + o) * MM_LD + (row & 15);
@@ -169,34 +173,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             *dst = __builtin_bit_cast(uint4, v[0]);
         } else {
             uint4 p[3];
-            split3_bf16(__builtin_bit_cast(uint4, v[0]), __builtin_bit_cast(uint4, v[1]), p);
+            split3_bf16<decltype(ex)::value>(__builtin_bit_cast(uint4, v[0]), __builtin_bit_cast(uint4, v[1]), p, lost);
 #pragma unroll
             for (int e = 0; e < 3; e++) dst[e * plane] = p[e];
         }
     };
-    auto store = [&](uint4* t, int k) {
+    auto store = [&](auto ex, uint4* t, int k) {
 #pragma unroll
         for (int i = 0; i < AT; i++) {
             int row, o;
             place(tid + 256 * i, MB * 16, AV, row, o);
-            if (AO % 256 == 0 || tid + 256 * i < AO) put(std::integral_constant<bool, ABF>{}, t, APL, row, o, ra[i], k);
+            if (AO % 256 == 0 || tid + 256 * i < AO) put(ex, std::integral_constant<bool, ABF>{}, t, APL, row, o, ra[i], k);
         }
 #pragma unroll
         for (int i = 0; i < BT; i++) {
             int row, o;
             place(tid + 256 * i, NB * 16, BV, row, o);
             if (BO % 256 == 0 || tid + 256 * i < BO)
-                put(std::integral_constant<bool, BBF>{}, t + PA * APL, BPL, row, o, rb[i], k);
+                put(ex, std::integral_constant<bool, BBF>{}, t + PA * APL, BPL, row, o, rb[i], k);
         }
     };
     f32x4_t acc[TM][TN];
-    auto sum = [&]() {
+    auto sum = [&](auto ex) {  // f32 operands times 2^ex
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         load(kb);
-        store(lds[0], kb);
+        store(ex, lds[0], kb);
         __syncthreads();
         int buf = 0;
         for (int k = kb; k < ke; k += 32) {
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 #pragma unroll
                 for (int j = 0; j < TN; j++) mfma_pin(acc[i][j]);
             buf ^= 1;
-            if (more) store(lds[buf], k + 32);
+            if (more) store(ex, lds[buf], k + 32);
             __syncthreads();
         }
     };
@@ -272,7 +276,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
                 }
         }
     };
-    sum();
+    sum(std::integral_constant<int, 0>{});
     if constexpr (PARTS) {
         auto any = [&](auto test) {
             bool t = false;
@@ -285,7 +289,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             return t;
         };
         const auto nonfinite = [](float v) { return !(v <= 3.402823466e38f); };
-        if (__syncthreads_or(ke <= kb + 32 || any(nonfinite))) sum_f32();
+        // parts of an operand or of a product below the formats' smallest numbers
+        const bool vanished = (lost & 0xFFFFu) != 0 || any([](float v) { return v > 0.0f && v < 0x1p-100f; });
+        const bool one_step = ke <= kb + 32;
+        if (__syncthreads_or(vanished || one_step || any(nonfinite))) {
+            if (__syncthreads_or(vanished)) {
+                sum(std::integral_constant<int, SPLIT_EXP>{});
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            acc[i][j][e] = __builtin_amdgcn_ldexpf(acc[i][j][e], -SPLIT_EXP * (!ABF + !BBF));
+            }
+            if (__syncthreads_or(one_step || any(nonfinite))) sum_f32();
+        }
     }
     float* cb = c + (size_t)split * split_stride;
     const int N = B.rows;

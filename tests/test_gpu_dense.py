@@ -70,6 +70,44 @@ def test_matmul_tiles_and_types(dev, m, k, n, ta, tb, ad, bd):
     assert np.all(np.abs(c.to_numpy().reshape(m, n) - ref) <= (k + 4) * 2.0 ** -24 * mag)
 
 
+def _spread(rng, shape, exps):
+    """Random signs and mantissas, a power of two per row (exps) down to f32's
+    subnormals."""
+    x = rng.uniform(1, 2, shape) * rng.choice([-1.0, 1.0], shape) * np.exp2(np.asarray(exps, np.float64))[:, None]
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("m,k,n", [(9, 70, 50), (80, 515, 140)])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+@pytest.mark.parametrize("ad,bd", [("f32", "bf16"), ("bf16", "f32"), ("f32", "f32")])
+@pytest.mark.parametrize("big", [False, True])
+def test_matmul_exponent_range(dev, m, k, n, ta, tb, ad, bd, big):
+    """Rows of f32's smallest numbers, subnormals among them, against large
+    partners keep f32's bits, and (big) so do sums near its largest: as many
+    roundings as anywhere else."""
+    rng = np.random.default_rng(m + k + big)
+    ea = rng.integers(90, 117, m) if big else rng.integers(-149, -95, m)
+    a = _spread(rng, (m, k), ea if ad == "f32" else rng.integers(90, 110, m))
+    b = _spread(rng, (n, k), (rng.integers(-4, 1, n) if big else rng.integers(95, 105, n)) if ad == "f32" else
+                (rng.integers(-9, 4, n) if big else rng.integers(-149, -95, n)))
+
+    def up(x, t, dt):
+        x = (x.T if t else x).reshape(-1).copy()
+        return dev.upload(oracle.f32_to_bf16(x), capi.BF16) if dt == "bf16" else dev.upload(x)
+
+    if ad == "bf16":
+        a = _bf16_round(a.reshape(-1)).reshape(m, k)
+    if bd == "bf16":
+        b = _bf16_round(b.reshape(-1)).reshape(n, k)
+    c = dev.alloc(m * n)
+    dev.zero_buffer(c)
+    dev.matmul(up(a, ta, ad), up(b, not tb, bd), m, k, n, trans_a=ta, trans_b=tb, accumulate_into=c)
+    a, b = a.astype(np.float64), b.astype(np.float64).T
+    mag = np.abs(a) @ np.abs(b)
+    assert np.all(mag > 2.0 ** -70) and np.all(mag < 2.0 ** 128)
+    assert np.all(np.abs(c.to_numpy().reshape(m, n) - a @ b) <= (k + 4) * 2.0 ** -24 * mag)
+
+
 @pytest.mark.parametrize("ad,bd", [("f32", "f32"), ("f32", "bf16"), ("bf16", "f32")])
 @pytest.mark.parametrize("m,k", [(5, 1), (40, 1), (40, 2), (40, 32), (40, 45)])
 def test_matmul_full_mantissas(dev, m, k, ad, bd):
