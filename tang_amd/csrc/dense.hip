@@ -130,7 +130,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     __shared__ uint4 lds[2][PA * APL + PB * BPL];
     int bx = blockIdx.x, by = blockIdx.y, split = blockIdx.z;
     gemm_xcd_tile(bx, by, split);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, r = lane & 15;
     const int m0 = by * MB * 16, n0 = bx * NB * 16;
     const int wm = (wave / WGN) * TM, wn = (wave % WGN) * TN;
@@ -294,6 +295,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         const bool one_step = ke <= kb + 32;
         if (__syncthreads_or(vanished || one_step || any(nonfinite))) {
             if (__syncthreads_or(vanished)) {
+                asm volatile("" : "+v"(tid));  // places are formed again, not kept through the first pass
                 sum(std::integral_constant<int, SPLIT_EXP>{});
 #pragma unroll
                 for (int i = 0; i < TM; i++)
