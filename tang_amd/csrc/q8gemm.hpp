@@ -61,7 +61,10 @@ __device__ __forceinline__ void split3_bf16(const uint4& a, const uint4& b, uint
 // starts from zero and its D is weighted with one FMA by the lane's scale
 // (the lane's D column is one weight row); with a scale per row the MFMAs
 // accumulate and the scale comes at the end.  A step sums up by itself before
-// it joins the accumulators: short chains of f32 additions, as the GEMV's.
+// it joins the accumulators: short chains of f32 additions, as the GEMV's.  A
+// workgroup that met f32 values with vanishing parts (split3_bf16) makes a
+// second, scaled pass; finding them costs 3 to 6% (m = 100: 48 -> 51 us per-row
+// scales, 52 -> 56 per-group).
 //
 // Bound by the weight stream up to about 32 rows, then by the conversions and
 // scale FMAs next to the MFMAs: 11008 x 4096, per-group scales, bf16 rows:
@@ -83,168 +86,180 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     __shared__ uint4 xt[2][PARTS * PLANE];
     int bx = blockIdx.x, by = blockIdx.y, split = blockIdx.z;
     gemm_xcd_tile(bx, by, split);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q = lane >> 4, r = lane & 15;
-    const int NCH = Kp >> 6, NT = (N + 15) >> 4, GPR = Kp >> 5;
-    const int c0 = split * ch_per_split, c1 = min(NCH, c0 + ch_per_split);
-    const int m0 = by * CB * 16, mrows = min(CB * 16, M - m0);
-    const int tile0 = (bx * 4 + wave) * RT;
-    const int octq = ((q & 1) << 1) | (q >> 1);  // octet of a 32-group that this lane multiplies
-
-    float4_t acc[RT][CB];
-#pragma unroll
-    for (int a = 0; a < RT; a++)
-#pragma unroll
-        for (int b = 0; b < CB; b++) acc[a][b] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
-
-    // Activation octets of a step: thread -> (row, octet), eight (or sixteen)
-    // consecutive threads per row.  Rows past the block re-read its last row
-    // (never stored); octets past K are zeroed when stored.
-    u32x4_t xa[PT], xb[XF32 ? PT : 1];  // native vectors: arrays of uint4 structs go to scratch
-    auto load_x = [&](int c) {
-#pragma unroll
-        for (int i = 0; i < PT; i++) {
-            const int idx = min(tid + 256 * i, NOCT - 1), row = min(idx / OCT, mrows - 1), o = idx % OCT;
-            uint4 a, b;
-            load_x8<XF32, VEC>(xin, m0 + row, ldx, K, c * 64 + o * 8, a, b);
-            xa[i] = __builtin_bit_cast(u32x4_t, a);
-            if constexpr (XF32) xb[i] = __builtin_bit_cast(u32x4_t, b);
-        }
-    };
     uint32_t lost = 0;
-    auto store_x = [&](uint4* t, int c) {
+    auto pass = [&](auto ex) {  // f32 rows times 2^ex
+        constexpr int EXP = decltype(ex)::value;
+        int tid = threadIdx.x;
+        if constexpr (XF32) asm volatile("" : "+v"(tid));  // a second pass forms its places again: none kept through the first
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int q = lane >> 4, r = lane & 15;
+        const int NCH = Kp >> 6, NT = (N + 15) >> 4, GPR = Kp >> 5;
+        const int c0 = split * ch_per_split, c1 = min(NCH, c0 + ch_per_split);
+        const int m0 = by * CB * 16, mrows = min(CB * 16, M - m0);
+        const int tile0 = (bx * 4 + wave) * RT;
+        const int octq = ((q & 1) << 1) | (q >> 1);  // octet of a 32-group that this lane multiplies
+
+        // Activation octets of a step: thread -> (row, octet), eight (or sixteen)
+        // consecutive threads per row.  Rows past the block re-read its last row
+        // (never stored); octets past K are zeroed when stored.
+        u32x4_t xa[PT], xb[XF32 ? PT : 1];  // native vectors: arrays of uint4 structs go to scratch
+        auto load_x = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < PT; i++) {
-            const int idx = tid + 256 * i, row = idx / OCT, o = idx % OCT;
-            if (NOCT % 256 != 0 && idx >= NOCT) break;
-            const uint4 z = make_uint4(0, 0, 0, 0);
-            const bool in = c * 64 + o * 8 < K;
-            uint4* dst = t + ((row >> 4) * OCT + o) * LD + (row & 15);
-            if constexpr (XF32) {
-                uint4 p[3];
-                split3_bf16<0>(in ? __builtin_bit_cast(uint4, xa[i]) : z, in ? __builtin_bit_cast(uint4, xb[i]) : z, p, lost);
-#pragma unroll
-                for (int e = 0; e < 3; e++) dst[e * PLANE] = p[e];
-            } else {
-                *dst = in ? __builtin_bit_cast(uint4, xa[i]) : z;
+            for (int i = 0; i < PT; i++) {
+                const int idx = min(tid + 256 * i, NOCT - 1), row = min(idx / OCT, mrows - 1), o = idx % OCT;
+                uint4 a, b;
+                load_x8<XF32, VEC>(xin, m0 + row, ldx, K, c * 64 + o * 8, a, b);
+                xa[i] = __builtin_bit_cast(u32x4_t, a);
+                if constexpr (XF32) xb[i] = __builtin_bit_cast(u32x4_t, b);
             }
-        }
-    };
-    u32x4_t wcur[RT][KG], wnxt[RT][KG];
-    float scur[RT][KG][2], snxt[RT][KG][2];
-    auto load_w = [&](int c, u32x4_t (&w)[RT][KG], float (&s)[RT][KG][2]) {
+        };
+        auto store_x = [&](uint4* t, int c) {
 #pragma unroll
-        for (int a = 0; a < RT; a++) {
-            const int t = min(tile0 + a, NT - 1);
+            for (int i = 0; i < PT; i++) {
+                const int idx = tid + 256 * i, row = idx / OCT, o = idx % OCT;
+                if (NOCT % 256 != 0 && idx >= NOCT) break;
+                const uint4 z = make_uint4(0, 0, 0, 0);
+                const bool in = c * 64 + o * 8 < K;
+                uint4* dst = t + ((row >> 4) * OCT + o) * LD + (row & 15);
+                if constexpr (XF32) {
+                    uint4 p[3];
+                    split3_bf16<EXP>(in ? __builtin_bit_cast(uint4, xa[i]) : z, in ? __builtin_bit_cast(uint4, xb[i]) : z, p, lost);
 #pragma unroll
-            for (int k = 0; k < KG; k++) {
-                const int ck = min(c + k, NCH - 1);
-                w[a][k] = *(const u32x4_t*)(wt + ((size_t)t * NCH + ck) * 64 + lane);
-                if constexpr (!PER_ROW) {
-                    const float2 v = *(const float2*)(sc + (size_t)(t * 16 + r) * GPR + 2 * ck);
-                    s[a][k][0] = v.x;
-                    s[a][k][1] = v.y;
+                    for (int e = 0; e < 3; e++) dst[e * PLANE] = p[e];
+                } else {
+                    *dst = in ? __builtin_bit_cast(uint4, xa[i]) : z;
                 }
             }
-        }
-    };
-    load_x(c0);
-    load_w(c0, wcur, scur);
-    store_x(xt[0], c0);
-    __syncthreads();
-    int buf = 0;
-    for (int c = c0; c < c1; c += KG) {
-        const uint4* t = xt[buf];
-        const bool more = c + KG < c1;
-        if (more) {
-            load_x(c + KG);
-            load_w(c + KG, wnxt, snxt);
-        }
-        bf16x8_t bw[RT][KG][2];
+        };
+        u32x4_t wcur[RT][KG], wnxt[RT][KG];
+        float scur[RT][KG][2], snxt[RT][KG][2];
+        auto load_w = [&](int c, u32x4_t (&w)[RT][KG], float (&s)[RT][KG][2]) {
+#pragma unroll
+            for (int a = 0; a < RT; a++) {
+                const int t = min(tile0 + a, NT - 1);
+#pragma unroll
+                for (int k = 0; k < KG; k++) {
+                    const int ck = min(c + k, NCH - 1);
+                    w[a][k] = *(const u32x4_t*)(wt + ((size_t)t * NCH + ck) * 64 + lane);
+                    if constexpr (!PER_ROW) {
+                        const float2 v = *(const float2*)(sc + (size_t)(t * 16 + r) * GPR + 2 * ck);
+                        s[a][k][0] = v.x;
+                        s[a][k][1] = v.y;
+                    }
+                }
+            }
+        };
+        float4_t acc[RT][CB];
 #pragma unroll
         for (int a = 0; a < RT; a++)
 #pragma unroll
-            for (int k = 0; k < KG; k++) {
-                // the last step's missing chunk (its activations are zeros
-                // past K) multiplies nothing
-                const u32x4_t w = c + k < c1 ? wcur[a][k] : (u32x4_t){0, 0, 0, 0};
-                const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
-                const auto s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-#pragma unroll
-                for (int g = 0; g < 2; g++) {
-                    uint4 f;
-                    i8x4_to_bf16(s0[g], f.x, f.y);
-                    i8x4_to_bf16(s1[g], f.z, f.w);
-                    bw[a][k][g] = __builtin_bit_cast(bf16x8_t, f);
-                }
+            for (int b = 0; b < CB; b++) acc[a][b] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        load_x(c0);
+        load_w(c0, wcur, scur);
+        store_x(xt[0], c0);
+        __syncthreads();
+        int buf = 0;
+        for (int c = c0; c < c1; c += KG) {
+            const uint4* t = xt[buf];
+            const bool more = c + KG < c1;
+            if (more) {
+                load_x(c + KG);
+                load_w(c + KG, wnxt, snxt);
             }
+            bf16x8_t bw[RT][KG][2];
 #pragma unroll
-        for (int b = 0; b < CB; b++) {
-            bf16x8_t af[KG][2][PARTS];
+            for (int a = 0; a < RT; a++)
 #pragma unroll
-            for (int k = 0; k < KG; k++)
+                for (int k = 0; k < KG; k++) {
+                    // the last step's missing chunk (its activations are zeros
+                    // past K) multiplies nothing
+                    const u32x4_t w = c + k < c1 ? wcur[a][k] : (u32x4_t){0, 0, 0, 0};
+                    const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+                    const auto s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
 #pragma unroll
-                for (int g = 0; g < 2; g++)
+                    for (int g = 0; g < 2; g++) {
+                        uint4 f;
+                        i8x4_to_bf16(s0[g], f.x, f.y);
+                        i8x4_to_bf16(s1[g], f.z, f.w);
+                        bw[a][k][g] = __builtin_bit_cast(bf16x8_t, f);
+                    }
+                }
 #pragma unroll
-                    for (int p = 0; p < PARTS; p++)
-                        af[k][g][p] = __builtin_bit_cast(bf16x8_t, t[p * PLANE + (b * OCT + k * 8 + g * 4 + octq) * LD + r]);
-#pragma unroll
-            for (int a = 0; a < RT; a++) {
-                float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};  // this step's sum: joins acc once
+            for (int b = 0; b < CB; b++) {
+                bf16x8_t af[KG][2][PARTS];
 #pragma unroll
                 for (int k = 0; k < KG; k++)
 #pragma unroll
-                    for (int g = 0; g < 2; g++) {
-                        float4_t d = PER_ROW ? v : (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int g = 0; g < 2; g++)
 #pragma unroll
-                        for (int p = PARTS - 1; p >= 0; p--)
-                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[k][g][p], bw[a][k][g], d, 0, 0, 0);
-                        if constexpr (PER_ROW) {
-                            v = d;
-                        } else {
+                        for (int p = 0; p < PARTS; p++)
+                            af[k][g][p] = __builtin_bit_cast(bf16x8_t, t[p * PLANE + (b * OCT + k * 8 + g * 4 + octq) * LD + r]);
 #pragma unroll
-                            for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(scur[a][k][g], d[e], v[e]);
-                        }
-                    }
-                acc[a][b] += v;
-            }
-            if constexpr (!PER_ROW) {
-                // The next block's MFMAs take the weights from here on: left
-                // alone the compiler runs every block's MFMAs first, and their
-                // results (16 registers a tile and step) spill or cost the
-                // SIMD its second and third wave.
-#pragma unroll
-                for (int a = 0; a < RT; a++)
+                for (int a = 0; a < RT; a++) {
+                    float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};  // this step's sum: joins acc once
 #pragma unroll
                     for (int k = 0; k < KG; k++)
-                        asm volatile("" : "+v"(acc[a][b]), "+v"(bw[a][k][0]), "+v"(bw[a][k][1]));
+#pragma unroll
+                        for (int g = 0; g < 2; g++) {
+                            float4_t d = PER_ROW ? v : (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                            for (int p = PARTS - 1; p >= 0; p--)
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[k][g][p], bw[a][k][g], d, 0, 0, 0);
+                            if constexpr (PER_ROW) {
+                                v = d;
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(scur[a][k][g], d[e], v[e]);
+                            }
+                        }
+                    acc[a][b] += v;
+                }
+                if constexpr (!PER_ROW) {
+                    // The next block's MFMAs take the weights from here on: left
+                    // alone the compiler runs every block's MFMAs first, and their
+                    // results (16 registers a tile and step) spill or cost the
+                    // SIMD its second and third wave.
+#pragma unroll
+                    for (int a = 0; a < RT; a++)
+#pragma unroll
+                        for (int k = 0; k < KG; k++)
+                            asm volatile("" : "+v"(acc[a][b]), "+v"(bw[a][k][0]), "+v"(bw[a][k][1]));
+                }
             }
+            buf ^= 1;  // last read in the step before, ordered by that step's barrier
+            if (more) store_x(xt[buf], c + KG);
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < RT; a++)
+#pragma unroll
+                for (int k = 0; k < KG; k++) {
+                    wcur[a][k] = wnxt[a][k];
+                    scur[a][k][0] = snxt[a][k][0];
+                    scur[a][k][1] = snxt[a][k][1];
+                }
         }
-        buf ^= 1;  // last read in the step before, ordered by that step's barrier
-        if (more) store_x(xt[buf], c + KG);
-        __syncthreads();
+        float* yb = y + (size_t)split * split_stride;
 #pragma unroll
-        for (int a = 0; a < RT; a++)
+        for (int a = 0; a < RT; a++) {
+            const int n = (tile0 + a) * 16 + r;
+            if (n >= N) continue;
+            const float s = PER_ROW ? sc[n] : 1.0f;
 #pragma unroll
-            for (int k = 0; k < KG; k++) {
-                wcur[a][k] = wnxt[a][k];
-                scur[a][k][0] = snxt[a][k][0];
-                scur[a][k][1] = snxt[a][k][1];
-            }
-    }
-    float* yb = y + (size_t)split * split_stride;
+            for (int b = 0; b < CB; b++)
 #pragma unroll
-    for (int a = 0; a < RT; a++) {
-        const int n = (tile0 + a) * 16 + r;
-        if (n >= N) continue;
-        const float s = PER_ROW ? sc[n] : 1.0f;
-#pragma unroll
-        for (int b = 0; b < CB; b++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int m = b * 16 + 4 * q + e;
-                if (m < mrows) yb[(size_t)(m0 + m) * ldy + n] = acc[a][b][e] * s;
-            }
+                for (int e = 0; e < 4; e++) {
+                    const int m = b * 16 + 4 * q + e;
+                    const float v = EXP ? __builtin_amdgcn_ldexpf(acc[a][b][e], -EXP) : acc[a][b][e];
+                    if (m < mrows && (!EXP || fabsf(v) <= 3.402823466e38f)) yb[(size_t)(m0 + m) * ldy + n] = v * s;
+                }
+        }
+    };
+    pass(std::integral_constant<int, 0>{});
+    if constexpr (XF32) {
+        // Rows with vanishing parts: once more, scaled.  A sum too large for
+        // that keeps its first value (what it misses is under 2^-110 of its
+        // group's scale).
+        if (__syncthreads_or((lost & 0xFFFFu) != 0)) pass(std::integral_constant<int, SPLIT_EXP>{});
     }
 }
 

@@ -14,7 +14,7 @@ namespace th {
 // no more than the MFMA GEMM and its split-K reduction (2048 x 2048, m = 5:
 // 8.5 against 9.1 us).  Beyond that the GEMM reads the weights once where the
 // GEMV took a launch per four rows: 11008 x 4096, f32 rows, m = 5 28.0 -> 16
-// us, m = 100 429 -> 46 us; at four rows on 4096 x 4096 the GEMV is still the
+// us, m = 100 429 -> 51 us; at four rows on 4096 x 4096 the GEMV is still the
 // faster one (7.9 against 12 us).
 static bool q8_uses_gemv(const th_qweight* w, size_t m) {
     return m <= 4 || (m <= 8 && w->rows * w->cols <= ((size_t)1 << 22));

@@ -296,6 +296,38 @@ def test_q8_gemm(dev, rows, cols, m, scales, dt):
     assert np.all(np.abs(y - ref) <= (cols + bpr + 16) * 2.0 ** -24 * mag)
 
 
+@pytest.mark.parametrize("rows,cols", [(130, 200), (40, 1100), (37, 45)])
+@pytest.mark.parametrize("m", [9, 33, 129])  # each block height of the GEMM
+@pytest.mark.parametrize("scales", ["row", "group"])
+def test_q8_gemm_exponent_range(dev, rows, cols, m, scales):
+    """f32 rows of the smallest numbers, subnormals among them, next to rows near
+    the largest, under scales that bring them back: the bound of test_q8_gemm."""
+    rng = np.random.default_rng(rows + cols + m)
+    bpr = (cols + 31) // 32
+    q = rng.integers(-127, 128, (rows, cols), np.int8)
+    sc = np.exp2(rng.uniform(-9, 100, (rows, 1 if scales == "row" else bpr))).astype(np.float32)
+    sc[rows // 2:] *= np.float32(2.0 ** -100)
+    if scales == "row":
+        w = dev.q8_upload_rowwise(q, sc.reshape(-1), rows, cols)
+    else:
+        blocks = np.zeros((rows, bpr), capi.Q8_BLOCK)
+        blocks["scale"] = sc
+        qp = np.zeros((rows, bpr * 32), np.int8)
+        qp[:, :cols] = q
+        blocks["values"] = qp.reshape(rows, bpr, 32)
+        w = dev.q8_upload_blocks(blocks.reshape(-1), rows, cols)
+    exps = rng.integers(-149, -90, m)
+    exps[::3] = rng.integers(60, 110, len(exps[::3]))
+    x = (rng.uniform(1, 2, (m, cols)) * rng.choice([-1.0, 1.0], (m, cols)) * np.exp2(exps)[:, None]).astype(np.float32)
+    y = dev.gemv_q8(dev.upload(x), m, w).to_numpy().reshape(m, rows).astype(np.float64)
+    wf = q.astype(np.float64) * np.repeat(sc.astype(np.float64), cols if scales == "row" else 32, axis=1)[:, :cols]
+    ref, mag = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    ok = (mag > 2.0 ** -100) & (mag < 2.0 ** 127)  # neither subnormal results nor sums beyond f32
+    assert ok.mean() > 0.2 and ok[::3].any() and ok[1::3].any()
+    with np.errstate(invalid="ignore"):
+        assert np.all(np.abs(y - ref)[ok] <= ((cols + bpr + 16) * 2.0 ** -24 * mag)[ok])
+
+
 def test_reference_kats_on_device(dev):
     """q8_matvec_basic / q4_matvec_basic (quantize.rs:326-353) through the device."""
     wf = np.array([1, 2, 3, 4, 5, 6], np.float32)
