@@ -11,9 +11,10 @@
 // rows of one tile, so a K/V row is read once for all of them; there is no
 // length cap (the reference CUDA kernel holds scores in a fixed 2048-float
 // array, attention_cuda.rs:85).  Scores, softmax and sums are f32: with an f16
-// cache the f32 operand of each product goes in as two f16 parts (hi + lo, 22
-// bits of a row brought to [2^12, 2^13); probabilities times 2^12), with an
-// f32 cache the products run on the f32 MFMA.
+// cache the f32 operand of each product goes in as three f16 parts, which hold
+// all 24 bits of a value down to 2^-26 of the row's largest (AttnParts); with an
+// f32 cache the products run on the f32 MFMA.  An MFMA truncates what it adds to
+// a larger sum, so sums stay short and meet in plain additions.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -100,13 +101,39 @@ typedef __attribute__((address_space(3))) attn_short4_t attn_lds_short4_t;
 // f16 cache: k octets as loaded, V^T from row-major LDS by transposing reads.
 // f32 cache: v_mfma_f32_16x16x4, contraction index g of step (c, e) = dim
 // 16c + 4g + e (S) and key 4g + e of a tile (P.V).
+//
+// The f32 operand against an f16 cache, brought to at most 2^15: x = h + 2^-11 (m
+// + l), each part f16 with the eleven bits that the ones before left.  m and l
+// share a factor, so what x keeps below h reaches 2^-35, and sum up apart from h.
+struct AttnParts {
+    _Float16 h, m, l;
+    __device__ __forceinline__ explicit AttnParts(float x) {
+        h = (_Float16)x;
+        const float r = (x - (float)h) * 2048.0f;
+        m = (_Float16)r;
+        l = (_Float16)(r - (float)m);
+    }
+    __device__ __forceinline__ static float join(float h, float ml) { return __builtin_fmaf(ml, 1.0f / 2048.0f, h); }
+};
+constexpr int ATTN_TOP = 15;  // the row's largest in [2^14, 2^15)
+
+// Sum of N values in pairs, then pairs of pairs.
+template <int N>
+__device__ __forceinline__ attn_f32x4_t attn_tree_sum(attn_f32x4_t (&v)[N]) {
+#pragma unroll
+    for (int w = 1; w < N; w *= 2)
+#pragma unroll
+        for (int i = 0; i + w < N; i += 2 * w) v[i] += v[i + w];
+    return v[0];
+}
+
 template <int D, typename CT, int KT>
 struct AttnWave {
     static constexpr bool H = sizeof(CT) == 2;
     static constexpr int NK = H ? D / 32 : D / 16;  // 16-byte pieces of a K row per lane
     static constexpr int NDT = D / 16;
     static constexpr int LD = D + (H ? 8 : 4);      // LDS row stride (elements)
-    attn_f16x8_t qh[H ? NK : 1], ql[H ? NK : 1];
+    attn_f16x8_t qh[H ? NK : 1], qm[H ? NK : 1], ql[H ? NK : 1];
     attn_f32x4_t qf[H ? 1 : NK];
     attn_f32x4_t o[NDT];
     float m, l;
@@ -133,14 +160,15 @@ struct AttnWave {
             }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            qe = range_exp(mx, XPREP_TOP);
+            qe = range_exp(mx, ATTN_TOP);
 #pragma unroll
             for (int c = 0; c < NK; c++)
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
-                    const float x = __builtin_amdgcn_ldexpf(v[c][i], -qe);
-                    qh[c][i] = (_Float16)x;
-                    ql[c][i] = (_Float16)(x - (float)qh[c][i]);
+                    const AttnParts x(__builtin_amdgcn_ldexpf(v[c][i], -qe));
+                    qh[c][i] = x.h;
+                    qm[c][i] = x.m;
+                    ql[c][i] = x.l;
                 }
         } else {
 #pragma unroll
@@ -150,23 +178,47 @@ struct AttnWave {
 
     // scores of one 16-key tile from its K pieces
     __device__ __forceinline__ attn_f32x4_t score(const attn_u32x4_t (&k)[NK]) const {
-        attn_f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+        const attn_f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (H) {
+            constexpr int CH = D > 128 ? 2 : 1;  // pieces that sum up in one chain (two: the registers end)
+            attn_f32x4_t ml = z, h[NK / CH];
 #pragma unroll
             for (int c = 0; c < NK; c++)
-                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(attn_f16x8_t, k[c]), ql[c], s, 0, 0, 0);
+                ml = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(attn_f16x8_t, k[c]), ql[c], ml, 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < NK; c++)
-                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(attn_f16x8_t, k[c]), qh[c], s, 0, 0, 0);
+                ml = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(attn_f16x8_t, k[c]), qm[c], ml, 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < NK; c++)
+                h[c / CH] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(attn_f16x8_t, k[c]), qh[c],
+                                                                   c % CH ? h[c / CH] : z, 0, 0, 0);
+            attn_f32x4_t s = attn_tree_sum(h);
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[i] = AttnParts::join(s[i], ml[i]);
             return s;
-        } else {  // four chains: short sums, and no MFMA waits for the one before it
-            attn_f32x4_t t[4] = {s, s, s, s};
+        } else {
+            // Sums of eight products, which meet in pairs as soon as the next
+            // piece's MFMAs are on their way.
+            attn_f32x4_t level[5], d[2], p[2];
 #pragma unroll
-            for (int c = 0; c < NK; c++)
+            for (int c = 0; c <= NK; c++) {
+                if (c < NK) {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    t[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(attn_f32x4_t, k[c])[e], qf[c][e], t[e], 0, 0, 0);
-            return (t[0] + t[1]) + (t[2] + t[3]);
+                    for (int e = 0; e < 4; e++)
+                        d[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(attn_f32x4_t, k[c < NK ? c : 0])[e],
+                                                                        qf[c < NK ? c : 0][e], e < 2 ? z : d[e & 1], 0, 0, 0);
+                }
+                if (c > 0) {
+                    attn_f32x4_t u = p[0] + p[1];
+                    int l = 0;
+#pragma unroll
+                    for (int n = c - 1; n & 1; n >>= 1) u = level[l++] + u;
+                    level[l] = u;
+                }
+                p[0] = d[0];
+                p[1] = d[1];
+            }
+            return level[NK == 4 ? 2 : NK == 8 ? 3 : 4];
         }
     }
 
@@ -211,19 +263,20 @@ struct AttnWave {
         };
         if constexpr (H) {
             constexpr int KP = (KT + 1) / 2;  // 32-key steps (an odd last tile pairs with zeros)
-            attn_f16x8_t ph[KP], pl[KP];
+            attn_f16x8_t ph[KP], pm[KP], pl[KP];
 #pragma unroll
             for (int c = 0; c < KP; c++)
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const int t = 2 * c + (i >> 2);
-                    const float x = t < KT ? p[t < KT ? t : 0][i & 3] * 4096.0f : 0.0f;
-                    ph[c][i] = (_Float16)x;
-                    pl[c][i] = (_Float16)(x - (float)ph[c][i]);
+                    const AttnParts x(t < KT ? p[t < KT ? t : 0][i & 3] * 32768.0f : 0.0f);
+                    ph[c][i] = x.h;
+                    pm[c][i] = x.m;
+                    pl[c][i] = x.l;
                 }
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
-                attn_f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
+                attn_f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f}, ml = d;
 #pragma unroll
                 for (int c = 0; c < KP; c++) {
                     // lane r of a row group addresses four dims of key (r >> 2) and gets four keys of dim r
@@ -236,9 +289,12 @@ struct AttnWave {
                     }
                     const attn_f16x4_t a0 = __builtin_bit_cast(attn_f16x4_t, v[0]), a1 = __builtin_bit_cast(attn_f16x4_t, v[1]);
                     const attn_f16x8_t va = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[c], d, 0, 0, 0);
+                    ml = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[c], ml, 0, 0, 0);
+                    ml = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pm[c], ml, 0, 0, 0);
                     d = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[c], d, 0, 0, 0);
                 }
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] = AttnParts::join(d[i], ml[i]);
                 join(dt, d);
             }
         } else {
@@ -256,12 +312,12 @@ struct AttnWave {
         }
     }
 
-    __device__ __forceinline__ void finish() {  // l over the row's lanes; o back from its 2^12
+    __device__ __forceinline__ void finish() {  // l over the row's lanes; o back from its 2^15
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
         if constexpr (H) {
 #pragma unroll
-            for (int t = 0; t < NDT; t++) o[t] *= 1.0f / 4096.0f;
+            for (int t = 0; t < NDT; t++) o[t] *= 1.0f / 32768.0f;
         }
     }
 };
@@ -315,15 +371,27 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
 #pragma unroll
             for (int c = 0; c < Wave::NK; c++) k[t][c] = *(const attn_u32x4_t*)(kr + Wave::dim0(c, g));
         }
+        auto load_v = [&]() {
 #pragma unroll
-        for (int i = 0; i < VL; i++) {
-            const int idx = lane + 64 * i;
-            v[i] = *(const attn_u32x4_t*)((const char*)(vc + (size_t)min(key0 + idx / CPR, j1 - 1) * kv_dim + kv_h * D) +
-                                          (idx % CPR) * 16);
-        }
+            for (int i = 0; i < VL; i++) {
+                const int idx = lane + 64 * i;
+                v[i] = *(const attn_u32x4_t*)((const char*)(vc + (size_t)min(key0 + idx / CPR, j1 - 1) * kv_dim + kv_h * D) +
+                                              (idx % CPR) * 16);
+            }
+        };
+        // every load on its way before the first is used (left alone the
+        // compiler sinks V's to their stores, one wait each); with 256 dims V
+        // takes the registers that K leaves
+        if constexpr (D <= 128) load_v();
+        __builtin_amdgcn_sched_barrier(0);
         attn_f32x4_t sc[KT];
 #pragma unroll
         for (int t = 0; t < KT; t++) sc[t] = w.score(k[t]);
+        if constexpr (D > 128) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_v();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         const float a = w.softmax(sc, key0, last, scale, g);
 #pragma unroll
         for (int i = 0; i < VL; i++) {
@@ -428,7 +496,7 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
 // in LDS, the next block's loads in flight meanwhile.  With one split the
 // result goes out, else a record per row that attn_rows_merge_kernel merges.
 // 384 queries behind 512 positions, 16 heads on 8 kv heads of 128 dims, f16
-// cache: 240 -> 24 us (the split kernel reads every K/V row once per query).
+// cache: 240 -> 31 us (the split kernel reads every K/V row once per query).
 template <int D, typename CT>
 struct AttnPre {
     static constexpr int KB = 128 * 64 / D * 2 / (int)sizeof(CT) < 64 ? 128 * 64 / D * 2 / (int)sizeof(CT) : 64;
@@ -598,9 +666,16 @@ static void launch_attn_rows(const float* q, const void* kc, const void* vc, int
         };
         // Up to 2048 keys four waves spread a context over more CUs (1200 keys,
         // D 128: 10.3 against 12.0 us); beyond, eight keep the splits few (8000
-        // keys, four query heads on each of 4 kv heads: 15.0 against 20.1).
-        if (n <= 2048) decode(std::integral_constant<int, 4>{});
-        else decode(std::integral_constant<int, 8>{});
+        // keys, four query heads on each of 4 kv heads: 15.0 against 20.1).  Two
+        // waves a SIMD have too few registers for 256 dims of f32 (9000 keys,
+        // four heads on each of 4: 41.9 with four waves, 44.8 with eight).
+        if constexpr (D <= 128 || sizeof(CT) == 2) {
+            if (n > 2048) {
+                decode(std::integral_constant<int, 8>{});
+                return;
+            }
+        }
+        decode(std::integral_constant<int, 4>{});
         return;
     }
     const size_t tiles = ceil_div(R, (size_t)64), nkb = ceil_div(n, (size_t)AttnPre<D, CT>::KB);

@@ -169,6 +169,14 @@ def _attention_f64(q, k, v, start, ql, H, Hkv, D):
     (4, 4, 256, 100, 65),   # one row past a 64-row tile
     (12, 4, 64, 700, 64),   # splits of the key blocks
     (8, 8, 128, 17, 130),
+    (2, 1, 64, 40, 8),      # sixteen rows, less than a pass of the waves
+    (2, 1, 256, 40, 8),
+    (8, 2, 64, 1100, 4),    # four waves, several splits
+    (8, 2, 128, 1600, 4),
+    (16, 2, 128, 2100, 2),  # eight waves
+    (3, 1, 256, 3500, 5),   # 256 dims: eight waves against f16, four against f32
+    (16, 16, 128, 0, 95),   # whole row tiles, one split
+    (8, 8, 256, 100, 65),   # one row past a 64-row tile of 256 dims
 ])
 @pytest.mark.parametrize("f16", [True, False])
 def test_kv_attention_tiles(dev, H, Hkv, D, start, ql, f16):
@@ -195,7 +203,52 @@ def test_kv_attention_tiles(dev, H, Hkv, D, start, ql, f16):
         assert np.max(np.abs(out - ref)) <= bound
 
 
-@pytest.mark.parametrize("ql,start", [(1, 600), (40, 0), (40, 600)])  # decode, one split, several splits
+def _two_key_attention(dev, ql, D, f16, q, k0, k1, v0, v1):
+    """One head; every query row is q and sees keys 0 and 1 (row 0 only key 0) next
+    to keys of weight zero, whose V is zero."""
+    start = 1 if ql == 1 else 0
+    T = start + ql
+    k = np.zeros((T, D), np.float32)
+    k[2:, 0] = -65504.0
+    k[0], k[1] = k0, k1
+    v = np.zeros((T, D), np.float32)
+    v[0], v[1] = v0, v1
+    up = (lambda a: dev.upload(oracle.f32_to_f16(a.reshape(-1)), capi.F16)) if f16 else (lambda a: dev.upload(a))
+    out = dev.kv_attention(dev.upload(np.tile(q, (ql, 1)).astype(np.float32)), up(k), up(v), start, ql, 1, 1, D)
+    return out.to_numpy().reshape(ql, D)[1 if ql > 1 else 0:]
+
+
+@pytest.mark.parametrize("ql", [1, 40])  # the decode and the prompt kernel
+@pytest.mark.parametrize("D", [64, 256])  # 1/sqrt(D) is exact
+@pytest.mark.parametrize("f16", [True, False])
+def test_kv_attention_last_bits_of_q(dev, ql, D, f16):
+    """Two scores that differ in the last bits of a 24-bit q.  The difference is
+    exact in f32; weights, sum and output round once each."""
+    for n in (1, 2049, 3001, 4095):  # past 2048 the f16 nearest to q leaves twelve bits
+        q = np.zeros(D, np.float32)
+        q[0], q[1] = 4096.0 + n * 2.0 ** -11, 4096.0
+        k0, k1 = np.eye(D, dtype=np.float32)[:2]
+        out = _two_key_attention(dev, ql, D, f16, q, k0, k1, 1.0, -1.0)
+        want = np.tanh(n * 2.0 ** -11 / np.sqrt(D) / 2)
+        assert np.max(np.abs(out - want)) <= 4 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("ql", [1, 40])
+@pytest.mark.parametrize("f16", [True, False])
+def test_kv_attention_small_probabilities(dev, ql, f16):
+    """A key of weight 2^-33 to 2^-47 whose V is large enough to count."""
+    D = 64
+    for bits in (33, 38, 42, 47):
+        q = np.zeros(D, np.float32)
+        q[0] = np.float32(bits * np.log(2.0) * 8)
+        k0, k1 = np.eye(D, dtype=np.float32)[0], np.zeros(D, np.float32)
+        out = _two_key_attention(dev, ql, D, f16, q, k0, k1, 2.0 ** -14, 49152.0)
+        p = np.exp(-float(q[0]) / 8)
+        want = (2.0 ** -14 + p * 49152.0) / (1 + p)
+        assert np.max(np.abs(out - want)) <= want * 2.0 ** -21
+
+
+@pytest.mark.parametrize("ql,start", [(1, 600), (1, 2100), (40, 0), (40, 600), (64, 1100)])  # each kernel, one or more splits
 @pytest.mark.parametrize("f16", [True, False])
 def test_kv_attention_infinities(dev, ql, start, f16):
     """An infinite V reaches the queries that attend to it, in its own dim
