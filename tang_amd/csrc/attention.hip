@@ -698,18 +698,32 @@ void launch_kv_attention(const float* q, const void* kc, const void* vc, bool f1
     if (q_len == 0 || n_heads == 0) return;
     const bool tuned = head_dim == 64 || head_dim == 128 || head_dim == 256;
     // The split kernel (one workgroup per query, head and 64 keys) remains for
-    // what is too small to pay for 16-row tiles.  Where the lines lie, in us a
-    // call (row tiles / split kernel), f16 cache: D 128, G 1, 60 keys 5.3 / 7.0,
-    // 300 9.3 / 7.6, 1200 10.3 / 9.2, 4000 12.6 / 15.5; G 2, 300 10.1 / 8.8,
-    // 1200 11.6 / 11.9, 8000 20.2 / 44.8; D 64, G 2, 300 7.7 / 7.7; D 256,
-    // G 2, 1200 15.2 / 14.1, 2000 16.7 / 17.6.  f32 cache (its MFMA has a
-    // sixteenth of the rate): D 128, G 1, 4000 17.5 / 16.7, 8000 22.3 / 26.6;
-    // G 4, 1200 15.7 / 12.5, 2000 15.7 / 15.8, 8000 20.4 / 40.2.
+    // what is too small to pay for 16-row tiles.  Its time grows with the work,
+    // the tiles' hardly does below a certain size.  Where the lines lie, in us a
+    // call (row tiles / split kernel), 8 kv heads unless stated, G query heads each.
+    // Up to 16 rows, f16 cache: few keys D 64 128 5.1 / 6.4, D 128 60 5.6 / 6.9,
+    // 128 6.5 / 7.0, D 256 60 8.5 / 8.7, 128 11.7 / 8.9; many D 64 G 2 512 8.4 / 7.6,
+    // 1024 8.6 / 9.1, G 4 512 8.4 / 7.8, 900 8.6 / 9.8, D 128 G 1 1200 10.0 / 8.4, 2048 10.6 / 10.3, 4000 12.5 / 14.4, G 2
+    // 1024 9.9 / 9.7, 8000 16.3 / 35.7, D 256 G 1 4096 19.7 / 17.4, 6144 20.9 / 20.4, G 2
+    // 2048 17.9 / 16.6, 3072 18.1 / 22.3.
+    // f32 cache (its MFMA has a sixteenth of the rate): few D 64 64 5.2 / 6.3, D 128
+    // 32 6.9 / 6.9, 64 7.6 / 7.1, D 256 64 9.1 / 9.0; many D 64 G 1 4096 12.3 / 13.7, G 4
+    // 700 9.5 / 8.6, 1024 9.6 / 10.2, D 128 G 1 8192 21.3 / 19.9, 12000 26.8 / 30.9, G 2
+    // 3000 16.1 / 19.6, G 4 1200 14.2 / 12.7, D 256 G 1 16000 57.4 / 59.5, G 4 3000 25.2 /
+    // 36.7.
+    // More rows (queries x keys), f16 cache: D 64 4 kv heads 64 x 256 9.7 / 8.1, 18 x
+    // 2000 14.6 / 17.7; D 128 17 x 17 6.4 / 7.4, 20 x 400 14.5 / 9.8, 40 x 400 14.8 / 13.0; D
+    // 256 4 kv heads 17 x 600 19.1 / 12.1, 64 x 256 16.8 / 19.1.  f32 cache: D 64 G 2 32 x
+    // 512 14.4 / 15.1, 4 kv heads 64 x 256 13.6 / 8.1; D 128 40 x 400 19.1 / 15.7, 40 x 800
+    // 21.7 / 23.5, 128 x 128 14.3 / 13.8; D 256 40 x 140 20.2 / 16.8, 64 x 256 20.4 / 29.4.
     const size_t G = n_heads / n_kv_heads, R = q_len * G, n = cache_start + q_len;
     bool tiles;
-    if (R > 16) tiles = f16 || R * n >= 4096;
-    else if (f16) tiles = n <= 128 || n * std::min<size_t>(G, 2) * 128 >= 2048 * head_dim;
-    else tiles = n <= 64 || n * std::min<size_t>(G, 4) * 128 >= 8192 * head_dim;
+    const size_t work = q_len * n_heads * n;  // times the dims: products of scores
+    if (R > 16 && f16) tiles = n <= 64 || work * std::max<size_t>(head_dim, 128) >= (size_t)1 << 24;
+    else if (R > 16) tiles = work * head_dim >= (size_t)1 << 24;
+    else if (f16) tiles = n <= (head_dim <= 128 ? 128 : 64) || n * std::min<size_t>(G, head_dim <= 64 ? 3 : 2) >= (head_dim <= 128 ? 2048 : 6144);
+    else if (G > 1) tiles = n <= (head_dim <= 64 ? 64 : 32) || n * std::min<size_t>(G, 4) >= 2048 + 32 * head_dim;
+    else tiles = n <= (head_dim <= 64 ? 64 : 32) || n >= (head_dim <= 64 ? 4096 : head_dim <= 128 ? 10240 : 16384);
     if (tuned && !tiles) {
         // enough 64-position chunks per split that the merge fits in LDS
         const size_t max_splits = 64 * 1024 / ((head_dim + 2) * sizeof(float));
