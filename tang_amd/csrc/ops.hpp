@@ -91,19 +91,24 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// MFMA results and branches.  The compiler keeps a read of a result the
-// required wait states behind its MFMA in straight code; moved past a taken
-// branch, a read was seen one or two states behind.  So every kernel keeps to
-// one of two forms: mfma_pin after reads that belong before a branch (the
-// additions of a step's sums), which holds them there, or mfma_settle on sums
+// MFMA results and branches.  Nothing holds a read of a result back that comes
+// too early; the compiler fills the distance up, but has left one or two wait
+// states of eight where a read was moved past a taken branch.  So every kernel
+// keeps to one of two forms: mfma_pin behind reads that belong before a branch
+// (the additions of a step's sums), which holds them there, or mfma_settle on sums
 // that are first read behind their loop, which waits out the longest MFMA.
+// tests/test_mfma_distance.py follows every path of the built code.
 template <typename V>
 __device__ __forceinline__ void mfma_pin(V& v) {
     asm volatile("" : "+v"(v));
 }
-template <typename V>
-__device__ __forceinline__ void mfma_settle(V& v) {
-    asm volatile("s_nop 15\n\ts_nop 3" : "+v"(v));
+template <typename V, int N, int M>
+__device__ __forceinline__ void mfma_settle(V (&v)[N][M]) {
+    asm volatile("s_nop 15\n\ts_nop 3");
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int j = 0; j < M; j++) mfma_pin(v[i][j]);
 }
 
 // One DPP move inside rows of 16 lanes (CTRL: the dpp_ctrl encoding).

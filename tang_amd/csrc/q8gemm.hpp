@@ -226,6 +226,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                             asm volatile("" : "+v"(acc[a][b]), "+v"(bw[a][k][0]), "+v"(bw[a][k][1]));
                 }
             }
+#pragma unroll
+            for (int a = 0; a < RT; a++)
+#pragma unroll
+                for (int b = 0; b < CB; b++) mfma_pin(acc[a][b]);
             buf ^= 1;  // last read in the step before, ordered by that step's barrier
             if (more) store_x(xt[buf], c + KG);
             __syncthreads();

@@ -1365,6 +1365,7 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
     }
 
     // D layout: lane holds rows 4*(lane/16)+i (weight rows) of column lane%16.
+    mfma_settle(acc);
     int xe[CB];
 #pragma unroll
     for (int b = 0; b < CB; b++) {
@@ -1487,6 +1488,7 @@ __global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __re
         for (int a = 0; a < RT; a++) wcur[a] = wnxt[a];
         scur = snxt;
     }
+    mfma_settle(acc);
 #pragma unroll
     for (int a = 0; a < RT; a++)
 #pragma unroll
@@ -1614,7 +1616,7 @@ __global__ __launch_bounds__(64 * KW) void q4_gemm_rows_kernel(const uint4* __re
         for (int a = 0; a < RT; a++) wcur[a] = wnxt[a];
         scur = snxt;
 #pragma unroll
-        for (int a = 0; a < RT; a++) asm volatile("" : "+v"(acc[a]));  // MFMA results are read past the loop's branch
+        for (int a = 0; a < RT; a++) mfma_pin(acc[a]);  // scaled by the next step, past the loop's branch
     }
     if (lp == 0) wexps[wave][lr] = xe;
     __syncthreads();  // the activations' LDS becomes the partial tiles'
