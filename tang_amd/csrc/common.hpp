@@ -134,9 +134,10 @@ struct th_device {
     int* counters = nullptr;  // see device_counters
     void* noalloc_scratch = nullptr;  // this device's address of the th_gemm_q4_noalloc workspace
     size_t n_counters = 0;
-    // Workspace blocks that grew out of use after a graph capture: a recorded
-    // graph may still name them, so they stay until the device goes.
-    bool captured = false;
+    // Workspace blocks outgrown while a captured graph was there that may still
+    // name them: they stay until the last such graph goes.
+    int graphs = 0;          // captured graphs, and a capture in progress
+    bool capturing = false;  // between th_capture_begin and th_capture_end
     std::vector<void*> retired;
     int live = 0;          // buffers, weights and engines that hold this device
     bool closed = false;   // th_device_destroy ran; the struct waits for live == 0

@@ -29,13 +29,13 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 // The workspace that a device starts with.
 constexpr size_t FIRST_WORKSPACE = (size_t)32 << 20;
 
-// Grow one of the device's workspaces to `bytes`.  Once a graph has been
-// captured on the device the outgrown block is kept (its graphs may name it)
-// and sizes double, so that the kept blocks stay below the one in use.
+// Grow one of the device's workspaces to `bytes`.  While a captured graph is
+// there the outgrown block is kept (the graph may name it) and sizes double, so
+// that the kept blocks stay below the one in use.
 static void* grow_workspace(th_device* dev, void*& ptr, size_t& have, size_t bytes) {
     if (bytes <= have) return ptr;
     size_t want = std::max(bytes, (size_t)1 << 20);
-    if (ptr && dev->captured) {
+    if (ptr && dev->graphs > 0) {
         want = std::max(want, 2 * have);
         dev->retired.push_back(ptr);
     } else if (ptr) {
@@ -66,6 +66,14 @@ int* device_counters(th_device* dev, size_t n) {
     dev->counters = (int*)p;
     dev->n_counters = have / sizeof(int);
     return dev->counters;
+}
+
+// One captured graph (or open capture) less: with the last one the outgrown
+// blocks go.  The device's work is drained.
+static void graph_gone(th_device* d) {
+    if (--d->graphs > 0) return;
+    for (void* p : d->retired) (void)hipFree(p);
+    d->retired.clear();
 }
 
 static void check_buf(const th_buffer* b, const char* what) {
@@ -332,7 +340,8 @@ int th_capture_begin(th_device* d) {
     TH_API_BEGIN
     TH_REQUIRE(d, "null device");
     TH_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-    d->captured = true;
+    d->capturing = true;
+    d->graphs++;
     TH_API_END
 }
 
@@ -340,10 +349,18 @@ int th_capture_end(th_device* d, th_graph** out) {
     TH_API_BEGIN
     TH_REQUIRE(d && out, "null argument");
     hipGraph_t g = nullptr;
-    TH_HIP(hipStreamEndCapture(d->stream, &g));
     hipGraphExec_t ge = nullptr;
-    const hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
+    hipError_t e = hipStreamEndCapture(d->stream, &g);
+    if (e == hipSuccess) {
+        e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+    }
+    const bool open = d->capturing;
+    d->capturing = false;
+    if (e != hipSuccess && open) {
+        device_drain(d);
+        graph_gone(d);
+    }
     TH_HIP(e);
     th_graph* r = new th_graph();
     r->dev = d;
@@ -367,6 +384,7 @@ int th_graph_destroy(th_graph* g) {
     (void)hipGraphExecDestroy(g->exec);
     th_device* d = g->dev;
     delete g;
+    graph_gone(d);
     device_release(d);
     TH_API_END
 }

@@ -52,3 +52,55 @@ def test_captured_gemm_splits_before_any_call(m):
             assert np.array_equal(y.to_numpy(), eager)
     finally:
         g.free()
+
+
+def test_replay_after_workspaces_grew():
+    """A graph names the workspaces that its calls used.  Larger calls afterwards
+    outgrow them (and other buffers take whatever is freed): every replay still
+    gives the eager result, and the outgrown memory comes back with the graph."""
+    dev = capi.HipComputeDevice(0)
+    rng = np.random.default_rng(3)
+    heads, hd, n = 16, 256, 3000
+    kv = [dev.upload(rng.standard_normal(n * heads * hd).astype(np.float16).view(np.uint16), capi.F16) for _ in range(2)]
+    q = dev.upload(rng.standard_normal(heads * hd).astype(np.float32))
+    nib, sc = capi.synth_q4(5, 512, 1024)
+    w4 = dev.q4_upload_packed(nib, sc, 512, 1024, capi.F16)
+    w8 = dev.q8_upload_rowwise(rng.integers(-128, 128, (1000, 4096), np.int8),
+                               rng.uniform(0.005, 0.02, 1000).astype(np.float32), 1000, 4096)
+    x4, x8 = dev.upload(rng.standard_normal(40 * 1024)), dev.upload(rng.standard_normal(20 * 4096))
+    out = [dev.alloc(heads * hd), dev.alloc(40 * 512), dev.alloc(20 * 1000)]
+
+    def calls():  # K splits' records and arrival counters, prepared activations, K splits' partial sums
+        capi.check(capi.lib().th_kv_attention(dev.handle, q.handle, kv[0].handle, kv[1].handle, n - 1, 1, heads, heads, hd,
+                                              out[0].handle))
+        dev.gemm_q4(x4, 40, w4, out[1])
+        dev.gemv_q8(x8, 20, w8, out[2])
+
+    calls()
+    eager = [o.to_numpy() for o in out]
+    g = dev.capture(calls)
+    big_q = dev.alloc(496 * 64 * hd)  # 64 heads on 16, two splits: records of 65 MB
+    dev.zero_buffer(big_q)
+    big_out = dev.alloc(496 * 64 * hd)
+    big_x, big_y = dev.alloc(4096 * 1024), dev.alloc(4096 * 512)
+    dev.zero_buffer(big_x)
+    for _ in range(2):
+        capi.check(capi.lib().th_kv_attention(dev.handle, big_q.handle, kv[0].handle, kv[1].handle, n - 496, 496, 64, heads, hd,
+                                              big_out.handle))
+        dev.gemm_q4(big_x, 4096, w4, big_y)
+        held = [dev.upload(np.full(k << 18, np.nan, np.float32)) for k in (1, 2, 4, 8, 16, 32)]
+        for i in range(3):
+            for o in out:
+                dev.zero_buffer(o)
+            g.launch()
+            dev.sync()
+            for o, e in zip(out, eager):
+                assert np.array_equal(o.to_numpy(), e)
+    free = dev.memory_info()[0]
+    g.free()
+    assert dev.memory_info()[0] >= free + (32 << 20)  # the blocks that only the graph named
+    calls()
+    assert all(np.array_equal(o.to_numpy(), e) for o, e in zip(out, eager))
+    for b in held + [big_q, big_out, big_x, big_y, q, x4, x8] + kv + out:
+        b.free()
+    dev.close()
