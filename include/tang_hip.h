@@ -78,7 +78,8 @@ int th_timer_stop(th_device* dev, float* ms);
  * for callers that repeat a fixed sequence of calls, as a decode loop does.
  * The recorded calls must not allocate: make each one once before capture
  * (workspaces grow on first use).  Replays read and write the same buffers
- * the recorded calls named. */
+ * the recorded calls named, and give the same bits as the calls made eagerly.
+ * Workspaces that a graph names stay until the device's last graph goes. */
 int th_capture_begin(th_device* dev);
 int th_capture_end(th_device* dev, th_graph** out);
 int th_graph_launch(th_graph* g);

@@ -40,6 +40,13 @@ inline bool stream_capturing(hipStream_t s) {
 
 // Grow-only stream-ordered workspace owned by the device.
 void* device_scratch(th_device* dev, size_t bytes);
+// K splits of a GEMM, at most `ks`, whose partial sums of `part` bytes each fit
+// the workspace that a device starts with.  A call so takes the same splits, and
+// gives the same bits, eagerly, captured, and whatever grew the workspace before.
+// (The GEMMs ask for some three workgroups a CU of at most 32 KiB each: 24 MiB on
+// 256 CUs.)  Only a device that found no room for that workspace runs a captured
+// call with the splits that it has.
+size_t workspace_splits(th_device* dev, size_t ks, size_t part, hipStream_t s);
 // The configuration a sampler was created with (sampling.cpp).
 const th_sampling_config& sampler_config(const th_sampler* s);
 // Zero-initialised ints that kernels leave zero again on exit (arrival

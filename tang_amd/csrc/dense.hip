@@ -336,10 +336,8 @@ static void matmul_launch(const MatOperand& A, const MatOperand& B, float* c, si
     const size_t m = A.rows, n = B.rows, part = m * n * sizeof(float), cus = dev->num_cus;
     const unsigned gx = (unsigned)ceil_div(n, (size_t)(4 / WGM * TN * 16)), gy = (unsigned)ceil_div(m, (size_t)(WGM * TM * 16));
     // Split K where the tiles leave CUs idle: two workgroups per CU, each
-    // split at least 128 deep.  (While a stream is captured the workspace may
-    // not grow: a call takes the splits that it holds.)
-    size_t ks = std::max<size_t>(1, std::min({2 * cus / ((size_t)gx * gy), k / 128, (size_t)16}));
-    if (ks * part > dev->scratch_bytes && stream_capturing(dev->stream)) ks = std::max<size_t>(1, dev->scratch_bytes / part);
+    // split at least 128 deep.
+    size_t ks = workspace_splits(dev, std::min({2 * cus / ((size_t)gx * gy), k / 128, (size_t)16}), part, dev->stream);
     const size_t per = round_up(ceil_div(k, ks), (size_t)32);
     ks = ceil_div(k, per);
     float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : c;

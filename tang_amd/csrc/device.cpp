@@ -51,6 +51,12 @@ static void* grow_workspace(th_device* dev, void*& ptr, size_t& have, size_t byt
 
 void* device_scratch(th_device* dev, size_t bytes) { return grow_workspace(dev, dev->scratch, dev->scratch_bytes, bytes); }
 
+size_t workspace_splits(th_device* dev, size_t ks, size_t part, hipStream_t s) {
+    ks = std::max<size_t>(1, std::min(ks, FIRST_WORKSPACE / part));
+    if (ks * part > dev->scratch_bytes && stream_capturing(s)) ks = std::max<size_t>(1, dev->scratch_bytes / part);
+    return ks;
+}
+
 void* device_scratch_x(th_device* dev, size_t bytes) {
     return grow_workspace(dev, dev->scratch_x, dev->scratch_x_bytes, bytes);
 }
@@ -265,8 +271,7 @@ int th_device_create(int ordinal, th_device** out) {
     hipDeviceProp_t prop;
     TH_HIP(hipGetDeviceProperties(&prop, ordinal));
     d->num_cus = prop.multiProcessorCount;
-    // Enough for the K splits of ordinary batches, so that a graph captured
-    // before any call of its size is not left unsplit.  Without it the device
+    // Enough for every GEMM's K splits (workspace_splits).  Without it the device
     // works all the same.
     if (hipMalloc(&d->scratch, FIRST_WORKSPACE) == hipSuccess) {
         d->scratch_bytes = FIRST_WORKSPACE;

@@ -316,16 +316,13 @@ static size_t q8_gemm_splits(size_t base, size_t NCH, size_t cus) {
     return best;
 }
 
-// While a stream is captured the workspace may not grow: a call takes the splits
-// that it holds (4096 x 7248, m = 6: 19 us split, 77 unsplit).
 template <int RT, int CB, int KG, bool XF32, bool PR, bool VEC>
 static void q8_gemm_launch(const th_qweight* w, const void* x, size_t m, size_t ldx, float* y, size_t ldy,
                            hipStream_t s, th_device* dev) {
     const size_t NT = w->Np / 16, NCH = w->Kp / 64;
     const unsigned gx = (unsigned)ceil_div(NT, (size_t)(4 * RT)), gy = (unsigned)ceil_div(m, (size_t)(16 * CB));
     const size_t part = m * w->rows * sizeof(float);
-    size_t ks = q8_gemm_splits((size_t)gx * gy, NCH, (size_t)dev->num_cus);
-    if (ks * part > dev->scratch_bytes && stream_capturing(s)) ks = std::max<size_t>(1, dev->scratch_bytes / part);
+    size_t ks = workspace_splits(dev, q8_gemm_splits((size_t)gx * gy, NCH, (size_t)dev->num_cus), part, s);
     const size_t cps = round_up(ceil_div(NCH, ks), (size_t)KG);
     ks = ceil_div(NCH, cps);
     float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : y;

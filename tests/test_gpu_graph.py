@@ -54,6 +54,38 @@ def test_captured_gemm_splits_before_any_call(m):
         g.free()
 
 
+@pytest.mark.parametrize("grown", [False, True])
+@pytest.mark.parametrize("m,k,n,bd", [(5, 4000, 700, capi.F32), (100, 2100, 1000, capi.BF16), (130, 4096, 8000, capi.F32)])
+def test_captured_matmul_matches_eager(grown, m, k, n, bd):
+    """A matmul captured as a device's first call, or after calls that outgrew the
+    first workspace, gives the eager call's bits on every replay."""
+    dev = capi.HipComputeDevice(0)
+    rng = np.random.default_rng(m)
+    if grown:
+        kv = dev.alloc(3000 * 16 * 256, capi.F16)
+        q, o = dev.alloc(496 * 64 * 256), dev.alloc(496 * 64 * 256)
+        for b in (kv, q):
+            dev.zero_buffer(b)
+        capi.check(capi.lib().th_kv_attention(dev.handle, q.handle, kv.handle, kv.handle, 2504, 496, 64, 16, 256, o.handle))
+    a = dev.upload(rng.standard_normal(m * k))
+    b = dev.convert(dev.upload(rng.standard_normal(k * n)), bd)
+    c = dev.alloc(m * n)
+    call = lambda: capi.check(capi.lib().th_matmul_ex(dev.handle, a.handle, b.handle, m, k, n, 0, 0, 0, c.handle))
+    g = dev.capture(call)
+    other = capi.HipComputeDevice(0)  # its workspace holds what a new device's does
+    a2 = other.upload(a.to_numpy())
+    b2 = other.convert(other.upload(dev.convert(b, capi.F32).to_numpy()), bd)
+    eager = other.matmul(a2, b2, m, k, n).to_numpy()
+    call()
+    assert np.array_equal(c.to_numpy(), eager)
+    for _ in range(3):
+        dev.zero_buffer(c)
+        g.launch()
+        dev.sync()
+        assert np.array_equal(c.to_numpy(), eager)
+    g.free()
+
+
 def test_replay_after_workspaces_grew():
     """A graph names the workspaces that its calls used.  Larger calls afterwards
     outgrow them (and other buffers take whatever is freed): every replay still
