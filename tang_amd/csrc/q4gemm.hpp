@@ -39,8 +39,8 @@ inline void q4_wave_launch(const th_qweight* w, PreparedX xp, size_t m, const Ep
 }
 
 // Weight tiles and waves of a workgroup by the number of workgroups that four
-// tiles each would give (`wgs`): the more there are, the larger the tile and
-// the fewer the waves that split its K.  Measured, us (4x4 / 4x8 / 2x8 / 1x8,
+// tiles each would give (`wgs`), per CU: the more there are, the larger the tile
+// and the fewer the waves that split its K.  Measured on 256 CUs, us (4x4 / 4x8 / 2x8 / 1x8,
 // tiles x waves): 2048 x 2048, m = 512 (256) 15.9 / 15.4 / 18.4 / 21.8; m = 384
 // (192) 14.8 / 14.3 / 17.1 / 18.0; m = 192 (96) 13.9 / 12.9 / 11.2 / 13.2;
 // m = 64 (32) 13.4 / 11.9 / 10.1 / 9.4; 11008 x 4096, m = 96 (344) 26.2 / 29.4 /
@@ -49,14 +49,14 @@ inline void q4_wave_launch(const th_qweight* w, PreparedX xp, size_t m, const Ep
 // sixteen waves (4096 x 11008, m = 16: 1x8 14.8, 1x16 13.3).
 template <int CB, typename ST, typename Epi>
 inline void q4_wave_shape(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
-    const size_t wgs = ceil_div(w->Np / 16, (size_t)4) * ceil_div(m, (size_t)(16 * CB));
+    const size_t wgs = ceil_div(w->Np / 16, (size_t)4) * ceil_div(m, (size_t)(16 * CB)), cus = w->dev->num_cus;
     if constexpr (CB <= 2) {
-        if (wgs > 144) return q4_wave_launch<2, CB, 4, ST>(w, xp, m, epi, s);
+        if (wgs > cus * 9 / 16) return q4_wave_launch<2, CB, 4, ST>(w, xp, m, epi, s);
     } else {
-        if (wgs > 224) return q4_wave_launch<4, CB, 4, ST>(w, xp, m, epi, s);
-        if (wgs > 144) return q4_wave_launch<4, CB, 8, ST>(w, xp, m, epi, s);
+        if (wgs > cus * 7 / 8) return q4_wave_launch<4, CB, 4, ST>(w, xp, m, epi, s);
+        if (wgs > cus * 9 / 16) return q4_wave_launch<4, CB, 8, ST>(w, xp, m, epi, s);
     }
-    if (wgs > 72) return q4_wave_launch<2, CB, 8, ST>(w, xp, m, epi, s);
+    if (wgs > cus * 9 / 32) return q4_wave_launch<2, CB, 8, ST>(w, xp, m, epi, s);
     if constexpr (CB == 1) {
         if (w->Kp >= 32 * 128) return q4_wave_launch<1, CB, 16, ST>(w, xp, m, epi, s);
     }
@@ -82,9 +82,9 @@ inline void q4_rows_launch(const th_qweight* w, const float* x, size_t m, size_t
 // Rows that cannot be read in aligned fours are prepared (scalar loads took
 // 3333 x 3333 from 76 to 137 us over eight linears).
 inline bool q4_rows_direct(const th_qweight* w, const float* x, size_t m, size_t ldx) {
-    const size_t tiles = w->Np / 16;
+    const size_t tiles = w->Np / 16, cus = w->dev->num_cus;
     return m <= 16 && w->cols % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
-           w->cols <= (tiles <= 256 ? 8192u : 3072u) && ldx < ((size_t)1 << 25);  // 32-bit offsets into 16 rows
+           w->cols <= (tiles <= cus ? 8192u : 3072u) && ldx < ((size_t)1 << 25);  // 32-bit offsets into 16 rows
 }
 
 // One weight tile a workgroup while that is at most one workgroup a CU, two
@@ -93,9 +93,9 @@ inline bool q4_rows_direct(const th_qweight* w, const float* x, size_t m, size_t
 // 5.2 / 5.5; 11264 x 2048 9.2 / 8.2 / 7.8).
 template <typename ST, typename Epi>
 inline void q4_gemm_rows(const th_qweight* w, const float* x, size_t m, size_t ldx, const Epi& epi, hipStream_t s) {
-    const size_t tiles = w->Np / 16;
-    if (tiles <= 256) q4_rows_launch<1, 8, ST>(w, x, m, ldx, epi, s);
-    else if (tiles <= 512) q4_rows_launch<2, 8, ST>(w, x, m, ldx, epi, s);
+    const size_t tiles = w->Np / 16, cus = w->dev->num_cus;
+    if (tiles <= cus) q4_rows_launch<1, 8, ST>(w, x, m, ldx, epi, s);
+    else if (tiles <= 2 * cus) q4_rows_launch<2, 8, ST>(w, x, m, ldx, epi, s);
     else q4_rows_launch<2, 4, ST>(w, x, m, ldx, epi, s);
 }
 
@@ -111,14 +111,14 @@ inline void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, const Ep
 }
 
 // The kernel with activations staged in LDS once a workgroup's waves would
-// load them from L2 too often: from some 5600 tiles of 64 x 64 (us, wave kernel
+// load them from L2 too often: from some 22 tiles of 64 x 64 a CU (us, wave kernel
 // / this one: 22016 x 4096, m = 768 191 / 199, 1024 253 / 249, 1536 381 / 364;
 // 11008 x 4096, m = 1536 195 / 220; 4096 x 4096 79 / 102).  128-row blocks
 // beyond m = 1024, 64-row ones before.
 template <typename ST, typename Epi>
 inline void q4_gemm_dense(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
     const size_t tiles = ceil_div(w->Np / 16, (size_t)4) * ceil_div(m, (size_t)64);
-    if (tiles >= 5600) {
+    if (tiles >= (size_t)w->dev->num_cus * 175 / 8) {
         if (m > 1024) q4_mfma_launch<2, 8, ST>(w, xp, m, epi, s);
         else q4_mfma_launch<2, 4, ST>(w, xp, m, epi, s);
         return;
