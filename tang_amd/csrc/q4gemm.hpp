@@ -27,14 +27,12 @@ inline void set_smem(K kernel, size_t bytes) {
 
 template <int RT, int CB, int KW, typename ST, typename Epi>
 inline void q4_wave_launch(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
-    GemmDense src;
-    src.M = (int)m;
-    auto k = q4_gemm_wave_kernel<RT, CB, KW, ST, GemmDense, Epi>;
+    auto k = q4_gemm_wave_kernel<RT, CB, KW, ST, Epi>;
     const size_t lds = (size_t)KW * RT * CB * 1024;
     set_smem(k, lds);
     TH_LAUNCH(k, dim3((unsigned)ceil_div(w->Np / 16, (size_t)RT), (unsigned)ceil_div(m, (size_t)(16 * CB))), dim3(64 * KW),
-              lds, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
-              (int)w->rows, (int)w->Kp, (int)w->Kp);
+              lds, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, (int)m,
+              (int)w->rows, (int)w->Kp);
     TH_LAUNCH_CHECK();
 }
 

@@ -1404,25 +1404,16 @@ __global__ __launch_bounds__(256) void q4_gemm_mfma_kernel(const uint4* __restri
 // second launch (same prepared layout): 2048 x 2048, m = 64 17.0 -> 9.4, m = 384
 // 25.7 -> 14.3; 4096 x 4096, m = 64 20.3 -> 13.0, m = 512 43 -> 33; 11008 x 4096,
 // m = 32 24.6 -> 14.5, m = 256 53 -> 40, m = 1024 145 -> 131 (705 TFLOP/s).
-template <int RT, int CB, int KW, typename ST, typename Src = GemmDense, typename Epi = EpiGemmStore>
+template <int RT, int CB, int KW, typename ST, typename Epi>
 __global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __restrict__ wt, const ST* __restrict__ sc,
                                                                const int* __restrict__ wexp,
                                                                const uint16_t* __restrict__ xin,
-                                                               const int* __restrict__ xexp, Epi epi, Src src, int N,
-                                                               int Kp, int ldx) {
+                                                               const int* __restrict__ xexp, Epi epi, int M, int N, int Kp) {
     extern __shared__ __align__(16) char wave_lds[];
     float4_t* part = (float4_t*)wave_lds;  // [KW][RT * CB][64]
-    int mrows = 0, bx = blockIdx.x, by = blockIdx.y, bz = 0;
-    if constexpr (!Src::GROUPED) gemm_xcd_tile(bx, by, bz);
-    {
-        const uint4* wsel = wt;
-        const ST* ssel = sc;
-        const int* esel = wexp;
-        if (!src.select(by, CB * 16, wsel, ssel, esel, mrows)) return;
-        wt = wsel;
-        sc = ssel;
-        wexp = esel;
-    }
+    int bx = blockIdx.x, by = blockIdx.y, bz = 0;
+    gemm_xcd_tile(bx, by, bz);
+    const int m0 = by * CB * 16, mrows = min(CB * 16, M - m0);
     const int GQ = Kp >> 7, NT = (N + 15) >> 4, tile0 = bx * RT;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, r = lane & 15;
@@ -1438,7 +1429,7 @@ __global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __re
     const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xin, 0xFFFFFFF0u);  // in-range offsets only
     uint32_t xoff[CB];  // bytes; rows past mrows re-read the last live row (never stored)
 #pragma unroll
-    for (int b = 0; b < CB; b++) xoff[b] = (uint32_t)xp_index(src.x_row(min(b * 16 + r, mrows - 1)), q, ldx >> 3) * 16u;
+    for (int b = 0; b < CB; b++) xoff[b] = (uint32_t)xp_index(m0 + min(b * 16 + r, mrows - 1), q, Kp >> 3) * 16u;
     u32x4_t xh[2][2][CB];  // [half][group of the half][block]
     auto load_x = [&](int gq, int h) {
 #pragma unroll
@@ -1499,13 +1490,13 @@ __global__ __launch_bounds__(64 * KW) void q4_gemm_wave_kernel(const uint4* __re
         float4_t v = part[t * 64 + lane];
 #pragma unroll
         for (int w = 1; w < KW; w++) v += part[(w * RT * CB + t) * 64 + lane];
-        const int xe = xexp[src.x_row(ml < mrows ? ml : 0)];
+        const int xe = xexp[m0 + (ml < mrows ? ml : 0)];
         const int4 we = *(const int4*)(wexp + min(tile, NT - 1) * 16 + 4 * q);
         const int wev[4] = {we.x, we.y, we.z, we.w};
         const bool live = ml < mrows && tile < NT;
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = __builtin_amdgcn_ldexpf(v[e], xe + wev[e]);
-        epi(src.out_row(live ? ml : 0), tile * 16 + 4 * q, N, live, v);
+        epi(m0 + (live ? ml : 0), tile * 16 + 4 * q, N, live, v);
     }
 }
 
