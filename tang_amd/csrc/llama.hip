@@ -764,25 +764,27 @@ static void llama_launch_steps(th_llama* m, size_t n) {
 
 static void llama_launch_step(th_llama* m) { llama_launch_steps(m, 1); }
 
-constexpr size_t PREFILL_CHUNK = 512;  // prompt rows per pass (workspace ~100 MB at the 7B shape)
+constexpr size_t PREFILL_CHUNK = 512;  // prompt rows per pass (workspace ~37 MB at the 7B shape)
 
 static void prefill_reserve(th_llama* m, size_t rows) {
     if (rows <= m->pf_rows) return;
     device_sync(m->dev);
-    void* old[] = {m->pf_x, m->pf_qkv, m->pf_q, m->pf_y, m->pf_gu, m->pf_xb, m->pf_att, m->pf_sg, m->pf_tok, m->pf_xe};
-    for (void* p : old)
-        if (p) (void)hipFree(p);
+    // (a failure below leaves no pointer to freed memory behind)
+    auto drop = [](auto*&... p) { ((p ? (void)hipFree(p) : void(), p = nullptr), ...); };
+    drop(m->pf_x, m->pf_qkv, m->pf_q, m->pf_y, m->pf_gu, m->pf_xb, m->pf_att, m->pf_sg, m->pf_tok, m->pf_xe);
+    m->pf_rows = 0;
     const th_llama_config& c = m->cfg;
     const size_t d = c.d_model, ff = c.d_ff;
+    const size_t few = std::min<size_t>(rows, 16);  // beyond that the GEMMs' epilogues and prepared rows take over
     m->pf_x = dalloc<float>(rows * d);
-    m->pf_y = dalloc<float>(rows * d);
-    m->pf_qkv = dalloc<float>(rows * (m->qd + 2 * m->kvd));
+    m->pf_y = dalloc<float>((c.head_dim == 64 || c.head_dim == 128 ? few : rows) * d);
+    m->pf_qkv = dalloc<float>(few * (m->qd + 2 * m->kvd));
     m->pf_q = dalloc<float>(rows * m->qd);
-    m->pf_gu = dalloc<float>(rows * 2 * ff);
+    m->pf_gu = dalloc<float>(std::max(few * 2 * ff, ceil_div(rows * ff, 2)));  // f32 gate and up, or bf16 products
     const size_t rows16 = round_up(rows, 16);  // prepared rows come in blocks of 16
     m->pf_xb = dalloc<uint16_t>(rows16 * round_up(d, 128));  // bf16 rows, or prepared rows of Kp
     m->pf_att = dalloc<uint16_t>(rows16 * round_up((size_t)m->qd, 128));
-    m->pf_sg = dalloc<uint16_t>(rows16 * round_up(ff, 128));
+    m->pf_sg = dalloc<uint16_t>(few * round_up(ff, 128));
     m->pf_xe = dalloc<int>(2 * rows);
     m->pf_tok = dalloc<int32_t>(rows);
     m->pf_rows = rows;
