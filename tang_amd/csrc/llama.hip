@@ -634,8 +634,6 @@ static void llama_start(th_llama* m, const LlamaState& start, hipStream_t s) {
 static void llama_read_results(th_llama* m, size_t n, int32_t* tokens, float* logits) {
     const size_t V = (size_t)m->cfg.vocab;
     if (tokens || logits) {
-        if (!m->results)
-            TH_HIP(hipHostMalloc((void**)&m->results, (V + (size_t)m->max_steps) * 4, hipHostMallocDefault));
         aql_wait(m->dev);
         float* lo = m->results;
         int32_t* to = (int32_t*)(m->results + V);
@@ -1063,6 +1061,7 @@ int th_llama_create(th_device* dev, const th_llama_config* cfg, th_llama** out) 
         m->sg = dalloc<uint16_t>(c.d_ff);
         m->st = dalloc<LlamaState>(1);
         m->history = dalloc<int32_t>(m->max_steps);
+        TH_HIP(hipHostMalloc((void**)&m->results, ((size_t)c.vocab + (size_t)m->max_steps) * 4, hipHostMallocDefault));
         std::vector<float> cs((size_t)c.max_seq * c.head_dim / 2), sn(cs.size());
         rope_tables_host(c.head_dim, c.max_seq, c.rope_theta, cs.data(), sn.data());
         TH_HIP(hipMemcpy(m->rope_cos, cs.data(), cs.size() * 4, hipMemcpyHostToDevice));
