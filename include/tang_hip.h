@@ -178,7 +178,8 @@ int th_gemv_q8(th_device* dev, const th_buffer* x, size_t m, const th_qweight* w
  * prepared activations) is a fixed per-GPU device array of
  * TH_NOALLOC_SCRATCH_BYTES, not an allocation: the call makes no hipMalloc /
  * hipFree.  Fails with TH_ERR_INVALID when the prepared activations, about
- * 2*m*K bytes, do not fit.  Every call on one GPU shares the array: calls that
+ * 2*m*K bytes, do not fit.  (Rows of K above 139,000 that fit only without their
+ * padding sum up in another order.)  Every call on one GPU shares the array: calls that
  * overlap on one GPU (two streams, two threads) race. */
 #define TH_NOALLOC_SCRATCH_BYTES (64u << 20)
 int th_gemm_q4_noalloc(th_device* dev, const th_buffer* x, size_t m, const th_qweight* w, th_buffer* y);

@@ -86,9 +86,9 @@ struct PreparedX {
 // false: rows of Kp one after the other, for the grouped source.
 PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t ldx, size_t K, size_t Kp,
                     hipStream_t s, const int* rows = nullptr, void* workspace = nullptr, bool blocked = true);
-size_t prepared_x_bytes(size_t m, size_t Kp);
+size_t prepared_x_bytes(size_t m, size_t Kp, bool blocked = true);
 // Beyond TH_NOALLOC_SCRATCH_BYTES: room for the last block's padding rows (K up
-// to 139,000).
+// to 139,000; wider rows whose padding does not fit stay row-major).
 constexpr size_t NOALLOC_SLACK = (size_t)4 << 20;
 // The MFMA GEMM on prepared activations, for producers that write the layout
 // directly.  accumulate: y += x.W^T (a fused residual add) instead of y = x.W^T.

@@ -97,11 +97,11 @@ inline void q4_gemm_rows(const th_qweight* w, const float* x, size_t m, size_t l
     else q4_rows_launch<2, 4, ST>(w, x, m, ldx, epi, s);
 }
 
-template <int RT, int CB, typename ST, typename Epi>
+template <int RT, int CB, typename ST, typename Src = GemmDense, typename Epi>
 inline void q4_mfma_launch(const th_qweight* w, PreparedX xp, size_t m, const Epi& epi, hipStream_t s) {
-    GemmDense src;
+    Src src;
     src.M = (int)m;
-    TH_LAUNCH((q4_gemm_mfma_kernel<RT, CB, ST, GemmDense, Epi>),
+    TH_LAUNCH((q4_gemm_mfma_kernel<RT, CB, ST, Src, Epi>),
               dim3((unsigned)ceil_div(w->Np / 16, (size_t)(4 * RT)), (unsigned)ceil_div(m, (size_t)(16 * CB)), 1), dim3(256),
               0, s, (const uint4*)w->data, (const ST*)w->scales, (const int*)w->row_exp, xp.x, xp.xexp, epi, src,
               (int)w->rows, (int)w->Kp, (int)w->Kp);

@@ -168,13 +168,18 @@ void launch_splitk_reduce(const float* part, float* y, size_t m, size_t n, size_
 
 // Convert m activation rows (f32 or bf16, rows of ldx) into the MFMA GEMM's
 // prepared layout in the device's operand workspace.
-size_t prepared_x_bytes(size_t m, size_t Kp) { return round_up(m, 16) * Kp * 2 + round_up(m * sizeof(int), 256); }
+static size_t prepared_rows_bytes(size_t m, size_t Kp, bool blocked) {
+    return blocked ? round_up(m, 16) * Kp * 2 : round_up(m * Kp * 2, 256);
+}
+size_t prepared_x_bytes(size_t m, size_t Kp, bool blocked) {
+    return prepared_rows_bytes(m, Kp, blocked) + round_up(m * sizeof(int), 256);
+}
 
 PreparedX prepare_x(th_device* dev, const void* x, bool xf32, size_t m, size_t ldx, size_t K, size_t Kp,
                     hipStream_t s, const int* rows, void* workspace, bool blocked) {
     TH_REQUIRE(m * Kp * 2 < 0x7FFFFFF0u, "prepared activations above 2 GiB");  // 32-bit buffer offsets
-    const size_t xbytes = round_up(m, 16) * Kp * 2;
-    char* ws = workspace ? (char*)workspace : (char*)device_scratch_x(dev, prepared_x_bytes(m, Kp));
+    const size_t xbytes = prepared_rows_bytes(m, Kp, blocked);
+    char* ws = workspace ? (char*)workspace : (char*)device_scratch_x(dev, prepared_x_bytes(m, Kp, blocked));
     PreparedX p{(const uint16_t*)ws, (const int*)(ws + xbytes)};
     const size_t cpr = Kp / 8;
     if (cpr <= 8 * 256) {  // row per workgroup, in registers
@@ -235,21 +240,20 @@ static void q4_linear_t(const th_qweight* w, const void* x, size_t m, size_t ldx
     else if (!XF32 && m <= 8 && fits8) q4_span_launch<8, false, ST>(w, x, m, ldx, y, ldy, s, cus);
     else if (!XF32 && m <= 16 && fits16) q4_span_launch<16, false, ST>(w, x, m, ldx, y, ldy, s, cus);
     else {  // activations prepared once per call, then the MFMA GEMM
-        if (ws) {
-            const size_t xb = prepared_x_bytes(m, w->Kp);
-            // the whole blocks' padding rows go into the workspace's slack
-            TH_REQUIRE(round_up(m * w->Kp * 2, 256) + round_up(m * sizeof(int), 256) <= TH_NOALLOC_SCRATCH_BYTES &&
-                           xb <= ws_bytes,
+        // the whole blocks' padding rows go into the workspace's slack
+        if (ws)
+            TH_REQUIRE(prepared_x_bytes(m, w->Kp, false) <= TH_NOALLOC_SCRATCH_BYTES,
                        "workspace too small for the prepared activations (m x K too large)");
-        }
         if constexpr (XF32) {
             if (q4_rows_direct(w, (const float*)x, m, ldx)) {
                 q4_gemm_rows<ST>(w, (const float*)x, m, ldx, q4_store_epi(w, y, ldy, false), s);
                 return;
             }
         }
-        const PreparedX xp = prepare_x(dev, x, XF32, m, ldx, w->cols, w->Kp, s, nullptr, ws);
-        q4_gemm_store<ST>(w, xp, m, y, ldy, s, false);
+        const bool blocked = !ws || prepared_x_bytes(m, w->Kp) <= ws_bytes;
+        const PreparedX xp = prepare_x(dev, x, XF32, m, ldx, w->cols, w->Kp, s, nullptr, ws, blocked);
+        if (blocked) q4_gemm_store<ST>(w, xp, m, y, ldy, s, false);
+        else q4_mfma_launch<2, 4, ST, GemmDenseRows>(w, xp, m, q4_store_epi(w, y, ldy, false), s);
     }
 }
 

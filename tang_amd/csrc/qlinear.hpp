@@ -1078,6 +1078,11 @@ struct GemmDense {
     __device__ __forceinline__ int out_row(int m) const { return m0 + m; }
 };
 
+// The same rows one after the other in memory, as the grouped source's.
+struct GemmDenseRows : GemmDense {
+    static constexpr bool GROUPED = true;
+};
+
 // Epilogue of the MFMA GEMM: D fragment (weight rows n0..n0+3, activation
 // row m) of one lane, already scaled back to the true result; `live` is false
 // for rows past the block or the matrix.  Called by every lane (pairing

@@ -39,6 +39,18 @@ def test_noalloc_matches_gemm_q4_on_consecutive_calls(dev):
             assert max_abs_rel(got, ref) < 2e-2
 
 
+def test_noalloc_takes_rows_that_fit_without_padding(dev):
+    """Seventeen rows of 1.9M columns fill the workspace but for 2.5 MB; padded to
+    whole blocks of sixteen they would take twice as much.  The f32 sums run in
+    another order: K / 32 MFMAs, each of which rounds once."""
+    rows, cols, m = 16, 1900000, 17
+    print("noalloc wide rows", flush=True)
+    nib, sc16 = capi.synth_q4(4, rows, cols)
+    w = dev.q4_upload_packed(nib, sc16, rows, cols, capi.F16)
+    x = dev.upload(capi.synth_normal(60, m * cols, 1.0, capi.BF16), capi.BF16)
+    assert max_abs_rel(_noalloc(dev, x, m, w, rows), dev.gemm_q4(x, m, w).to_numpy().reshape(m, rows)) < cols / 32 * 2.0 ** -24
+
+
 def test_noalloc_rejects_oversize(dev):
     rows, cols, m = 64, 11008, 4096  # prepared activations: 4096 x 11008 x 2 B > 64 MiB
     nib, sc16 = capi.synth_q4(3, rows, cols)
