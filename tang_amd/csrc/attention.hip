@@ -57,36 +57,72 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const float* __restric
     for (int i = 0, d = lane; d < head_dim; i++, d += 64) out[(size_t)qi * total_dim + h * head_dim + d] = acc[i] * inv;
 }
 
-// One row (query qi, head h) by one wave in plain f32: the rows whose MFMA
-// result is not finite (an infinity times a part that is zero is NaN, and a
-// block's later keys carry weight zero rather than being left out).
+// One row (query, head) over some keys by one wave in plain f32, for the rows
+// whose MFMA sums are not finite (an infinity times a part that is zero is NaN, and
+// a block's later keys carry weight zero rather than being left out): blocks of
+// `block` keys every `step` from `from` on, up to `to`.  D / 8 lanes share a key;
+// the wave's keys meet at the end, when lane e holds sums of dims 8e..8e+7.
+struct AttnRow {
+    float m, l, acc[8];
+};
 template <int D, typename CT>
-__device__ __noinline__ void attn_row_plain(const float* __restrict__ q, const CT* __restrict__ kc,
-                                            const CT* __restrict__ vc, int kv_dim, int kv_off, int attend,
-                                            float* __restrict__ out, int lane) {
-    constexpr int E = D / 64;
+__device__ __noinline__ AttnRow attn_row_plain(const float* __restrict__ q, const CT* __restrict__ kc,
+                                               const CT* __restrict__ vc, int kv_dim, int from, int to, int block, int step,
+                                               int lane) {
+    constexpr int LPK = D / 8, KPW = 64 / LPK, U = sizeof(CT) == 2 ? 4 : 2;
+    const int slot = lane / LPK, e = lane % LPK;
     const float scale = 1.0f / sqrtf((float)D);
-    float qv[E], acc[E];
+    float qv[8];
+    AttnRow x;
+    x.m = -INFINITY;
+    x.l = 0.0f;
 #pragma unroll
-    for (int e = 0; e < E; e++) { qv[e] = q[lane + 64 * e]; acc[e] = 0.0f; }
-    float m = -INFINITY, l = 0.0f;
-    for (int j = 0; j < attend; j++) {
-        const CT* kr = kc + (size_t)j * kv_dim + kv_off;
-        const CT* vr = vc + (size_t)j * kv_dim + kv_off;
-        float d = 0.0f;
-#pragma unroll
-        for (int e = 0; e < E; e++) d += qv[e] * (float)kr[lane + 64 * e];
-        const float s = wave_sum(d) * scale;
-        const float mn = fmaxf(m, s), ref = mn == -INFINITY ? 0.0f : mn;
-        const float p = expf(s - ref), a = expf(m - ref);
-        l = l * a + p;
-#pragma unroll
-        for (int e = 0; e < E; e++) acc[e] = acc[e] * a + p * (float)vr[lane + 64 * e];
-        m = mn;
+    for (int i = 0; i < 8; i++) {
+        qv[i] = q[e * 8 + i];
+        x.acc[i] = 0.0f;
     }
-    const float inv = 1.0f / l;
+    bool nan = false;  // a NaN score: so is every output
+    for (int base = from; base < to && !nan; base += step) {
+        const int end = min(to, base + block);
+        for (int j0 = base; j0 < end && !nan; j0 += KPW * U) {
+            float k[U][8], v[U][8];
 #pragma unroll
-    for (int e = 0; e < E; e++) out[lane + 64 * e] = acc[e] * inv;
+            for (int u = 0; u < U; u++) {
+                const size_t at = (size_t)min(j0 + u * KPW + slot, end - 1) * kv_dim + e * 8;
+                load8<CT>(kc + at, k[u]);
+                load8<CT>(vc + at, v[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                float d = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) d += qv[i] * k[u][i];
+#pragma unroll
+                for (int o = LPK / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+                if (j0 + u * KPW + slot >= end) continue;
+                const float s = d * scale, mn = fmaxf(x.m, s), ref = mn == -INFINITY ? 0.0f : mn;
+                const float p = expf(s - ref), a = expf(x.m - ref);
+                x.l = x.l * a + p;
+#pragma unroll
+                for (int i = 0; i < 8; i++) x.acc[i] = x.acc[i] * a + p * v[u][i];
+                x.m = mn;
+            }
+            nan = __any(x.l != x.l);
+        }
+    }
+#pragma unroll
+    for (int o = LPK; o < 64; o <<= 1) {
+        const float mo = __shfl_xor(x.m, o, 64), lo = __shfl_xor(x.l, o, 64);
+        const float M = fmaxf(x.m, mo), f = x.m == -INFINITY ? 0.0f : expf(x.m - M), g = mo == -INFINITY ? 0.0f : expf(mo - M);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float ao = __shfl_xor(x.acc[i], o, 64);
+            x.acc[i] = x.acc[i] * f + ao * g;
+        }
+        x.l = x.l * f + lo * g;
+        x.m = M;
+    }
+    return x;
 }
 
 typedef _Float16 attn_f16x4_t __attribute__((ext_vector_type(4)));
@@ -312,6 +348,16 @@ struct AttnWave {
         }
     }
 
+    // whether this lane's sums are (a NaN score makes l one)
+    __device__ __forceinline__ bool finite() const {
+        bool f = l == l;
+#pragma unroll
+        for (int t = 0; t < NDT; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) f &= fabsf(o[t][i]) <= 3.402823466e38f;
+        return f;
+    }
+
     __device__ __forceinline__ void finish() {  // l over the row's lanes; o back from its 2^15
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
@@ -350,14 +396,13 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
     constexpr int CPR = D * (int)sizeof(CT) / 16, VL = KB * CPR / 64;
     extern __shared__ __align__(16) char lds[];
     __shared__ float sm[NW][16], sl[NW][16], sM[16];
-    __shared__ int s_flag, s_bad[16];
+    __shared__ int s_flag;
     const int kv_h = blockIdx.x, s = blockIdx.y, R = q_len * G, n_heads = n_kv_heads * G, kv_dim = n_kv_heads * D;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r = lane & 15;
     const int row = min(r, R - 1), qi = row / G;
     const int j0 = s * per, j1 = min(cache_start + q_len, j0 + per);
     CT* vs = (CT*)(lds + wave * T::REGION);
-    if (tid < 16) s_bad[tid] = 0;
     Wave w;
     w.init(q + ((size_t)qi * n_heads + kv_h * G + (row - qi * G)) * D, g);
     const float scale = 1.0f / sqrtf((float)D);
@@ -407,6 +452,20 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
 #pragma unroll
     for (int t = 0; t < Wave::NDT; t++) *(attn_f32x4_t*)(mo + r * D + t * 16 + 4 * g) = w.o[t];
     if (g == 0) { sm[wave][r] = w.m; sl[wave][r] = w.l; }
+    if (__any(!w.finite())) {
+        wave_lds_fence();
+        for (int rw = 0; rw < R; rw++) {
+            const int qr = rw / G;
+            const AttnRow x = attn_row_plain<D, CT>(q + ((size_t)qr * n_heads + kv_h * G + rw - qr * G) * D, kc + kv_h * D,
+                                                    vc + kv_h * D, kv_dim, j0 + wave * KB, min(j1, cache_start + qr + 1), KB,
+                                                    NW * KB, lane);
+            if (lane < D / 8) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) mo[rw * D + lane * 8 + i] = x.acc[i];
+            }
+            if (lane == 0) { sm[wave][rw] = x.m; sl[wave][rw] = x.l; }
+        }
+    }
     __syncthreads();
     if (tid < 16) {  // row tid: the waves' weights relative to the workgroup's maximum, and their sum
         float M = -INFINITY, L = 0.0f;
@@ -423,17 +482,13 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
     }
     __syncthreads();
     auto out_row = [&](int rw) { return out + ((size_t)(rw / G) * n_heads + kv_h * G + rw % G) * D; };
-    auto put = [&](int rw, int d, float o) {
-        out_row(rw)[d] = o;
-        if (!(fabsf(o) <= 3.402823466e38f)) s_bad[rw] = 1;
-    };
     for (int i = tid; i < R * D; i += 64 * NW) {
         const int rw = i / D, d = i % D;
         float A = 0.0f;
 #pragma unroll
         for (int x = 0; x < NW; x++) A = __builtin_fmaf(sm[x][rw], ((const float*)(lds + x * T::REGION))[rw * D + d], A);
         if (n_splits == 1) {
-            put(rw, d, A * (1.0f / sl[0][rw]));
+            out_row(rw)[d] = A * (1.0f / sl[0][rw]);
         } else {
             const size_t rec = ((size_t)kv_h * R + rw) * n_splits + s;
             st_coherent(&part_o[rec * D + d], A);
@@ -481,14 +536,9 @@ __global__ __launch_bounds__(64 * NW) void attn_rows_decode_kernel(
                 for (int u = 0; u < U; u++)
                     if (c + u < n_splits) A = __builtin_fmaf(wr[2 * (c + u)], o[u], A);
             }
-            put(i / D, i % D, A);
+            out_row(i / D)[i % D] = A;
         }
     }
-    __syncthreads();
-    for (int rw = wave; rw < R; rw += NW)
-        if (s_bad[rw])
-            attn_row_plain<D, CT>(q + ((size_t)(rw / G) * n_heads + kv_h * G + rw % G) * D, kc, vc, kv_dim, kv_h * D,
-                                  cache_start + rw / G + 1, out_row(rw), lane);
 }
 
 // More than 16 rows: workgroup = (64 rows of one kv head, kv head, split of
@@ -561,40 +611,39 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const float* __restrict_
     }
     w.finish();
     const bool live = w0 + r < R;
-    if (n_splits > 1) {
-        const size_t rec = ((size_t)kv_h * R + row) * n_splits + s;
-        if (live) {
+    const float inv = n_splits > 1 ? 1.0f : 1.0f / w.l;
+    // the record, or (one split) the result, of a row
+    auto place = [&](int rw) {
+        if (n_splits > 1) return part_o + (((size_t)kv_h * R + rw) * n_splits + s) * D;
+        return out + ((size_t)(rw / G) * n_heads + kv_h * G + rw % G) * D;
+    };
+    auto ml = [&](int rw) { return (float2*)(part_ml + 2 * (((size_t)kv_h * R + rw) * n_splits + s)); };
+    if (live) {
+        float* p = place(row);
 #pragma unroll
-            for (int t = 0; t < Wave::NDT; t++) *(attn_f32x4_t*)(part_o + rec * D + t * 16 + 4 * g) = w.o[t];
-            if (g == 0) *(float2*)(part_ml + 2 * rec) = make_float2(w.m, w.l);
-        }
-        return;
+        for (int t = 0; t < Wave::NDT; t++) *(attn_f32x4_t*)(p + t * 16 + 4 * g) = w.o[t] * inv;
+        if (n_splits > 1 && g == 0) *ml(row) = make_float2(w.m, w.l);
     }
-    const float inv = 1.0f / w.l;
-    float* orow = out + ((size_t)qi * n_heads + h) * D;
-    bool bad = false;
-#pragma unroll
-    for (int t = 0; t < Wave::NDT; t++) {
-        const attn_f32x4_t v = w.o[t] * inv;
-#pragma unroll
-        for (int i = 0; i < 4; i++) bad |= !(fabsf(v[i]) <= 3.402823466e38f);
-        if (live) *(attn_f32x4_t*)(orow + t * 16 + 4 * g) = v;
-    }
-    uint64_t todo = __ballot(bad && live);
+    uint64_t todo = __ballot(live && !w.finite());
     todo = (todo | (todo >> 16) | (todo >> 32) | (todo >> 48)) & 0xFFFF;
     for (; todo; todo &= todo - 1) {
-        const int rw = w0 + (int)__builtin_ctzll(todo), qx = rw / G, hx = kv_h * G + rw % G;
-        attn_row_plain<D, CT>(q + ((size_t)qx * n_heads + hx) * D, kc, vc, kv_dim, kv_h * D, cache_start + qx + 1,
-                              out + ((size_t)qx * n_heads + hx) * D, lane);
+        const int rw = w0 + (int)__builtin_ctzll(todo), qx = rw / G;
+        const AttnRow x = attn_row_plain<D, CT>(q + ((size_t)qx * n_heads + kv_h * G + rw % G) * D, kc + kv_h * D, vc + kv_h * D,
+                                                kv_dim, b0 * KB, min(b1 * KB, cache_start + qx + 1), KB, KB, lane);
+        const float xi = n_splits > 1 ? 1.0f : 1.0f / x.l;
+        float* p = place(rw);
+        if (lane < D / 8) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) p[lane * 8 + i] = x.acc[i] * xi;
+        }
+        if (n_splits > 1 && lane == 0) *ml(rw) = make_float2(x.m, x.l);
     }
 }
 
 // One wave per row: the splits' records merged in split order.
-template <int D, typename CT>
+template <int D>
 __global__ __launch_bounds__(256) void attn_rows_merge_kernel(const float* __restrict__ part_o,
-                                                              const float* __restrict__ part_ml, int n_splits,
-                                                              const float* __restrict__ q, const CT* __restrict__ kc,
-                                                              const CT* __restrict__ vc, int cache_start, int q_len,
+                                                              const float* __restrict__ part_ml, int n_splits, int q_len,
                                                               int G, int n_kv_heads, float* __restrict__ out) {
     constexpr int E = D / 64;
     const int R = q_len * G, n_heads = n_kv_heads * G, lane = threadIdx.x & 63;
@@ -614,15 +663,8 @@ __global__ __launch_bounds__(256) void attn_rows_merge_kernel(const float* __res
         for (int e = 0; e < E; e++) A[e] = __builtin_fmaf(f, po[(size_t)s * D + lane + 64 * e], A[e]);
     }
     const size_t o = ((size_t)qi * n_heads + h) * D;
-    bool bad = false;
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const float v = A[e] * (1.0f / L);
-        bad |= !(fabsf(v) <= 3.402823466e38f);
-        out[o + lane + 64 * e] = v;
-    }
-    if (__any(bad))
-        attn_row_plain<D, CT>(q + o, kc, vc, n_kv_heads * D, kv_h * D, cache_start + qi + 1, out + o, lane);
+    for (int e = 0; e < E; e++) out[o + lane + 64 * e] = A[e] * (1.0f / L);
 }
 
 template <int D, typename CT>
@@ -686,8 +728,8 @@ static void launch_attn_rows(const float* q, const void* kc, const void* vc, int
               k, v, cache_start, q_len, G, n_kv_heads, (int)splits, po, pml, out);
     TH_LAUNCH_CHECK();
     if (splits > 1) {
-        TH_LAUNCH((attn_rows_merge_kernel<D, CT>), dim3((unsigned)ceil_div(R * n_kv_heads, (size_t)4)), dim3(256), 0, s, po,
-                  pml, (int)splits, q, k, v, cache_start, q_len, G, n_kv_heads, out);
+        TH_LAUNCH(attn_rows_merge_kernel<D>, dim3((unsigned)ceil_div(R * n_kv_heads, (size_t)4)), dim3(256), 0, s, po, pml,
+                  (int)splits, q_len, G, n_kv_heads, out);
         TH_LAUNCH_CHECK();
     }
 }

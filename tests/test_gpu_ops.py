@@ -268,6 +268,26 @@ def test_kv_attention_infinities(dev, ql, start, f16):
     assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.max(np.abs(out[fin] - ref[fin])) < 1e-5
 
 
+@pytest.mark.parametrize("ql,start", [(1, 600), (4, 2100), (40, 0), (64, 1100)])
+@pytest.mark.parametrize("f16", [True, False])
+def test_kv_attention_nans(dev, ql, start, f16):
+    """A NaN in q takes its own row, in K the rows that attend to the key, in V its
+    dim; everything else is as without."""
+    H, Hkv, D, T = 4, 2, 64, start + ql
+    rng = np.random.default_rng(ql)
+    q = rng.standard_normal((ql, H, D)).astype(np.float16).astype(np.float32)
+    k, v = (rng.standard_normal((T, Hkv, D)).astype(np.float16).astype(np.float32) for _ in range(2))
+    q[0, 3, 11] = np.nan
+    if ql > 1:
+        k[T - 2, 1, 7] = np.nan
+    v[3 if T > 300 else 0, 0, 5] = np.nan
+    up = (lambda a: dev.upload(oracle.f32_to_f16(a.reshape(-1)), capi.F16)) if f16 else (lambda a: dev.upload(a))
+    out = dev.kv_attention(dev.upload(q.reshape(-1)), up(k), up(v), start, ql, H, Hkv, D).to_numpy()
+    ref, _ = _attention_f64(q, k, v, start, ql, H, Hkv, D)
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    assert np.max(np.abs(out - ref)[~np.isnan(ref)]) < 1e-5
+
+
 def test_convert_roundtrip(dev):
     x = np.concatenate([capi.synth_normal(1, 5000), np.array([65504.0, 1e-7, -0.0], np.float32)]).astype(np.float32)
     b = dev.convert(dev.upload(x), capi.BF16).to_numpy()
