@@ -754,14 +754,15 @@ void launch_kv_attention(const float* q, const void* kc, const void* vc, bool f1
     // 3000 16.1 / 19.6, G 4 1200 14.2 / 12.7, D 256 G 1 16000 57.4 / 59.5, G 4 3000 25.2 /
     // 36.7.
     // More rows (queries x keys), f16 cache: D 64 4 kv heads 64 x 256 9.7 / 8.1, 18 x
-    // 2000 14.6 / 17.7; D 128 17 x 17 6.4 / 7.4, 20 x 400 14.5 / 9.8, 40 x 400 14.8 / 13.0; D
-    // 256 4 kv heads 17 x 600 19.1 / 12.1, 64 x 256 16.8 / 19.1.  f32 cache: D 64 G 2 32 x
-    // 512 14.4 / 15.1, 4 kv heads 64 x 256 13.6 / 8.1; D 128 40 x 400 19.1 / 15.7, 40 x 800
-    // 21.7 / 23.5, 128 x 128 14.3 / 13.8; D 256 40 x 140 20.2 / 16.8, 64 x 256 20.4 / 29.4.
+    // 2000 14.6 / 17.7; D 128 17 x 17 6.4 / 7.4, 30 x 100 9.0 / 8.0, 64 x 128 9.7 / 9.3, 16 kv
+    // heads 77 x 80 9.2 / 13.4, 40 x 400 14.8 / 13.0, 100 x 200 12.6 / 14.6; D 256 64 x 128
+    // 16.0 / 12.8, 64 x 256 16.8 / 19.1.  f32 cache: D 64 G 2 32 x 512 14.4 / 15.1, 4 kv heads
+    // 64 x 256 13.6 / 8.1; D 128 40 x 400 19.1 / 15.7, 100 x 200 17.8 / 18.8; D 256 40 x 140
+    // 20.2 / 16.8, 64 x 128 18.3 / 17.7, 64 x 256 20.4 / 29.4.
     const size_t G = n_heads / n_kv_heads, R = q_len * G, n = cache_start + q_len;
     bool tiles;
-    const size_t work = q_len * n_heads * n;  // times the dims: products of scores
-    if (R > 16 && f16) tiles = n <= 64 || work * std::max<size_t>(head_dim, 128) >= (size_t)1 << 24;
+    const size_t work = q_len * n_heads * n;  // scores
+    if (R > 16 && f16) tiles = n <= 64 || work >= (size_t)1 << (n <= 128 && head_dim <= 128 ? 16 : 17);
     else if (R > 16) tiles = work * head_dim >= (size_t)1 << 24;
     else if (f16) tiles = n <= (head_dim <= 128 ? 128 : 64) || n * std::min<size_t>(G, head_dim <= 64 ? 3 : 2) >= (head_dim <= 128 ? 2048 : 6144);
     else if (G > 1) tiles = n <= (head_dim <= 64 ? 64 : 32) || n * std::min<size_t>(G, 4) >= 2048 + 32 * head_dim;

@@ -176,7 +176,7 @@ def _attention_f64(q, k, v, start, ql, H, Hkv, D):
     (16, 2, 128, 2100, 2),  # eight waves
     (3, 1, 256, 3500, 5),   # 256 dims: eight waves against f16, four against f32
     (16, 16, 128, 0, 95),   # whole row tiles, one split
-    (8, 8, 256, 100, 65),   # one row past a 64-row tile of 256 dims
+    (16, 16, 256, 100, 65),  # one row past a 64-row tile of 256 dims
 ])
 @pytest.mark.parametrize("f16", [True, False])
 def test_kv_attention_tiles(dev, H, Hkv, D, start, ql, f16):
