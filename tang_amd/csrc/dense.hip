@@ -25,12 +25,6 @@ namespace th {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-template <bool BF16>
-__device__ __forceinline__ float ld_el(const void* p, size_t i) {
-    if constexpr (BF16) return __uint_as_float((uint32_t)((const uint16_t*)p)[i] << 16);
-    else return ((const float*)p)[i];
-}
-
 // ---------------------------------------------------------------------------
 // matmul: C[m][n] (+)= op(A)[m][k] . op(B)[k][n].  A is [m][k] row-major, or
 // [k][m] transposed; B is [k][n], or [n][k] transposed (device.rs:103,407,425);
@@ -44,9 +38,10 @@ __device__ __forceinline__ float ld_el(const void* p, size_t i) {
 // - Operands or results so small that parts of them vanish: the tile is summed
 //   once more with its f32 operands times 2^SPLIT_EXP.
 // - A result that is not finite (an infinity times a part that is zero, a value
-//   or a sum too large for that factor): summed on the f32 MFMA.  So is a K of
-//   one step, where the truncation inside an MFMA costs more than f32's
-//   roundings (from two steps on it costs less).
+//   or a sum too large for that factor): summed on the f32 MFMA.
+// A K of one step goes there at once (direct): the truncation inside an MFMA costs
+// more than f32's roundings (from two steps on it costs less).  So does f32 x f32 of
+// a shallow K in few tiles, where splitting takes longer than the slower MFMA.
 //
 // Workgroup: 4 waves, WGM along m; each wave TM x TN 16x16 tiles; K in steps
 // of 32, both operands double-buffered in LDS as 8-value octets.  A step sums
@@ -120,7 +115,8 @@ constexpr int MM_LD = 17;  // octet stride in 16-byte units (16 rows + 1: spread
 
 template <bool ABF, bool BBF, bool AV, bool BV, int TM, int TN, int WGM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void matmul_kernel(
-    MatOperand A, MatOperand B, float* __restrict__ c, int K, size_t split_stride, int k_per_split, int accumulate) {
+    MatOperand A, MatOperand B, float* __restrict__ c, int K, size_t split_stride, int k_per_split, int direct,
+    int accumulate) {
     constexpr int PA = ABF ? 1 : 3, PB = BBF ? 1 : 3, WGN = 4 / WGM;
     constexpr bool PARTS = PA * PB > 1;
     constexpr int MB = WGM * TM, NB = WGN * TN;           // 16-row blocks of the workgroup
@@ -277,8 +273,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
                 }
         }
     };
-    sum(std::integral_constant<int, 0>{});
-    if constexpr (PARTS) {
+    if constexpr (!PARTS) {
+        sum(std::integral_constant<int, 0>{});
+    } else if (direct) {
+        sum_f32();
+    } else {
+        sum(std::integral_constant<int, 0>{});
         auto any = [&](auto test) {
             bool t = false;
 #pragma unroll
@@ -292,8 +292,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
         const auto nonfinite = [](float v) { return !(v <= 3.402823466e38f); };
         // parts of an operand or of a product below the formats' smallest numbers
         const bool vanished = (lost & 0xFFFFu) != 0 || any([](float v) { return v > 0.0f && v < 0x1p-100f; });
-        const bool one_step = ke <= kb + 32;
-        if (__syncthreads_or(vanished || one_step || any(nonfinite))) {
+        if (__syncthreads_or(vanished || any(nonfinite))) {
             if (__syncthreads_or(vanished)) {
                 asm volatile("" : "+v"(tid));  // places are formed again, not kept through the first pass
                 sum(std::integral_constant<int, SPLIT_EXP>{});
@@ -305,7 +304,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
                         for (int e = 0; e < 4; e++)
                             acc[i][j][e] = __builtin_amdgcn_ldexpf(acc[i][j][e], -SPLIT_EXP * (!ABF + !BBF));
             }
-            if (__syncthreads_or(one_step || any(nonfinite))) sum_f32();
+            if (__syncthreads_or(any(nonfinite))) sum_f32();
         }
     }
     float* cb = c + (size_t)split * split_stride;
@@ -331,6 +330,96 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     }
 }
 
+// f32 x f32 of a shallow K over more tiles than the CUs: 64x64 tiles on the f32
+// MFMA, four waves of 32x32, K in steps of 16 through LDS rows padded to 68 floats
+// (the operand reads hit distinct banks).  Splitting the operands would take longer
+// than the MFMAs save (matmul_dispatch has the line).
+constexpr int MF_T = 64, MF_K = 16, MF_LD = MF_T + 4;
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256) void matmul_f32_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                         float* __restrict__ c, int M, int N, int K, int accumulate) {
+    __shared__ float As[MF_K][MF_LD];  // As[kk][row]
+    __shared__ float Bs[MF_K][MF_LD];  // Bs[kk][col]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.y * MF_T, n0 = blockIdx.x * MF_T;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    f32x4_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    // staging: each thread moves 4 elements of each 64x16 tile; the fast
+    // index follows the contiguous dimension of the source
+    auto stage = [&](int k0, float ra[4], float rb[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int e = tid + 256 * u;
+            int row, kk;
+            if (TA) { row = e & 63; kk = e >> 6; }   // A[k][m]: m contiguous
+            else { kk = e & 15; row = e >> 4; }      // A[m][k]: k contiguous
+            const int gm = m0 + row, gk = k0 + kk;
+            ra[u] = (gm < M && gk < K) ? a[TA ? (size_t)gk * M + gm : (size_t)gm * K + gk] : 0.0f;
+            int col, kb;
+            if (TB) { kb = e & 15; col = e >> 4; }   // B[n][k]: k contiguous
+            else { col = e & 63; kb = e >> 6; }      // B[k][n]: n contiguous
+            const int gn = n0 + col, gkb = k0 + kb;
+            rb[u] = (gn < N && gkb < K) ? b[TB ? (size_t)gn * K + gkb : (size_t)gkb * N + gn] : 0.0f;
+        }
+    };
+    auto store = [&](const float ra[4], const float rb[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int e = tid + 256 * u;
+            if (TA) As[e >> 6][e & 63] = ra[u];
+            else As[e & 15][e >> 4] = ra[u];
+            if (TB) Bs[e & 15][e >> 4] = rb[u];
+            else Bs[e >> 6][e & 63] = rb[u];
+        }
+    };
+    float ra[4], rb[4];
+    stage(0, ra, rb);
+    for (int k0 = 0; k0 < K; k0 += MF_K) {
+        store(ra, rb);
+        __syncthreads();
+        if (k0 + MF_K < K) stage(k0 + MF_K, ra, rb);  // next tile's loads in flight during the MFMAs
+#pragma unroll
+        for (int ks = 0; ks < MF_K; ks += 4) {
+            // 16x16x4: lane (g, r) supplies A[row r][k g] and B[k g][col r]
+            const int g = lane >> 4, r = lane & 15;
+            float av[2], bv[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) av[i] = As[ks + g][wm + 16 * i + r];
+#pragma unroll
+            for (int j = 0; j < 2; j++) bv[j] = Bs[ks + g][wn + 16 * j + r];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+    mfma_settle(acc);
+    // D: lane (g, r) holds rows 4g..4g+3 of column r
+    const int g = lane >> 4, r = lane & 15;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int col = n0 + wn + 16 * j + r;
+            if (col >= N) continue;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = m0 + wm + 16 * i + 4 * g + e;
+                if (row < M) {
+                    float* p = c + (size_t)row * N + col;
+                    *p = accumulate ? *p + acc[i][j][e] : acc[i][j][e];
+                }
+            }
+        }
+}
+
 template <bool ABF, bool BBF, bool AV, bool BV, int TM, int TN, int WGM>
 static void matmul_launch(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
     const size_t m = A.rows, n = B.rows, part = m * n * sizeof(float), cus = dev->num_cus;
@@ -341,24 +430,54 @@ static void matmul_launch(const MatOperand& A, const MatOperand& B, float* c, si
     const size_t per = round_up(ceil_div(k, ks), (size_t)32);
     ks = ceil_div(k, per);
     float* out = ks > 1 ? (float*)device_scratch(dev, ks * part) : c;
+    // (us, parts / direct, 16 x 64 tiles: 33 x 216 x 2866, 135 workgroups, 9.2 / 6.6; 300 x
+    // 300 x 1000, 304, 12.9 / 9.9; 300 x 200 x 4000, 1197, 16.9 / 20.4)
+    const bool direct = k <= 32 || (!ABF && !BBF && TM == 1 && k <= 320 && (size_t)gx * gy <= 2 * cus);
     TH_LAUNCH((matmul_kernel<ABF, BBF, AV, BV, TM, TN, WGM>), dim3(gx, gy, (unsigned)ks), dim3(256), 0, dev->stream, A, B,
-              out, (int)k, m * n, (int)per, ks > 1 ? 0 : acc);
+              out, (int)k, m * n, (int)per, (int)direct, ks > 1 ? 0 : acc);
     TH_LAUNCH_CHECK();
     if (ks > 1) launch_splitk_reduce(out, c, m, n, n, ks, acc != 0, dev->stream);
 }
 
 template <bool ABF, bool BBF, bool AV, bool BV>
 static void matmul_shape(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
-    if (A.rows <= 16) matmul_launch<ABF, BBF, AV, BV, 1, 1, 1>(A, B, c, k, acc, dev);  // 16 x 64
-    else matmul_launch<ABF, BBF, AV, BV, 2, 4, 2>(A, B, c, k, acc, dev);               // 64 x 128
+    // 16 x 64 tiles up to 16 rows and where 64 x 128 ones, their K split, come to half
+    // the CUs or fewer: more workgroups, each with less to split and stage a step
+    // (us, 16 x 64 / 64 x 128, f32 x bf16: 64 x 1024 x 1024, 64 workgroups, 10.6 / 12.7;
+    // 100 x 576 x 1536, 96, 10.1 / 12.3; 100 x 100 x 8192, 128, 7.9 / 8.9; 300 x 100 x 4000,
+    // 160, 9.2 / 9.4; 40 x 4096 x 1536, 192, 19.3 / 18.5; 128 x 2048 x 2048, 512, 26.2 / 21.3).
+    const size_t large = ceil_div(A.rows, (size_t)64) * ceil_div(B.rows, (size_t)128) * std::clamp<size_t>(k / 128, 1, 16);
+    if (A.rows <= 16 || 2 * large <= (size_t)dev->num_cus) matmul_launch<ABF, BBF, AV, BV, 1, 1, 1>(A, B, c, k, acc, dev);
+    else matmul_launch<ABF, BBF, AV, BV, 2, 4, 2>(A, B, c, k, acc, dev);
 }
 
 template <bool ABF, bool BBF>
-static void matmul_dispatch(const MatOperand& A, const MatOperand& B, float* c, size_t k, int acc, th_device* dev) {
+static void matmul_dispatch(const MatOperand& A, const MatOperand& B, float* c, size_t k, bool trans_a, bool trans_b,
+                            int acc, th_device* dev) {
     // one 16-byte load per octet where k is contiguous, rows are whole dwords
     // and a block's offsets fit 32 bits
     auto vec = [](const MatOperand& m, bool bf) { return m.ks == 1 && (!bf || m.rs % 2 == 0) && m.rs <= (1l << 21); };
     const bool av = vec(A, ABF), bv = vec(B, BBF);
+    if constexpr (!ABF && !BBF) {
+        // us, 64x64 on the f32 MFMA / parts: 100 x 100 x 8192 7.6 / 10.0, k 160 9.5 / 10.4, k
+        // 256 13.3 / 14.8; 300 x 200 x 4000 15.2 / 16.9; 1024 x 64 x 1024 5.8 / 6.6; but 512 x 128 x
+        // 512 (16 x 64 tiles, direct) 7.8 / 4.7, 1000 x 200 x 200 10.9 / 6.5
+        const size_t gx = ceil_div(B.rows, (size_t)MF_T), gy = ceil_div(A.rows, (size_t)MF_T);
+        if (A.rows > 16 && k <= 256 && 2 * gx * gy > (size_t)dev->num_cus) {
+            auto f32 = [&](auto ta, auto tb) {
+                TH_LAUNCH((matmul_f32_kernel<decltype(ta)::value, decltype(tb)::value>), dim3((unsigned)gx, (unsigned)gy),
+                          dim3(256), 0, dev->stream, (const float*)A.p, (const float*)B.p, c, A.rows, B.rows, (int)k, acc);
+                TH_LAUNCH_CHECK();
+            };
+            const std::true_type t;
+            const std::false_type n;
+            if (trans_a && trans_b) f32(t, t);
+            else if (trans_a) f32(t, n);
+            else if (trans_b) f32(n, t);
+            else f32(n, n);
+            return;
+        }
+    }
     if (av && bv) matmul_shape<ABF, BBF, true, true>(A, B, c, k, acc, dev);
     else if (av) matmul_shape<ABF, BBF, true, false>(A, B, c, k, acc, dev);
     else if (bv) matmul_shape<ABF, BBF, false, true>(A, B, c, k, acc, dev);
@@ -437,10 +556,10 @@ int th_matmul_ex(th_device* dev, const th_buffer* a, const th_buffer* b, size_t 
     const MatOperand B{b->ptr, (int)n, trans_b ? (long)k : 1l, trans_b ? 1l : (long)n};
     float* out = (float*)c->ptr;
     const bool abf = a->dtype == TH_BF16, bbf = b->dtype == TH_BF16;
-    if (abf && bbf) matmul_dispatch<true, true>(A, B, out, k, accumulate, dev);
-    else if (abf) matmul_dispatch<true, false>(A, B, out, k, accumulate, dev);
-    else if (bbf) matmul_dispatch<false, true>(A, B, out, k, accumulate, dev);
-    else matmul_dispatch<false, false>(A, B, out, k, accumulate, dev);
+    if (abf && bbf) matmul_dispatch<true, true>(A, B, out, k, trans_a != 0, trans_b != 0, accumulate, dev);
+    else if (abf) matmul_dispatch<true, false>(A, B, out, k, trans_a != 0, trans_b != 0, accumulate, dev);
+    else if (bbf) matmul_dispatch<false, true>(A, B, out, k, trans_a != 0, trans_b != 0, accumulate, dev);
+    else matmul_dispatch<false, false>(A, B, out, k, trans_a != 0, trans_b != 0, accumulate, dev);
     TH_API_END
 }
 

@@ -42,7 +42,7 @@ def test_matmul_variants(dev, m, k, n, ta, tb):
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 1, 3), (16, 31, 64), (17, 33, 65), (64, 32, 128), (65, 130, 129), (3, 1000, 70),
-                                   (130, 515, 260), (1, 100, 1)])
+                                   (130, 515, 260), (1, 100, 1), (33, 200, 100), (610, 100, 1210)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("ad,bd", [("f32", "bf16"), ("bf16", "f32"), ("bf16", "bf16"), ("f32", "f32")])
 def test_matmul_tiles_and_types(dev, m, k, n, ta, tb, ad, bd):
@@ -77,7 +77,7 @@ def _spread(rng, shape, exps):
     return x.astype(np.float32)
 
 
-@pytest.mark.parametrize("m,k,n", [(9, 70, 50), (80, 515, 140)])
+@pytest.mark.parametrize("m,k,n", [(9, 70, 50), (80, 515, 140), (620, 70, 1160)])
 @pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
 @pytest.mark.parametrize("ad,bd", [("f32", "bf16"), ("bf16", "f32"), ("f32", "f32")])
 @pytest.mark.parametrize("big", [False, True])
@@ -129,12 +129,12 @@ def test_matmul_full_mantissas(dev, m, k, ad, bd):
     assert np.max(np.abs(err)) <= (1 if k == 1 else k / 8 + 2)
 
 
-@pytest.mark.parametrize("m", [5, 70])
+@pytest.mark.parametrize("m,k", [(5, 200), (70, 200), (5, 400), (70, 400)])
 @pytest.mark.parametrize("bd", ["f32", "bf16"])
-def test_matmul_infinities(dev, m, bd):
+def test_matmul_infinities(dev, m, k, bd):
     """An infinity times finite values gives infinities, times zero NaN, and
     reaches no other row or column."""
-    k, n = 200, 40
+    n = 40
     rng = np.random.default_rng(m)
     a = rng.integers(1, 9, (m, k)).astype(np.float32)
     b = rng.integers(1, 9, (k, n)).astype(np.float32)
