@@ -26,7 +26,7 @@ def test_noalloc_matches_gemm_q4_on_consecutive_calls(dev):
     rows, cols = 11008, 4096
     nib, sc16 = capi.synth_q4(2, rows, cols)
     w = dev.q4_upload_packed(nib, sc16, rows, cols, capi.F16)
-    for m in (300, 40, 3):  # MFMA with split-K, MFMA with more splits, then the GEMV path
+    for m in (300, 40, 3):  # the MFMA GEMMs of many and of few rows, then the GEMV path
         print(f"noalloc m={m}", flush=True)
         xb = capi.synth_normal(50 + m, m * cols, 1.0, capi.BF16)
         x = dev.upload(xb, capi.BF16)
