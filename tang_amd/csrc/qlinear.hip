@@ -352,8 +352,14 @@ static void q8_dispatch(const th_qweight* w, const void* x, size_t m, size_t ldx
     if (!q8_uses_gemv(w, m)) {
         // the rows that the GEMV stages bound K for every m above three
         TH_REQUIRE((Q8GemvSmem<4, 8>::bytes((int)w->Kp)) <= 160 * 1024, "activation too large for the LDS-staged GEMV");
-        if (x_vec_ok(x, ldx, w->cols)) q8_gemm_dispatch<XF32, PR, true>(w, x, m, ldx, y, ldy, s, dev);
-        else q8_gemm_dispatch<XF32, PR, false>(w, x, m, ldx, y, ldy, s, dev);
+        constexpr size_t ROWS = (size_t)1 << 21;  // a grid has at most 65535 blocks of 64 rows
+        for (size_t m0 = 0; m0 < m; m0 += ROWS) {
+            const void* xo = (const char*)x + m0 * ldx * (XF32 ? 4 : 2);
+            float* yo = y + m0 * ldy;
+            const size_t mm = std::min(ROWS, m - m0);
+            if (x_vec_ok(xo, ldx, w->cols)) q8_gemm_dispatch<XF32, PR, true>(w, xo, mm, ldx, yo, ldy, s, dev);
+            else q8_gemm_dispatch<XF32, PR, false>(w, xo, mm, ldx, yo, ldy, s, dev);
+        }
         return;
     }
     for (size_t m0 = 0; m0 < m; m0 += 4) {

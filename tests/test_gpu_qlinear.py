@@ -351,3 +351,18 @@ def test_full_size_linearity(dev):
     y2 = dev.gemm_q4(dev.upload(x2), 1, w).to_numpy()
     y3 = dev.gemm_q4(dev.upload(2.0 * x1 + x2), 1, w).to_numpy()
     assert max_abs_rel(y3, 2.0 * y1 + y2) < 1e-4
+
+
+def test_q8_gemm_rows_beyond_one_grid(dev):
+    """More blocks of 64 rows than a grid has in y: the bound of test_q8_gemm."""
+    rows, cols, m, period = 5, 32, 65536 * 64 + 3, 1009
+    rng = np.random.default_rng(5)
+    q, sc = rng.integers(-127, 128, (rows, cols), np.int8), rng.uniform(0.5, 1, rows).astype(np.float32)
+    w = dev.q8_upload_rowwise(q, sc, rows, cols)
+    base = oracle.f32_to_bf16(rng.standard_normal(period * cols).astype(np.float32))
+    x = oracle.bf16_to_f32(base).reshape(period, cols).astype(np.float64)
+    wf = q.astype(np.float64) * sc.astype(np.float64)[:, None]
+    ref, bound = x @ wf.T, (cols + 17) * 2.0 ** -24 * (np.abs(x) @ np.abs(wf).T)
+    y = dev.gemv_q8(dev.upload(np.resize(base, m * cols), capi.BF16), m, w).to_numpy().reshape(m, rows)
+    i = np.arange(m) % period
+    assert np.all(np.abs(y - ref[i]) <= bound[i])
